@@ -537,7 +537,8 @@ int psb_hip_csr_slices(void *dmat);
    columns are solved one after another. */
 int psb_hip_csr_spsv(void *dmat, int lower, int unit, int trans, double alpha, void *x,
                      double beta, void *y);
-/* levels and workgroup runs of the prepared solve (0, 0 before the first) */
+/* levels of the prepared solve and its tiles, each solved by one workgroup
+   (0, 0 before the first; 0 tiles when it launches once per level) */
 int psb_hip_csr_spsv_levels(void *dmat, int *levels, int *segments);
 
 /* ===================================================================== */
@@ -618,10 +619,12 @@ int psb_hip_ilu_alloc(void **ilu, int n, const int *lirp, const int *lja, const 
                       const int *uirp, const int *uja, const double *uval, const double *d);
 int psb_hip_ilu_free(void *ilu);
 int psb_hip_ilu_levels(void *ilu, int *lower_levels, int *upper_levels);
-/* runs of small levels solved by one workgroup (0 when the variant is 1) */
+/* tiles of each factor, each solved by one workgroup (0 when the solves launch
+   once per level: the variant is 1, the factors have few levels, or a row does
+   not fit a tile) */
 int psb_hip_ilu_segments(void *ilu, int *lower_segments, int *upper_segments);
-/* triangular-solve kernels for factors allocated afterwards: 0 (default) runs
-   of small levels by one workgroup each, other levels one launch each; 1 one
+/* triangular-solve kernels for factors allocated afterwards: 0 (default) tiles
+   of rows, one workgroup each, that wait for one another's entries; 1 one
    launch per level.  Same results either way.  Returns the previous value. */
 int psb_hip_ilu_set_variant(int variant);
 /* psb_d_bjac_apply_vect (ILU, trans 'N'): y = alpha * U^-1 (d .* L^-1 x) + beta * y */

@@ -22,98 +22,118 @@
 // computed as the CPU updates them, by running subtraction
 // y(c) = ((x(c) - v1 y(i1)) - v2 y(i2)) ..., then the division.
 //
-// The solve runs in level order: each triangle is renumbered so that level l
-// holds positions lev_ptr[l] .. lev_ptr[l+1]-1 (rows ascending inside a
-// level), x is gathered into that order by one full-grid kernel and the
-// solution scattered back by another (the last one also applies alpha and
-// beta), so every level reads and writes a contiguous range.
+// The triangle is cut into tiles of at most kTileRows rows and one workgroup
+// solves a tile: its rows in steps (the levels inside the tile, 64 rows at a
+// time, one wavefront), with the entries, the right-hand side and the solution
+// staged in LDS, so a step costs LDS traffic and arithmetic only.  A row's
+// dependencies outside its tile (its halo) are polled from the solution array
+// itself, which starts out filled with one NaN bit pattern that no solve
+// stores (tri_unset): an entry is ready once it holds anything else, so a
+// value needs no flag and no fence (8- or 4-byte agent-scope loads and
+// stores).  Three wavefronts of the workgroup poll while the fourth solves.
+// Workgroups take their tiles by a ticket, in an order where a tile depends
+// only on tiles before it, so a workgroup waits only for tiles whose
+// workgroups already run: every wait ends whatever the number of resident
+// workgroups.  Two solution arrays alternate; a tile resets its rows of the
+// other one for the solve after.
 //
-// A launch per level costs a few microseconds of dispatch, more than the work
-// of a small level, so runs of consecutive small levels (each at most 2048
-// rows of at most 4 entries, or 1024 rows of at most 8) are solved by ONE
-// workgroup of 1024 threads that walks the levels with an LDS barrier
-// between them.  Everything a run reads of the solution lives in LDS
-// (128 KB): its own rows (first holding x, then overwritten by the solution)
-// and the "halo" of positions solved before the run that it depends on,
-// loaded once at the start.  A level therefore waits only for the LDS traffic
-// of the level before it; the run's solution goes to global memory once, at
-// its end.  A run's entries (16-bit LDS slot, value) are laid out per level,
-// column-major and padded to the run's width, the smallest of 2, 3, 4, 8 that
-// fits (entry k of the level's t-th row at off + k*count + t; a padding slot
-// adds value 0 times a zero LDS slot, which leaves the sum's bits unchanged),
-// and are loaded two levels ahead.  Larger or wider levels get a launch of
-// their own (one thread per row, level-ordered CSR).  The permutations, both
-// triangles and the pivot scaling are captured once into a graph that works
-// on internal buffers.
+// Tiles follow the grid when the triangle's entries sit at the offsets of a
+// regular grid in natural order (1, p and q, p dividing q: 5- and 7-point
+// stencils and their ILU(0) factors), as boxes of 8 x 8 x 8 or 24 x 24 rows;
+// otherwise they are runs of consecutive rows.  The chain of dependencies
+// then crosses tiles once in 8 (24) rows along each axis, and only a crossing
+// pays the way through memory between XCDs.
+//
+// Measured against one workgroup walking runs of small levels and a launch for
+// each larger one, which this replaced (7-point stencil, lower, non-unit,
+// FP64): L = 32 156 -> 41 us, L = 64 438 -> 91 us, L = 110 903 -> 204 us (boxes of
+// 10 x 10 x 10 53 / 114 / 228 us, of 8 x 8 x 4 44 / 106 / 224 us); 5-point
+// 1000 x 1000 2562 -> 647 us; 27-point L = 40, runs of rows, 1373 -> 407 us.
+//
+// A triangle of at most kFewLevels levels, with a row of more than
+// kTileEntries / 2 entries, or with the launch-per-level variant set, is
+// solved in level order instead: renumbered
+// so that level l holds positions lev_ptr[l] .. lev_ptr[l+1]-1 (rows ascending
+// inside a level), x gathered into that order, one launch per level (one
+// thread per row), the solution scattered back; captured once into a graph
+// that works on internal buffers.
 #pragma clang fp contract(off)
 
 #include <string.h>
 
 #include <algorithm>
+#include <thread>
 #include <vector>
 
 #include "psb_hip_internal.hpp"
 
 namespace psbhip {
 
-// A run of levels solved by one workgroup: levels [lev0, lev1), entry width
-// W, nhalo positions from before the run at halo[hoff ..].
-struct TriSegment {
-  int lev0, lev1, width, hoff, nhalo;
-};
+// Limits of a tile: rows, stored entries, halo entries, LDS bytes (64 KB
+// lets two workgroups share a CU; an 8 x 8 x 8 tile takes about 31 KB).
+constexpr int kTileRows = 512;
+constexpr int kTileEntries = 2048;
+constexpr int kTileHalo = 1024;
+constexpr size_t kTileLds = (size_t)64 << 10;
+constexpr int kTileThreads = 256;
+// polls of a halo entry before the wait is given up (the entry then counts
+// as NaN); a poll takes about a microsecond, a real wait far fewer
+constexpr int kTilePolls = 1 << 23;
 
-constexpr int kSegThreads = 1024;
-constexpr int kSegRows = 16384;          // LDS slots of a run: its rows, its halo, two spare
-constexpr int kSinkSlot = kSegRows - 2;  // written by lanes beyond their level, never read
-constexpr int kZeroSlot = kSegRows - 1;  // holds 0, read by padding entries
-constexpr int kSegLevels = 1024;         // levels of a run (their descriptors sit in LDS)
+// A tile: its rows at positions row0 .. row0+nrow-1 of the tile-ordered
+// arrays, its entries at ent0 .., its steps at step0 .., its halo at halo0 ..
+struct TriTile {
+  int row0, nrow, ent0, nent, step0, nstep, halo0, nhalo;
+};
 
 template <typename T>
 struct TriLevels {
   int n = 0, nnz = 0, nlev = 0;
+  // level order (one launch per level)
   int* perm = nullptr;          // level position -> row
   int* irp = nullptr;           // level-ordered CSR, 0-based; columns are level positions
   int* ja = nullptr;
   T* val = nullptr;
   std::vector<int> lev_ptr;     // host: level l = positions lev_ptr[l] .. lev_ptr[l+1]-1
-  // per-level column-major copies for the workgroup-solved runs
-  int4* lev_info = nullptr;     // {count, width, entry offset, first position} per level
-  uint16_t* eja = nullptr;      // LDS slot of each dependency (kSegRows <= 65536)
-  T* eval = nullptr;
-  int* halo = nullptr;          // positions before each run that the run reads
-  std::vector<TriSegment> segs; // host: the runs, in level order
-  std::vector<int> seg_of;      // host: segment index of a level, -1 if launched alone
+  // tiles (ntiles > 0: this form is used)
+  int ntiles = 0;
+  int width = 0;                // entries of every row, padding included; 0: per step
+  size_t lds = 0;               // LDS bytes of the largest tile
+  TriTile* tiles = nullptr;     // in ticket order
+  int* trow = nullptr;          // row of each position
+  T* tdv = nullptr;             // diagonal of each position (non-unit triangles)
+  T* tval = nullptr;            // entry k of a step's t-th row at ent + k*count + t
+  uint16_t* tdep = nullptr;     // LDS slot of the entry's dependency
+  int2* tstep = nullptr;        // {first row | rows << 16, first entry | width << 16}
+  int* thalo = nullptr;         // rows of earlier tiles the tile reads
+  T* sol = nullptr;             // two solution arrays of n entries
+  unsigned long long* ticket = nullptr;
 };
 
-// 0: runs of small levels by one workgroup (default); 1: one launch per level.
+// 0: tiles (default); 1: one launch per level.
 static int g_trsv_variant = 0;
-// Register stages of a run's entry pipeline: entries are loaded two levels
-// ahead (five stages measured 5% slower at L=40 and 64).
-constexpr int kSegStages = 3;
-
-// Rows per thread and entry width a workgroup run supports.
-__host__ __device__ constexpr int seg_rpt(int W) { return W <= 4 ? 2 : 1; }
-constexpr int kSegWidths[] = {2, 3, 4, 8};   // the entry widths a run can be built with
 
 struct IluDev {
   int n = 0;
   TriLevels<double> L, U;
   double* d = nullptr;          // inverse pivots
+  double* t1 = nullptr;         // L^-1 x (row order)
+  // launch-per-level form
   double* xa = nullptr;         // right-hand side of the triangle being solved (level order)
   double* ya = nullptr;         // its solution (level order)
-  double* t1 = nullptr;         // L^-1 x (row order)
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 };
 
 // A CSR matrix's triangle prepared for op(T)^-1 x: the strict part (or, for
-// op 'T' / 'C', the strict part of the transpose) in level order, and the
-// diagonal in the same order when the triangle is not unit.
+// op 'T' / 'C', the strict part of the transpose), and the diagonal when the
+// triangle is not unit.
 template <typename T>
 struct TriSolve {
   int n = 0, key = -1;          // key: lower | unit << 1 | transposed << 2
   bool run = false;             // transposed: rows by running subtraction
   TriLevels<T> tl;
+  // launch-per-level form
   T* dv = nullptr;              // diagonal in level order (non-unit), else null
   T* xa = nullptr;              // right-hand side (level order)
   T* ya = nullptr;              // solution (level order)
@@ -184,126 +204,267 @@ __global__ __launch_bounds__(kBlock) void k_trsv_level(int p0, int count,
   y[p] = DIV ? r / dv[p] : r;
 }
 
-// Levels [lev0, lev1) by one workgroup.  Row r of thread t in a level is
-// level row t + r*kSegThreads; lanes beyond the level work on the level's last
-// row and write the sink slot.  Loads are unconditional and neither the sum
-// nor the stores are behind a branch, so a level's LDS reads are in flight
-// together.  The sum runs over the row's entries in CSR order, then the
-// padding adds +0 to it (never -0: the sum starts at +0), which leaves it
-// unchanged; in the running form the padding subtracts +0, which leaves
-// every value, -0 included, unchanged.
+// The bit pattern of a solution entry that is not there yet: a quiet NaN with
+// a payload of its own.  A computed NaN with exactly these bits is stored as
+// the default NaN instead.
+template <typename T>
+struct TriBits;
+template <>
+struct TriBits<double> {
+  typedef unsigned long long U;
+  static constexpr U unset = 0x7ff8a5c3e1d2b497ull, nan = 0x7ff8000000000000ull;
+};
+template <>
+struct TriBits<float> {
+  typedef unsigned int U;
+  static constexpr U unset = 0x7fe5a3c9u, nan = 0x7fc00000u;
+};
+template <typename T>
+__device__ __forceinline__ bool tri_unset(T v) {
+  return __builtin_bit_cast(typename TriBits<T>::U, v) == TriBits<T>::unset;
+}
+template <typename T>
+__device__ __forceinline__ T tri_value(T v) {   // v, never the unset pattern
+  typedef typename TriBits<T>::U U;
+  const U u = __builtin_bit_cast(U, v);
+  return __builtin_bit_cast(T, u == TriBits<T>::unset ? TriBits<T>::nan : u);
+}
+// agent-scope (all XCDs) and workgroup-scope (LDS) accesses of one entry
+template <typename T>
+__device__ __forceinline__ T ld_agent(const T* p) {
+  typedef typename TriBits<T>::U U;
+  return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const U*>(p), __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT));
+}
+template <typename T>
+__device__ __forceinline__ void st_agent(T* p, T v) {
+  typedef typename TriBits<T>::U U;
+  __hip_atomic_store(reinterpret_cast<U*>(p), __builtin_bit_cast(U, v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T ld_lds(const T* p) {
+  typedef typename TriBits<T>::U U;
+  return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const U*>(p), __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+template <typename T>
+__device__ __forceinline__ void st_lds(T* p, T v) {
+  typedef typename TriBits<T>::U U;
+  __hip_atomic_store(reinterpret_cast<U*>(p), __builtin_bit_cast(U, v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_tri_unset(int64_t n, T* __restrict__ sol) {
+  const T u = __builtin_bit_cast(T, TriBits<T>::unset);
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kBlock)
+    sol[i] = u;
+}
+
+// LDS of a tile, in this order (each part 16-byte aligned): solution slots
+// (rows, halo, a zero slot), entry values, diagonals, rows, steps, entry
+// slots.  The host's tile_lds adds up the same parts.
+__host__ __device__ inline size_t lds16(size_t b) { return (b + 15) & ~(size_t)15; }
+template <typename T>
+__host__ __device__ inline size_t tile_lds(int nrow, int nhalo, int nent, int nstep, bool dv) {
+  return lds16(sizeof(T) * (size_t)(nrow + nhalo + 1)) + lds16(sizeof(T) * (size_t)nent) +
+         (dv ? lds16(sizeof(T) * (size_t)nrow) : 0) + lds16(sizeof(int) * (size_t)nrow) +
+         lds16(sizeof(int2) * (size_t)nstep) + lds16(sizeof(uint16_t) * (size_t)nent);
+}
+
+// Registers of one row's step: the operands that do not depend on the
+// solution, loaded a step ahead.
 template <typename T, int W, bool DIV>
-struct SegStage {
-  static constexpr int R = seg_rpt(W);
-  int dep[R][W];
-  T v[R][W];
-  T dv[DIV ? R : 1];
+struct TileStep {
+  int roff, cnt;
+  int dep[W];
+  T v[W];
+  T xi, dv;
+  int row;
 };
 
-template <typename T, int W, bool DIV>
-__device__ __forceinline__ void seg_fetch(SegStage<T, W, DIV>& S, const int4 L,
-                                          const uint16_t* __restrict__ eja,
-                                          const T* __restrict__ eval,
-                                          const T* __restrict__ dv) {
-#pragma unroll
-  for (int r = 0; r < SegStage<T, W, DIV>::R; r++) {
-    const int tt = min((int)threadIdx.x + r * kSegThreads, L.x - 1);
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-      const int64_t e = (int64_t)L.z + (int64_t)k * L.x + tt;
-      S.dep[r][k] = eja[e];
-      S.v[r][k] = eval[e];
-    }
-    if (DIV) S.dv[r] = dv[L.w + tt];
-  }
-}
-
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
+// One tile per workgroup.  Bound by the chain of dependencies: a step (the
+// LDS reads of W solution entries, W multiply-adds and, when DIV, a division)
+// is 0.26 us with the division (a chain of 20,000 rows 5.1 ms), a crossing
+// into the next tile one store and one load through memory between XCDs,
+// 1-2 us; the bytes (40 a row) would take 2 us at L = 64, not 91.  Polling by
+// every lane from the start instead of by the first ones until an entry
+// comes: 97 and 254 us at L = 64 and 110.  W > 0: every row has W entries
+// (padding: value 0 times the zero slot, which leaves the sum's bits
+// unchanged; the sum starts at +0, so it is never -0 there, and the running
+// form subtracts +0); W == 0: the step's own width.  Rows sum in CSR order.
 template <typename T, int W, bool DIV, bool RUN>
-__device__ __forceinline__ void seg_solve(const SegStage<T, W, DIV>& S, const int4 L, int base,
-                                          T* ys) {
-  constexpr int R = SegStage<T, W, DIV>::R;
-  lds_barrier();   // the LDS slots of the levels before this one are written
-  T yi[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    const int tt = min((int)threadIdx.x + r * kSegThreads, L.x - 1);
-    T yk[W];
-#pragma unroll
-    for (int k = 0; k < W; k++) yk[k] = ys[S.dep[r][k]];
-    const T xi = ys[L.w - base + tt];
-    T v;
-    if (RUN) {
-      v = xi;
-#pragma unroll
-      for (int k = 0; k < W; k++) v = v - S.v[r][k] * yk[k];
-    } else {
-      T acc = T(0);
-#pragma unroll
-      for (int k = 0; k < W; k++) acc = acc + S.v[r][k] * yk[k];
-      v = xi - acc;
-    }
-    yi[r] = DIV ? v / S.dv[r] : v;
+__global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
+    int n, int ntiles, const TriTile* __restrict__ tiles, const int* __restrict__ trow,
+    const T* __restrict__ tdv, const T* __restrict__ tval, const uint16_t* __restrict__ tdep,
+    const int2* __restrict__ tstep, const int* __restrict__ thalo, T* sol2,
+    unsigned long long* ticket, const T* x, const T* __restrict__ scale, T alpha, T beta, T* y) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ unsigned long long my;
+  if (threadIdx.x == 0) my = atomicAdd(ticket, 1ull);
+  __syncthreads();
+  // a launch draws exactly ntiles tickets, so all of its tickets share one epoch
+  const unsigned long long epoch = my / (unsigned)ntiles;
+  const TriTile t = tiles[(int)(my - epoch * (unsigned)ntiles)];
+  T* sol = sol2 + (epoch & 1 ? (size_t)n : 0);
+  T* next = sol2 + (epoch & 1 ? 0 : (size_t)n);
+  T* ys = reinterpret_cast<T*>(lds);
+  char* at = lds + lds16(sizeof(T) * (size_t)(t.nrow + t.nhalo + 1));
+  T* ev = reinterpret_cast<T*>(at);
+  at += lds16(sizeof(T) * (size_t)t.nent);
+  T* dvs = reinterpret_cast<T*>(at);
+  if (DIV) at += lds16(sizeof(T) * (size_t)t.nrow);
+  int* rows = reinterpret_cast<int*>(at);
+  at += lds16(sizeof(int) * (size_t)t.nrow);
+  int2* steps = reinterpret_cast<int2*>(at);
+  at += lds16(sizeof(int2) * (size_t)t.nstep);
+  uint16_t* ed = reinterpret_cast<uint16_t*>(at);
+  const T unset = __builtin_bit_cast(T, TriBits<T>::unset);
+
+  for (int p = threadIdx.x; p < t.nrow; p += kTileThreads) {
+    const int r = trow[t.row0 + p];
+    rows[p] = r;
+    T xv = x[r];
+    if (scale) xv = xv * scale[r];
+    ys[p] = xv;
+    if (DIV) dvs[p] = tdv[t.row0 + p];
+    next[r] = unset;
   }
+  for (int h = threadIdx.x; h < t.nhalo; h += kTileThreads) ys[t.nrow + h] = unset;
+  if (threadIdx.x == 0) ys[t.nrow + t.nhalo] = T(0);
+  for (int e = threadIdx.x; e < t.nent; e += kTileThreads) {
+    ev[e] = ld_stream(tval + t.ent0 + e);
+    ed[e] = tdep[t.ent0 + e];
+  }
+  for (int q = threadIdx.x; q < t.nstep; q += kTileThreads) steps[q] = tstep[t.step0 + q];
+  __syncthreads();
+
+  if (threadIdx.x >= kWave) {
+    // Pollers: each lane walks its halo entries (step order) and passes every
+    // one on to LDS as it comes.  Until the first entry is there only the
+    // first lanes poll, so tiles whose turn is far off load the memory little.
+    constexpr int kPollers = kTileThreads - kWave;
+    constexpr int kFirst = 8;
+    const int lane = threadIdx.x - kWave;
+    int h = lane, polls = 0;
+    int src = h < t.nhalo ? thalo[t.halo0 + h] : 0;
+    bool open = lane < kFirst;
+    while (__any(h < t.nhalo)) {
+      if (!open) open = !tri_unset(ld_lds(ys + t.nrow));
+      if (open && h < t.nhalo) {
+        const T v = ld_agent(sol + src);
+        if (!tri_unset(v)) {
+          st_lds(ys + t.nrow + h, v);
+          h += kPollers;
+          if (h < t.nhalo) src = thalo[t.halo0 + h];
+        }
+      } else {
+        __builtin_amdgcn_s_sleep(2);
+      }
+      if (++polls > kTilePolls) {
+        for (; h < t.nhalo; h += kPollers)
+          st_lds(ys + t.nrow + h, __builtin_bit_cast(T, TriBits<T>::nan));
+      }
+    }
+  } else {
+    const int lane = threadIdx.x;
+    constexpr int WR = W > 0 ? W : 4;
+    auto step = [&](int q) { return steps[q < t.nstep ? q : t.nstep - 1]; };
+    auto fetch = [&](int2 d, TileStep<T, WR, DIV>& s) {
+      s.roff = d.x & 0xffff;
+      s.cnt = d.x >> 16;
+      const int ln = lane < s.cnt ? lane : s.cnt - 1;
+      s.xi = ys[s.roff + ln];
+      s.row = rows[s.roff + ln];
+      if (DIV) s.dv = dvs[s.roff + ln];
+      if (W > 0) {
 #pragma unroll
-  for (int r = 0; r < R; r++) {
-    const int t = threadIdx.x + r * kSegThreads;
-    ys[t < L.x ? L.w - base + t : kSinkSlot] = yi[r];
+        for (int k = 0; k < WR; k++) {
+          const int e = W * s.roff + k * s.cnt + ln;
+          s.dep[k] = ed[e];
+          s.v[k] = ev[e];
+        }
+      }
+    };
+    // reads the solution entries; whether all of the step's have arrived
+    auto read = [&](const int (&dep)[WR], T (&yk)[WR]) {
+#pragma unroll
+      for (int k = 0; k < WR; k++) yk[k] = ld_lds(ys + dep[k]);
+    };
+    auto wait = [&](const int (&dep)[WR], T (&yk)[WR]) {
+      for (;;) {
+        bool ready = true;
+#pragma unroll
+        for (int k = 0; k < WR; k++) ready = ready && !tri_unset(yk[k]);
+        if (__all(ready)) break;
+        __builtin_amdgcn_s_sleep(1);
+        read(dep, yk);
+      }
+    };
+    auto add = [&](T& acc, const T (&v)[WR], const T (&yk)[WR]) {
+#pragma unroll
+      for (int k = 0; k < WR; k++) acc = RUN ? acc - v[k] * yk[k] : acc + v[k] * yk[k];
+    };
+    TileStep<T, WR, DIV> cur, nxt;
+    int2 d0 = step(0), d1 = step(1);
+    fetch(d0, cur);
+    for (int q = 0; q < t.nstep; q++) {
+      const int2 d2 = step(q + 2);
+      T acc = RUN ? cur.xi : T(0);
+      T yk[WR];
+      if constexpr (W > 0) {
+        read(cur.dep, yk);   // the critical reads first, the next step's behind them
+        fetch(d1, nxt);
+        wait(cur.dep, yk);
+        add(acc, cur.v, yk);
+      } else {
+        fetch(d1, nxt);
+        const int e0 = d0.y & 0xffff, w = d0.y >> 16;
+        const int ln = lane < cur.cnt ? lane : cur.cnt - 1;
+        for (int k0 = 0; k0 < w; k0 += WR) {
+          int dep[WR];
+          T v[WR];
+#pragma unroll
+          for (int k = 0; k < WR; k++) {   // past the width: the zero slot, value 0
+            const bool in = k0 + k < w;
+            const int e = e0 + (in ? k0 + k : 0) * cur.cnt + ln;
+            dep[k] = in ? (int)ed[e] : t.nrow + t.nhalo;
+            v[k] = in ? ev[e] : T(0);
+          }
+          read(dep, yk);
+          wait(dep, yk);
+          add(acc, v, yk);
+        }
+      }
+      T r = RUN ? acc : cur.xi - acc;
+      if (DIV) r = r / cur.dv;
+      r = tri_value(r);
+      if (lane < cur.cnt) {
+        st_lds(ys + cur.roff + lane, r);
+        st_agent(sol + cur.row, r);
+      }
+      cur = nxt;
+      d0 = d1;
+      d1 = d2;
+    }
+  }
+  __syncthreads();
+  for (int p = threadIdx.x; p < t.nrow; p += kTileThreads) {
+    const int i = rows[p];
+    const T s = ys[p];
+    T r;
+    if (alpha == T(0)) r = (beta == T(0)) ? T(0) : (beta == T(1) ? y[i] : beta * y[i]);
+    else if (beta == T(0)) r = (alpha == T(1)) ? s : alpha * s;
+    else r = alpha * s + beta * y[i];
+    y[i] = r;
   }
 }
 
-// x and y in level order; the run's positions are base .. base+nrun-1; dv
-// the diagonal in level order when DIV.
-template <typename T, int W, int NS, bool DIV, bool RUN>
-__global__ __launch_bounds__(kSegThreads) void k_trsv_seg(int lev0, int lev1, int base, int nrun,
-                                                          const int* __restrict__ halo, int nhalo,
-                                                          const int4* __restrict__ info,
-                                                          const uint16_t* __restrict__ eja,
-                                                          const T* __restrict__ eval,
-                                                          const T* __restrict__ dv,
-                                                          const T* __restrict__ x, T* y) {
-  __shared__ T ys[kSegRows];
-  __shared__ int4 linfo[kSegLevels];   // the run's level descriptors: no scalar load per level
-  for (int q = threadIdx.x; q < lev1 - lev0; q += kSegThreads) linfo[q] = info[lev0 + q];
-  for (int p = threadIdx.x; p < nrun; p += kSegThreads) ys[p] = x[base + p];
-  for (int h = threadIdx.x; h < nhalo; h += kSegThreads) ys[nrun + h] = y[halo[h]];
-  if (threadIdx.x == 0) ys[kZeroSlot] = T(0);
-  lds_barrier();
-  // Entries NS-1 levels ahead: NS register stages rotate, the one solved
-  // holds level l.  The loop runs whole rounds of NS (the stage indices are
-  // compile-time constants once unrolled) and the fetches are unconditional
-  // (past the run's end they repeat its last level), so every path leaves the
-  // same loads in flight and the compiler's waits stay exact.
-  SegStage<T, W, DIV> st[NS];
-  int4 Ls[NS];
-  auto level = [&](int l) { return linfo[min(l, lev1 - 1) - lev0]; };
-#pragma unroll
-  for (int q = 0; q < NS - 1; q++) {
-    Ls[q] = level(lev0 + q);
-    seg_fetch<T, W, DIV>(st[q], Ls[q], eja, eval, dv);
-  }
-  for (int l = lev0; l < lev1; l += NS) {
-#pragma unroll
-    for (int j = 0; j < NS; j++) {
-      const int ahead = (j + NS - 1) % NS;
-      Ls[ahead] = level(l + j + NS - 1);
-      seg_fetch<T, W, DIV>(st[ahead], Ls[ahead], eja, eval, dv);
-      if (l + j < lev1) seg_solve<T, W, DIV, RUN>(st[j], Ls[j], base, ys);   // uniform
-    }
-  }
-  lds_barrier();
-  for (int p = threadIdx.x; p < nrun; p += kSegThreads) y[base + p] = ys[p];
-}
-
-// Level of every row (longest chain of dependencies through the triangle),
-// rows grouped by level in ascending row order within a level.
-static void analyse(int n, bool lower, const int* irp, const int* ja, std::vector<int>& rows,
-                    std::vector<int>& lev_ptr, std::vector<int>& lev) {
+// Level of every row (longest chain of dependencies through the triangle);
+// the number of levels.
+static int count_levels(int n, bool lower, const int* irp, const int* ja, std::vector<int>& lev) {
   lev.assign(n, 0);
   int nlev = 0;
   for (int t = 0; t < n; t++) {
@@ -313,6 +474,12 @@ static void analyse(int n, bool lower, const int* irp, const int* ja, std::vecto
     lev[i] = l;
     nlev = std::max(nlev, l + 1);
   }
+  return nlev;
+}
+
+// Rows grouped by level, in ascending row order within a level.
+static void order_levels(int n, int nlev, const std::vector<int>& lev, std::vector<int>& rows,
+                         std::vector<int>& lev_ptr) {
   lev_ptr.assign(nlev + 1, 0);
   for (int i = 0; i < n; i++) lev_ptr[lev[i] + 1]++;
   for (int l = 0; l < nlev; l++) lev_ptr[l + 1] += lev_ptr[l];
@@ -321,140 +488,372 @@ static void analyse(int n, bool lower, const int* irp, const int* ja, std::vecto
   for (int i = 0; i < n; i++) rows[fill[lev[i]]++] = i;
 }
 
-// Runs of consecutive levels a workgroup can take: every level of a run has
-// at most seg_rpt(W) * kSegThreads rows of at most W entries, W one of
-// kSegWidths; the run's rows plus its halo fill at most kSegRows - 2 LDS
-// slots, and it has at most kSegLevels levels.
-template <typename V>
-static void plan_segments(TriLevels<V>& T, const int* irp, const int* ja,
-                          const std::vector<int>& rows, const std::vector<int>& lev) {
-  T.segs.clear();
-  T.seg_of.assign(T.nlev, -1);
-  std::vector<int> width(T.nlev, 0);
-  for (int l = 0; l < T.nlev; l++)
-    for (int p = T.lev_ptr[l]; p < T.lev_ptr[l + 1]; p++)
-      width[l] = std::max(width[l], irp[rows[p] + 1] - irp[rows[p]]);
-  auto fits = [&](int l, int W) {
-    return width[l] <= W && T.lev_ptr[l + 1] - T.lev_ptr[l] <= seg_rpt(W) * kSegThreads;
-  };
-  auto first_fit = [&](int q, int from) {   // smallest width >= from that level q fits
-    for (int W : kSegWidths)
-      if (W >= from && fits(q, W)) return W;
-    return 0;
-  };
-  std::vector<int> stamp(T.n > 0 ? T.n : 1, -1);
-  int cand = 0;
-  int l = 0;
-  while (l < T.nlev) {
-    int W = first_fit(l, 1);
-    if (!W) {
-      l++;
-      continue;
+// f(thread, lo, hi) over [0, n) on host threads (one below min_n).
+template <typename F>
+static void host_parallel(int n, int min_n, F f) {
+  const int hw = (int)std::thread::hardware_concurrency();
+  const int nt = n < min_n ? 1 : std::max(1, std::min({hw, 8, n}));
+  std::vector<std::thread> th;
+  for (int k = 1; k < nt; k++)
+    th.emplace_back([=, &f] { f(k, (int)((int64_t)n * k / nt), (int)((int64_t)n * (k + 1) / nt)); });
+  f(0, 0, (int)((int64_t)n / nt));
+  for (auto& t : th) t.join();
+}
+constexpr int kHostThreads = 8;
+constexpr int kHostMin = 32768;   // rows from which the planning uses threads
+
+// The offsets of a regular grid in natural order: every entry of the triangle
+// sits 1, p or q rows before its row (in solve order), q a multiple of p.
+// Returns the number of distinct offsets (2 or 3), 0 for any other triangle.
+static int grid_offsets(int n, bool lower, const int* irp, const int* ja, int (&o)[3]) {
+  int m = 0;
+  for (int i = 0; i < n; i++)
+    for (int e = irp[i] - 1; e < irp[i + 1] - 1; e++) {
+      const int d = lower ? i - (ja[e] - 1) : (ja[e] - 1) - i;
+      int k = 0;
+      while (k < m && o[k] != d) k++;
+      if (k < m) continue;
+      if (m == 3) return 0;
+      o[m++] = d;
     }
-    cand++;
-    int nh = 0;
-    auto add_halo = [&](int q) {   // the rows before the run that level q reads
-      for (int p = T.lev_ptr[q]; p < T.lev_ptr[q + 1]; p++)
-        for (int e = irp[rows[p]] - 1; e < irp[rows[p] + 1] - 1; e++) {
-          const int j = ja[e] - 1;
-          if (lev[j] < l && stamp[j] != cand) {
-            stamp[j] = cand;
-            nh++;
-          }
-        }
-    };
-    add_halo(l);
-    int e = l + 1;
-    for (; e < T.nlev; e++) {
-      bool ok = fits(e, W);
-      for (int W2 = first_fit(e, W + 1); !ok && W2; W2 = first_fit(e, W2 + 1)) {
-        bool all = true;   // every level so far must also fit the wider limits
-        for (int q = l; q < e && all; q++) all = fits(q, W2);
-        if (all) {
-          W = W2;
-          ok = true;
+  std::sort(o, o + m);
+  if (m < 2 || o[0] != 1 || o[1] < 8 || (m == 3 && o[2] % o[1] != 0)) return 0;
+  return m;
+}
+
+// Tile of every row in solve order t (row t of a lower triangle, n-1-t of an
+// upper one), tile numbers ascending along the dependencies; the number of
+// tiles.  Boxes of the grid when the triangle is one and no entry leaves a box
+// against its order (an entry that wraps round a grid line can), else runs of
+// consecutive rows within the limits of a tile.
+static int assign_tiles(int n, bool lower, const int* irp, const int* ja,
+                        std::vector<int>& tile) {
+  tile.assign(n, 0);
+  auto row = [&](int t) { return lower ? t : n - 1 - t; };
+  auto dep = [&](int e) { return lower ? ja[e] - 1 : n - ja[e]; };   // solve order of entry e
+  int o[3] = {1, 0, 0};
+  const int m = grid_offsets(n, lower, irp, ja, o);
+  if (m > 0) {
+    // 8 x 8 x 8: a level of the box is at most 48 rows, one step; 24 x 24 in
+    // two dimensions takes the same number of rows
+    const int nx = o[1], ny = m == 3 ? o[2] / nx : (n + nx - 1) / nx;
+    const int bx = m == 3 ? 8 : 24, by = bx, bz = 8;
+    const int tx = (nx + bx - 1) / bx, ty = (ny + by - 1) / by;
+    const int pl = nx * ny;
+    int nt[kHostThreads] = {};
+    host_parallel(n, kHostMin, [&](int th, int lo, int hi) {
+      int most = 0;
+      for (int t = lo; t < hi; t++) {
+        const int z = m == 3 ? t / pl : 0, r = m == 3 ? t - z * pl : t;
+        const int yy = r / nx, xx = r - yy * nx;
+        tile[t] = ((z / bz) * ty + yy / by) * tx + xx / bx;
+        most = std::max(most, tile[t] + 1);
+      }
+      nt[th] = most;
+    });
+    bool bad[kHostThreads] = {};
+    host_parallel(n, kHostMin, [&](int th, int lo, int hi) {
+      bool any = false;
+      for (int t = lo; t < hi; t++)
+        for (int e = irp[row(t)] - 1; e < irp[row(t) + 1] - 1; e++)
+          any = any || tile[dep(e)] > tile[t];
+      bad[th] = any;
+    });
+    if (!*std::max_element(bad, bad + kHostThreads))
+      return *std::max_element(nt, nt + kHostThreads);
+  }
+  std::vector<int> seen(n > 0 ? n : 1, -1);
+  int nt = 0, rows = 0, ent = 0, halo = 0, t0 = 0;
+  for (int t = 0; t < n; t++) {
+    const int b = irp[row(t)] - 1, e = irp[row(t) + 1] - 1;
+    for (;;) {
+      int fresh = 0;   // halo entries this row would add
+      for (int k = b; k < e; k++) {
+        const int d = dep(k);
+        if (d < t0 && seen[d] != nt) {
+          seen[d] = nt;
+          fresh++;
         }
       }
-      if (!ok) break;
-      add_halo(e);
-      if (T.lev_ptr[e + 1] - T.lev_ptr[l] + nh > kSegRows - 2 || e + 1 - l > kSegLevels) break;
+      if (rows == 0 || (rows < kTileRows && ent + (e - b) <= kTileEntries / 2 &&
+                        halo + fresh <= kTileHalo)) {
+        rows++;
+        ent += e - b;
+        halo += fresh;
+        break;
+      }
+      nt++;   // a new tile starts at this row
+      rows = ent = halo = 0;
+      t0 = t;
     }
-    if (e - l >= 2) {   // a lone level is as cheap as its own launch
-      for (int q = l; q < e; q++) T.seg_of[q] = (int)T.segs.size();
-      T.segs.push_back({l, e, W, 0, 0});
-    }
-    l = e;
+    tile[t] = nt;
   }
+  return nt + (n > 0 ? 1 : 0);
 }
 
 template <typename V>
-static int upload_segments(TriLevels<V>& T, const int* irp, const int* ja, const V* val,
-                           const std::vector<int>& rows, const std::vector<int>& pos,
-                           const std::vector<int>& lev) {
-  if (T.segs.empty()) return PSB_HIP_SUCCESS;
-  std::vector<int4> info(T.nlev, make_int4(0, 0, 0, 0));
-  int64_t ent = 0;
-  for (const TriSegment& S : T.segs)
-    for (int l = S.lev0; l < S.lev1; l++) {
-      const int c = T.lev_ptr[l + 1] - T.lev_ptr[l];
-      info[l] = make_int4(c, S.width, (int)std::min<int64_t>(ent, INT32_MAX), T.lev_ptr[l]);
-      ent += (int64_t)c * S.width;
-    }
-  if (ent > INT32_MAX) return set_error(PSB_HIP_UNSUPPORTED, "trsv", "triangle too large");
-  std::vector<uint16_t> eja(ent, kZeroSlot);   // padding: the zero slot, value 0
-  std::vector<V> eval(ent, V(0));
-  std::vector<int> halo, slot(T.n > 0 ? T.n : 1, -1);
-  for (TriSegment& S : T.segs) {
-    const int base = T.lev_ptr[S.lev0], nrun = T.lev_ptr[S.lev1] - base;
-    S.hoff = (int)halo.size();
-    for (int l = S.lev0; l < S.lev1; l++) {
-      const int4 L = info[l];
-      for (int t = 0; t < L.x; t++) {
-        const int i = rows[L.w + t];
-        const int b = irp[i] - 1, c = irp[i + 1] - 1 - b;
-        for (int k = 0; k < c; k++) {
-          const int j = ja[b + k] - 1;
-          int sl;
-          if (lev[j] >= S.lev0) {
-            sl = pos[j] - base;   // solved inside the run
-          } else {
-            if (slot[j] < 0) {     // first use of this position of the halo
-              slot[j] = nrun + (int)halo.size() - S.hoff;
-              halo.push_back(pos[j]);
-            }
-            sl = slot[j];
-          }
-          eja[(size_t)L.z + (size_t)k * L.x + t] = (uint16_t)sl;
-          eval[(size_t)L.z + (size_t)k * L.x + t] = val[b + k];
-        }
+static int upload(V** dst, const V* src, size_t count) {
+  PSB_HIP_CHECK(hipMalloc((void**)dst, sizeof(V) * std::max<size_t>(count, 1)));
+  if (count > 0)
+    PSB_HIP_CHECK(hipMemcpyAsync(*dst, src, sizeof(V) * count, hipMemcpyHostToDevice,
+                                 ctx().stream));
+  return PSB_HIP_SUCCESS;
+}
+
+// The tiles [q0, q1) as one host thread packs them, offsets from its own start.
+template <typename V>
+struct TilePack {
+  int q0 = 0, q1 = 0;
+  size_t lds = 0;
+  std::vector<V> val;
+  std::vector<uint16_t> dep;
+  std::vector<int2> step;
+  std::vector<int> halo;
+};
+constexpr unsigned kHaloHash = 4 * kTileHalo;   // a tile has at most kTileHalo halo entries
+
+// Cuts the triangle into tiles and uploads them (T.ntiles > 0 then); leaves
+// T.ntiles at 0 when a row does not fit a tile.
+template <typename V>
+static int plan_tiles(TriLevels<V>& T, bool lower, const int* irp, const int* ja, const V* val,
+                      const V* diag, const std::vector<int>& lev) {
+  const int n = T.n;
+  if (n == 0) return PSB_HIP_SUCCESS;
+  int wmax = 0;
+  for (int i = 0; i < n; i++) wmax = std::max(wmax, irp[i + 1] - irp[i]);
+  if (wmax > kTileEntries / 2) return PSB_HIP_SUCCESS;
+  auto row = [&](int t) { return lower ? t : n - 1 - t; };
+  auto dep = [&](int e) { return lower ? ja[e] - 1 : n - ja[e]; };
+  std::vector<int> tile;
+  const int nt = assign_tiles(n, lower, irp, ja, tile);
+  // ticket order: tiles by their level in the graph of tiles, so that the
+  // tiles that run together are the ones whose turn it is
+  std::vector<int> ptr(nt + 1, 0), order(n), tlev(nt, 0), tnew(nt);
+  for (int t = 0; t < n; t++) ptr[tile[t] + 1]++;
+  for (int k = 0; k < nt; k++) ptr[k + 1] += ptr[k];
+  {
+    std::vector<int> fill(ptr.begin(), ptr.end() - 1);
+    for (int t = 0; t < n; t++) order[fill[tile[t]]++] = t;
+  }
+  int nlev = 0;
+  for (int k = 0; k < nt; k++) {
+    int l = 0;
+    for (int p = ptr[k]; p < ptr[k + 1]; p++) {
+      const int i = row(order[p]);
+      for (int e = irp[i] - 1; e < irp[i + 1] - 1; e++) {
+        const int q = tile[dep(e)];
+        if (q != k) l = std::max(l, tlev[q] + 1);
       }
     }
-    S.nhalo = (int)halo.size() - S.hoff;
-    for (int h = S.hoff; h < (int)halo.size(); h++) slot[rows[halo[h]]] = -1;
-    if (nrun + S.nhalo > kSegRows - 2)
-      return set_error(PSB_HIP_RUNTIME, "trsv", "run larger than its LDS slots");
+    tlev[k] = l;
+    nlev = std::max(nlev, l + 1);
   }
-  PSB_HIP_CHECK(hipMalloc(&T.lev_info, sizeof(int4) * (size_t)T.nlev));
-  PSB_HIP_CHECK(hipMalloc(&T.eja, sizeof(uint16_t) * eja.size()));
-  PSB_HIP_CHECK(hipMalloc(&T.eval, sizeof(V) * eval.size()));
-  PSB_HIP_CHECK(hipMalloc(&T.halo, sizeof(int) * std::max<size_t>(halo.size(), 1)));
+  std::vector<int> lptr(nlev + 1, 0), byl(nt);
+  for (int k = 0; k < nt; k++) lptr[tlev[k] + 1]++;
+  for (int l = 0; l < nlev; l++) lptr[l + 1] += lptr[l];
+  for (int k = 0; k < nt; k++) byl[lptr[tlev[k]]++] = k;
+  // pack the tiles: a step is the tile's rows of one level of the whole
+  // triangle, at most 64.  (By levels inside the tile a row whose own chain
+  // starts in an earlier tile would sit in the first step and hold up rows
+  // that are ready long before: runs of consecutive rows of the L = 110
+  // stencil took 70 ms that way.)
+  const int width = wmax <= 2 ? 2 : (wmax <= 4 ? wmax : 0);
+  std::vector<TriTile> tiles(nt);
+  for (int q = 0, pos = 0; q < nt; q++) {
+    tiles[q].row0 = pos;
+    pos += tiles[q].nrow = ptr[byl[q] + 1] - ptr[byl[q]];
+  }
+  std::vector<int> trow(n), at(n);   // at: position of a row (solve order) inside its tile
+  std::vector<V> tdv(diag ? n : 0);
+  TilePack<V> pack[kHostThreads];
+  host_parallel(nt, (kHostMin + kTileRows - 1) / kTileRows, [&](int th, int q0, int q1) {
+    TilePack<V>& P = pack[th];
+    P.q0 = q0;
+    P.q1 = q1;
+    std::vector<int> begin, fill, trs, key(kHaloHash, 0), where(kHaloHash);
+    std::vector<unsigned> stamp(kHaloHash, 0);
+    auto lv = [&](int t) { return lev[row(t)]; };
+    auto len = [&](int t) { return irp[row(t) + 1] - irp[row(t)]; };
+    for (int q = q0; q < q1; q++) {
+      const int k = byl[q], nrow = ptr[k + 1] - ptr[k];
+      TriTile& D = tiles[q];
+      D.ent0 = (int)P.val.size();
+      D.step0 = (int)P.step.size();
+      D.halo0 = (int)P.halo.size();
+      // the tile's rows by level; begin: where each level that occurs begins
+      trs.assign(order.begin() + ptr[k], order.begin() + ptr[k + 1]);
+      int l0 = lv(trs[0]), l1 = l0;
+      for (int t : trs) {
+        l0 = std::min(l0, lv(t));
+        l1 = std::max(l1, lv(t));
+      }
+      begin.clear();
+      if (l1 - l0 < 4 * nrow) {
+        fill.assign(l1 - l0 + 2, 0);
+        for (int t : trs) fill[lv(t) - l0 + 1]++;
+        for (int l = 0; l <= l1 - l0; l++) {
+          if (fill[l + 1] > 0) begin.push_back(fill[l]);
+          fill[l + 1] += fill[l];
+        }
+        for (int p = ptr[k]; p < ptr[k + 1]; p++) trs[fill[lv(order[p]) - l0]++] = order[p];
+      } else {
+        std::stable_sort(trs.begin(), trs.end(), [&](int x, int z) { return lv(x) < lv(z); });
+        for (int p = 0; p < nrow; p++)
+          if (p == 0 || lv(trs[p]) != lv(trs[p - 1])) begin.push_back(p);
+      }
+      const int nl = (int)begin.size();
+      begin.push_back(nrow);
+      if (width == 0)   // longest rows first: a step's rows are at least half as long as its widest
+        for (int l = 0; l < nl; l++)
+          std::stable_sort(trs.begin() + begin[l], trs.begin() + begin[l + 1],
+                           [&](int x, int z) { return len(x) > len(z); });
+      for (int p = 0; p < nrow; p++) {
+        at[trs[p]] = p;
+        trow[D.row0 + p] = row(trs[p]);
+        if (diag) tdv[D.row0 + p] = diag[row(trs[p])];
+      }
+      int nhalo = 0;
+      auto slot = [&](int d) {   // LDS slot of the row at d in solve order
+        if (tile[d] == k) return at[d];
+        unsigned h = (unsigned)d * 2654435761u % kHaloHash;
+        while (stamp[h] == (unsigned)q + 1 && key[h] != d) h = (h + 1) % kHaloHash;
+        if (stamp[h] != (unsigned)q + 1) {   // first use of an entry outside the tile
+          stamp[h] = (unsigned)q + 1;
+          key[h] = d;
+          where[h] = nrow + nhalo++;
+          P.halo.push_back(row(d));
+        }
+        return where[h];
+      };
+      for (int l = 0; l < nl; l++)
+        for (int r0 = begin[l], c = 0; r0 < begin[l + 1]; r0 += c) {
+          const int w = width > 0 ? width : len(trs[r0]);
+          c = std::min(kWave, begin[l + 1] - r0);
+          if (width == 0)
+            for (int p = 1; p < c; p++)
+              if (2 * len(trs[r0 + p]) < w) c = p;
+          const int e0 = (int)P.val.size() - D.ent0;
+          P.step.push_back(make_int2(r0 | c << 16, e0 | w << 16));
+          P.val.resize(P.val.size() + (size_t)w * c, V(0));
+          P.dep.resize(P.dep.size() + (size_t)w * c, 0xffff);   // padding, set below
+          for (int p = r0; p < r0 + c; p++) {
+            const int b = irp[row(trs[p])] - 1, m = len(trs[p]);
+            for (int u = 0; u < m; u++) {
+              const size_t x = (size_t)D.ent0 + e0 + (size_t)u * c + (p - r0);
+              P.val[x] = val[b + u];
+              P.dep[x] = (uint16_t)slot(dep(b + u));
+            }
+          }
+        }
+      D.nhalo = nhalo;
+      D.nent = (int)P.val.size() - D.ent0;
+      D.nstep = (int)P.step.size() - D.step0;
+      for (int e = D.ent0; e < D.ent0 + D.nent; e++)
+        if (P.dep[e] == 0xffff) P.dep[e] = (uint16_t)(nrow + nhalo);   // the zero slot
+      P.lds = std::max(P.lds, tile_lds<V>(nrow, nhalo, D.nent, D.nstep, diag != nullptr));
+    }
+  });
+  size_t lds = 0, ents = 0, steps = 0, halos = 0;
+  for (TilePack<V>& P : pack) {
+    for (int q = P.q0; q < P.q1; q++) {
+      tiles[q].ent0 += (int)ents;
+      tiles[q].step0 += (int)steps;
+      tiles[q].halo0 += (int)halos;
+    }
+    lds = std::max(lds, P.lds);
+    ents += P.val.size();
+    steps += P.step.size();
+    halos += P.halo.size();
+    if (ents > (size_t)INT32_MAX) return PSB_HIP_SUCCESS;
+  }
+  if (lds > kTileLds) return PSB_HIP_SUCCESS;
+  int rc = upload(&T.tiles, tiles.data(), tiles.size());
+  if (!rc) rc = upload(&T.trow, trow.data(), trow.size());
+  if (!rc && diag) rc = upload(&T.tdv, tdv.data(), tdv.size());
+  if (rc) return rc;
   hipStream_t s = ctx().stream;
-  PSB_HIP_CHECK(hipMemcpyAsync(T.lev_info, info.data(), sizeof(int4) * info.size(),
-                               hipMemcpyHostToDevice, s));
-  PSB_HIP_CHECK(hipMemcpyAsync(T.eja, eja.data(), sizeof(uint16_t) * eja.size(),
-                               hipMemcpyHostToDevice, s));
-  PSB_HIP_CHECK(hipMemcpyAsync(T.eval, eval.data(), sizeof(V) * eval.size(),
-                               hipMemcpyHostToDevice, s));
-  if (!halo.empty())
-    PSB_HIP_CHECK(hipMemcpyAsync(T.halo, halo.data(), sizeof(int) * halo.size(),
-                                 hipMemcpyHostToDevice, s));
+  PSB_HIP_CHECK(hipMalloc((void**)&T.tval, sizeof(V) * std::max<size_t>(ents, 1)));
+  PSB_HIP_CHECK(hipMalloc((void**)&T.tdep, sizeof(uint16_t) * std::max<size_t>(ents, 1)));
+  PSB_HIP_CHECK(hipMalloc((void**)&T.tstep, sizeof(int2) * steps));
+  PSB_HIP_CHECK(hipMalloc((void**)&T.thalo, sizeof(int) * std::max<size_t>(halos, 1)));
+  size_t e0 = 0, s0 = 0, h0 = 0;
+  for (const TilePack<V>& P : pack) {
+    if (!P.val.empty()) {
+      PSB_HIP_CHECK(hipMemcpyAsync(T.tval + e0, P.val.data(), sizeof(V) * P.val.size(),
+                                   hipMemcpyHostToDevice, s));
+      PSB_HIP_CHECK(hipMemcpyAsync(T.tdep + e0, P.dep.data(), sizeof(uint16_t) * P.dep.size(),
+                                   hipMemcpyHostToDevice, s));
+    }
+    if (!P.step.empty())
+      PSB_HIP_CHECK(hipMemcpyAsync(T.tstep + s0, P.step.data(), sizeof(int2) * P.step.size(),
+                                   hipMemcpyHostToDevice, s));
+    if (!P.halo.empty())
+      PSB_HIP_CHECK(hipMemcpyAsync(T.thalo + h0, P.halo.data(), sizeof(int) * P.halo.size(),
+                                   hipMemcpyHostToDevice, s));
+    e0 += P.val.size();
+    s0 += P.step.size();
+    h0 += P.halo.size();
+  }
+  const unsigned long long zero = 0;
+  rc = upload(&T.ticket, &zero, 1);
+  if (rc) return rc;
+  PSB_HIP_CHECK(hipMalloc((void**)&T.sol, sizeof(V) * 2 * (size_t)n));
+  hipLaunchKernelGGL((k_tri_unset<V>), dim3(stream_grid(2 * (int64_t)n)), dim3(kBlock), 0, s,
+                     2 * (int64_t)n, T.sol);
+  PSB_HIP_LAUNCH_CHECK();
   PSB_HIP_CHECK(hipStreamSynchronize(s));   // the host vectors go out of scope
+  T.width = width;
+  T.lds = lds;
+  T.ntiles = nt;
+  return PSB_HIP_SUCCESS;
+}
+
+// y = alpha * T^-1 (scale .* x) + beta * y by tiles (scale null: x itself).
+// x and y may be the same vector: a tile reads its rows of x before it writes
+// its rows of y, and no other tile's.
+template <typename V, bool DIV, bool RUN>
+static int solve_tiles_t(const TriLevels<V>& T, const V* x, const V* scale, V alpha, V beta, V* y,
+                         hipStream_t s) {
+#define PSB_TILE_LAUNCH(W)                                                                    \
+  hipLaunchKernelGGL((k_trsv_tiles<V, W, DIV, RUN>), dim3(T.ntiles), dim3(kTileThreads), T.lds, \
+                     s, T.n, T.ntiles, T.tiles, T.trow, T.tdv, T.tval, T.tdep, T.tstep, T.thalo, \
+                     T.sol, T.ticket, x, scale, alpha, beta, y)
+  switch (T.width) {
+    case 2: PSB_TILE_LAUNCH(2); break;
+    case 3: PSB_TILE_LAUNCH(3); break;
+    case 4: PSB_TILE_LAUNCH(4); break;
+    default: PSB_TILE_LAUNCH(0); break;
+  }
+#undef PSB_TILE_LAUNCH
+  PSB_HIP_LAUNCH_CHECK();
   return PSB_HIP_SUCCESS;
 }
 
 template <typename V>
+static int solve_tiles(const TriLevels<V>& T, bool run, const V* x, const V* scale, V alpha,
+                       V beta, V* y, hipStream_t s) {
+  if (T.tdv && run) return solve_tiles_t<V, true, true>(T, x, scale, alpha, beta, y, s);
+  if (T.tdv) return solve_tiles_t<V, true, false>(T, x, scale, alpha, beta, y, s);
+  if (run) return solve_tiles_t<V, false, true>(T, x, scale, alpha, beta, y, s);
+  return solve_tiles_t<V, false, false>(T, x, scale, alpha, beta, y, s);
+}
+
+// How a triangle is solved: as its shape decides, as tiles where they can, or
+// by levels.
+enum TriForm { TRI_AUTO, TRI_TILES, TRI_LEVELS };
+
+// Levels up to which a launch per level is at least as fast as tiles: 2
+// levels of 500,000 rows 61 against 71 us, a diagonal of a million rows 36
+// against 40 us; a launch is about 3 us, so from 5 levels on tiles win (38
+// levels of 20,000 rows 634 against 182 us).
+constexpr int kFewLevels = 4;
+
+// The triangle (diag: its diagonal, null for a unit one) as tiles, or in level
+// order with the launch-per-level variant, with few levels and where tiles
+// refuse.
+template <typename V>
 static int upload_tri(TriLevels<V>& T, int n, bool lower, const int* irp, const int* ja,
-                      const V* val, bool segments) {
+                      const V* val, const V* diag, TriForm form = TRI_AUTO) {
   T.n = n;
   T.nnz = irp[n] - 1;
   for (int i = 0; i < n; i++)
@@ -463,9 +862,14 @@ static int upload_tri(TriLevels<V>& T, int n, bool lower, const int* irp, const 
       if (c < 1 || c > n || (lower ? c > i : c < i + 2))
         return set_error(PSB_HIP_INVALID, "trsv", "entry outside its triangle");
     }
-  std::vector<int> rows, lev;
-  analyse(n, lower, irp, ja, rows, T.lev_ptr, lev);
-  T.nlev = (int)T.lev_ptr.size() - 1;
+  std::vector<int> lev;
+  T.nlev = count_levels(n, lower, irp, ja, lev);
+  if (form != TRI_LEVELS && g_trsv_variant != 1 && (form == TRI_TILES || T.nlev > kFewLevels)) {
+    const int rc = plan_tiles(T, lower, irp, ja, val, diag, lev);
+    if (rc || T.ntiles > 0) return rc;
+  }
+  std::vector<int> rows;
+  order_levels(n, T.nlev, lev, rows, T.lev_ptr);
   std::vector<int> pos(n > 0 ? n : 1, 0);
   for (int p = 0; p < n; p++) pos[rows[p]] = p;
   // the triangle in level order: row rows[p] becomes position p, its entries
@@ -480,28 +884,13 @@ static int upload_tri(TriLevels<V>& T, int n, bool lower, const int* irp, const 
     }
     pirp[p + 1] = pirp[p] + c;
   }
-  PSB_HIP_CHECK(hipMalloc(&T.irp, sizeof(int) * pirp.size()));
-  PSB_HIP_CHECK(hipMalloc(&T.ja, sizeof(int) * pja.size()));
-  PSB_HIP_CHECK(hipMalloc(&T.val, sizeof(V) * pval.size()));
-  PSB_HIP_CHECK(hipMalloc(&T.perm, sizeof(int) * (size_t)(n > 0 ? n : 1)));
-  hipStream_t s = ctx().stream;
-  PSB_HIP_CHECK(hipMemcpyAsync(T.irp, pirp.data(), sizeof(int) * pirp.size(),
-                               hipMemcpyHostToDevice, s));
-  PSB_HIP_CHECK(hipMemcpyAsync(T.ja, pja.data(), sizeof(int) * pja.size(), hipMemcpyHostToDevice,
-                               s));
-  PSB_HIP_CHECK(hipMemcpyAsync(T.val, pval.data(), sizeof(V) * pval.size(),
-                               hipMemcpyHostToDevice, s));
-  if (n > 0)
-    PSB_HIP_CHECK(hipMemcpyAsync(T.perm, rows.data(), sizeof(int) * (size_t)n,
-                                 hipMemcpyHostToDevice, s));
-  PSB_HIP_CHECK(hipStreamSynchronize(s));   // the host vectors go out of scope
-  if (segments) {
-    plan_segments(T, irp, ja, rows, lev);
-  } else {
-    T.segs.clear();
-    T.seg_of.assign(T.nlev, -1);   // every level launched alone
-  }
-  return upload_segments(T, irp, ja, val, rows, pos, lev);
+  int rc = upload(&T.irp, pirp.data(), pirp.size());
+  if (!rc) rc = upload(&T.ja, pja.data(), pja.size());
+  if (!rc) rc = upload(&T.val, pval.data(), pval.size());
+  if (!rc) rc = upload(&T.perm, rows.data(), rows.size());
+  if (rc) return rc;
+  PSB_HIP_CHECK(hipStreamSynchronize(ctx().stream));   // the host vectors go out of scope
+  return PSB_HIP_SUCCESS;
 }
 
 // x and y in level order; dv the diagonal in level order (null: unit);
@@ -509,29 +898,10 @@ static int upload_tri(TriLevels<V>& T, int n, bool lower, const int* irp, const 
 template <typename V, bool DIV, bool RUN>
 static void enqueue_levels_t(const TriLevels<V>& T, const V* dv, const V* x, V* y,
                              hipStream_t s) {
-  for (int l = 0; l < T.nlev;) {
-    const int g = T.seg_of[l];
-    if (g >= 0) {
-      const TriSegment& S = T.segs[g];
-      const int base = T.lev_ptr[S.lev0], nrun = T.lev_ptr[S.lev1] - base;
-#define PSB_SEG_LAUNCH(W)                                                                     \
-  hipLaunchKernelGGL((k_trsv_seg<V, W, kSegStages, DIV, RUN>), dim3(1), dim3(kSegThreads), 0, s, \
-                     S.lev0, S.lev1, base, nrun, T.halo + S.hoff, S.nhalo, T.lev_info, T.eja,   \
-                     T.eval, dv, x, y)
-      switch (S.width) {
-        case 2: PSB_SEG_LAUNCH(2); break;
-        case 3: PSB_SEG_LAUNCH(3); break;
-        case 4: PSB_SEG_LAUNCH(4); break;
-        default: PSB_SEG_LAUNCH(8); break;
-      }
-#undef PSB_SEG_LAUNCH
-      l = S.lev1;
-      continue;
-    }
+  for (int l = 0; l < T.nlev; l++) {
     const int count = T.lev_ptr[l + 1] - T.lev_ptr[l];
     hipLaunchKernelGGL((k_trsv_level<V, DIV, RUN>), dim3((count + kBlock - 1) / kBlock),
                        dim3(kBlock), 0, s, T.lev_ptr[l], count, T.irp, T.ja, T.val, dv, x, y);
-    l++;
   }
 }
 
@@ -544,7 +914,7 @@ static void enqueue_levels(const TriLevels<V>& T, const V* dv, bool run, const V
   else enqueue_levels_t<V, false, false>(T, dv, x, y, s);
 }
 
-// The captured part of an application: x in L level order (xa) -> U^-1
+// The captured part of a launch-per-level application: x in L level order (xa) -> U^-1
 // (d .* L^-1 x) in U level order (ya).  The gather of the caller's x and the
 // scatter into the caller's y (with alpha and beta) run around it.
 static void enqueue_apply(IluDev* F, hipStream_t s) {
@@ -559,7 +929,8 @@ static void enqueue_apply(IluDev* F, hipStream_t s) {
 
 template <typename V>
 static void free_tri(TriLevels<V>& T) {
-  void* p[] = {T.perm, T.irp, T.ja, T.val, T.lev_info, T.eja, T.eval, T.halo};
+  void* p[] = {T.perm, T.irp, T.ja, T.val, T.tiles, T.trow, T.tdv, T.tval, T.tdep, T.tstep,
+               T.thalo, T.sol, T.ticket};
   for (void* q : p)
     if (q) (void)hipFree(q);
   T = TriLevels<V>{};
@@ -648,8 +1019,8 @@ static int build_sv(TriSolve<V>* S, int n, const int* irp, const int* ja, const 
     tlower = !lower;
   }
   int rc = upload_tri(S->tl, n, tlower, sirp.data(), sja.data(), sval.data(),
-                      g_trsv_variant != 1);
-  if (rc) return rc;
+                      unit ? (const V*)nullptr : dv.data());
+  if (rc || S->tl.ntiles > 0) return rc;
   const size_t nb = sizeof(V) * (size_t)(n > 0 ? n : 1);
   hipError_t e = hipSuccess;
   V** bufs[] = {&S->xa, &S->ya};
@@ -725,6 +1096,10 @@ static int csr_sv_apply(CsrDev* m, int key, V alpha, const MultiVec* x, V beta, 
   for (int c = 0; c < x->count; c++) {
     const V* xc = (const V*)x->v + (size_t)c * x->pitch;
     V* yc = (V*)y->v + (size_t)c * y->pitch;
+    if (S->tl.ntiles > 0) {
+      if ((rc = solve_tiles<V>(S->tl, S->run, xc, nullptr, alpha, beta, yc, s))) return rc;
+      continue;
+    }
     hipLaunchKernelGGL(k_perm_gather<V>, dim3(g), dim3(kBlock), 0, s, n, S->tl.perm, xc,
                        (const V*)nullptr, S->xa);
     PSB_HIP_LAUNCH_CHECK();
@@ -756,21 +1131,28 @@ int psb_hip_ilu_alloc(void** ilu, int n, const int* lirp, const int* lja, const 
   *ilu = nullptr;
   IluDev* F = new IluDev();
   F->n = n;
-  const bool seg = g_trsv_variant != 1;
-  int rc = upload_tri(F->L, n, true, lirp, lja, lval, seg);
-  if (!rc) rc = upload_tri(F->U, n, false, uirp, uja, uval, seg);
+  int rc = PSB_HIP_SUCCESS;
+  for (TriForm form : {TRI_AUTO, TRI_TILES, TRI_LEVELS}) {   // both factors in the same form
+    free_tri(F->L);
+    free_tri(F->U);
+    rc = upload_tri(F->L, n, true, lirp, lja, lval, (const double*)nullptr, form);
+    if (!rc) rc = upload_tri(F->U, n, false, uirp, uja, uval, (const double*)nullptr, form);
+    if (rc || (F->L.ntiles > 0) == (F->U.ntiles > 0)) break;
+  }
   if (rc) {
     destroy_ilu(F);
     return rc;
   }
   const size_t nb = sizeof(double) * (size_t)(n > 0 ? n : 1);
   hipError_t e = hipSuccess;
-  double** bufs[] = {&F->d, &F->xa, &F->ya, &F->t1};
-  for (double** b : bufs)
-    if (e == hipSuccess) e = hipMalloc((void**)b, nb);
+  // both factors as tiles, or the levels of both in one graph
+  const bool tiled = F->L.ntiles > 0 && F->U.ntiles > 0;
+  double** bufs[] = {&F->d, &F->t1, &F->xa, &F->ya};
+  for (int k = 0; k < (tiled ? 2 : 4); k++)
+    if (e == hipSuccess) e = hipMalloc((void**)bufs[k], nb);
   if (e == hipSuccess && n > 0)
     e = hipMemcpy(F->d, d, sizeof(double) * (size_t)n, hipMemcpyHostToDevice);
-  if (e == hipSuccess && n > 0) {
+  if (e == hipSuccess && n > 0 && !tiled) {
     hipStream_t s = ctx().stream;
     e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
@@ -797,8 +1179,8 @@ int psb_hip_ilu_set_variant(int variant) {
 int psb_hip_ilu_segments(void* ilu, int* lower_segments, int* upper_segments) {
   IluDev* F = (IluDev*)ilu;
   if (!F) return PSB_HIP_INVALID;
-  if (lower_segments) *lower_segments = (int)F->L.segs.size();
-  if (upper_segments) *upper_segments = (int)F->U.segs.size();
+  if (lower_segments) *lower_segments = F->L.ntiles;
+  if (upper_segments) *upper_segments = F->U.ntiles;
   return PSB_HIP_SUCCESS;
 }
 
@@ -824,6 +1206,12 @@ int psb_hip_ilu_apply(void* ilu, double alpha, void* xv, double beta, void* yv) 
     return set_error(PSB_HIP_INVALID, __func__, "x/y type or size");
   if (F->n == 0) return PSB_HIP_SUCCESS;
   hipStream_t s = ctx().stream;
+  if (!F->exec) {   // t1 = L^-1 x, then y = alpha U^-1 (d .* t1) + beta y
+    int rc = solve_tiles<double>(F->L, false, (const double*)x->v, nullptr, 1.0, 0.0, F->t1, s);
+    if (!rc)
+      rc = solve_tiles<double>(F->U, false, F->t1, F->d, alpha, beta, (double*)y->v, s);
+    return rc;
+  }
   const int n = F->n, g = stream_grid(n);
   hipLaunchKernelGGL(k_perm_gather<double>, dim3(g), dim3(kBlock), 0, s, n, F->L.perm,
                      (const double*)x->v, (const double*)nullptr, F->xa);
@@ -859,10 +1247,10 @@ int psb_hip_csr_spsv_levels(void* dmat, int* levels, int* segments) {
   int nl = 0, ns = 0;
   if (m->sv && m->elem_type == PSB_HIP_TYPE_DOUBLE) {
     nl = ((TriSolve<double>*)m->sv)->tl.nlev;
-    ns = (int)((TriSolve<double>*)m->sv)->tl.segs.size();
+    ns = ((TriSolve<double>*)m->sv)->tl.ntiles;
   } else if (m->sv) {
     nl = ((TriSolve<float>*)m->sv)->tl.nlev;
-    ns = (int)((TriSolve<float>*)m->sv)->tl.segs.size();
+    ns = ((TriSolve<float>*)m->sv)->tl.ntiles;
   }
   if (levels) *levels = nl;
   if (segments) *segments = ns;

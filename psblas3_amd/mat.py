@@ -795,7 +795,7 @@ class psb_d_hip_csrg_sparse_mat(_hip_base_mat):
         return int(N.fn("psb_hip_csr_slices")(self.dev))
 
     def sv_levels(self):
-        """(levels, workgroup runs) of the prepared triangular solve, (0, 0)
+        """(levels, workgroup tiles) of the prepared triangular solve, (0, 0)
         before the first solve."""
         lv, sg = C.c_int(), C.c_int()
         N.call("psb_hip_csr_spsv_levels", self.dev, C.byref(lv), C.byref(sg))

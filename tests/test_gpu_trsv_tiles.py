@@ -1,0 +1,101 @@
+"""Triangular solves by tiles at the shapes where a tile can go wrong: ragged
+boxes, grids with one line, entries that wrap round a grid line, rows of more
+entries than a step holds in registers, rows beyond a tile's entries, more
+than 64 rows in a level, one row; every solve repeated (the solution arrays
+alternate) and equal to the oracle bit for bit."""
+import numpy as np
+import pytest
+
+import psblas3_amd as P
+from test_gpu_spsv import _bits, _tri_mat, _vec
+
+pytestmark = pytest.mark.gpu
+
+
+def _csr(n, rows, rng, lower):
+    """Triangle with the given strictly-lower column lists (mirrored for an upper
+    one), the diagonal included, diagonally dominant."""
+    irp, ja, val = [1], [], []
+    for i in range(n):
+        t = i if lower else n - 1 - i
+        c = sorted(set(rows(t)))
+        c = c if lower else [n - 1 - q for q in reversed(c)]
+        v = list(rng.uniform(-1.0, 1.0, len(c)) / max(1, len(c)))
+        c, v = (c + [i], v + [2.0]) if lower else ([i] + c, [2.0] + v)
+        ja += [q + 1 for q in c]
+        val += v
+        irp.append(len(ja) + 1)
+    return np.array(irp, np.int32), np.array(ja, np.int32), np.array(val)
+
+
+def _grid(nx, ny, nz, wrap=False):
+    def rows(t):
+        x, y, z = t % nx, t // nx % ny, t // (nx * ny)
+        c = [t - 1] if x > 0 or (wrap and t > 0) else []
+        return c + ([t - nx] if y > 0 else []) + ([t - nx * ny] if z > 0 else [])
+    return nx * ny * nz, rows
+
+
+def _random(n, w, span, wide=0):
+    rng = np.random.default_rng(n)
+    cols = [rng.integers(max(0, t - span), t, wide if wide and t % 401 == 400 else w).tolist()
+            if t else [] for t in range(n)]
+    return n, lambda t: cols[t]
+
+
+SHAPES = {"8x8x8": _grid(8, 8, 8), "9x8x17": _grid(9, 8, 17), "31x5x3": _grid(31, 5, 3),
+          "2d_49x25": _grid(49, 25, 1), "2d_24x24": _grid(24, 24, 1),
+          "wrap_16x9x4": _grid(16, 9, 4, wrap=True), "narrow_7x9x9": _grid(7, 9, 9),
+          "chain_600": (600, lambda t: [t - 1] if t else []),
+          "width4": _random(1500, 4, 40), "width6": _random(1500, 6, 600),
+          "wide_rows": _random(2500, 3, 900, wide=300),
+          "row_past_a_tile": _random(2500, 2, 2400, wide=1300),
+          "levels_of_700": (4200, lambda t: [t - 700] if t >= 700 else []), "one": (1, lambda t: [])}
+
+
+@pytest.mark.parametrize("name", list(SHAPES))
+@pytest.mark.parametrize("lower,trans,single", [(True, "N", False), (False, "N", False),
+                                                (True, "T", False), (False, "N", True)],
+                         ids=["L", "U", "LT", "U-f32"])
+def test_tiles_bitexact(gpu, orc, name, lower, trans, single):
+    print(f"[gpu] case trsv tiles {name} lower={lower} trans={trans} single={single}", flush=True)
+    n, rows = SHAPES[name]
+    dt = np.float32 if single else np.float64
+    irp, ja, val = _csr(n, rows, np.random.default_rng(5), lower)
+    a, desc = _tri_mat(irp, ja, val, lower, False, single=single)
+    for k in range(3):
+        x = orc.uniform_pm1(30 + k, n).astype(dt)
+        y0 = orc.uniform_pm1(40 + k, n).astype(dt)
+        alpha, beta = [(1.0, 0.0), (2.0, -0.5), (-1.0, 0.0)][k]
+        y = _vec(y0.copy(), single)
+        P.psb_spsm(alpha, a, _vec(x, single), beta, y, desc, trans=trans)
+        ref = orc.csr_cssv(irp, ja, val.astype(dt), x, lower=lower, trans=trans, alpha=alpha,
+                           beta=beta, y=y0)
+        assert np.array_equal(_bits(y.get_vect()), _bits(ref)), k
+    a.free()
+
+
+@pytest.mark.parametrize("single", [False, True], ids=["f64", "f32"])
+def test_tiles_nonfinite(gpu, orc, single):
+    """A right-hand side with infinities, NaN and the very pattern that marks an
+    entry as not solved yet: the solve ends, and is non-finite where the
+    oracle's is."""
+    print(f"[gpu] case trsv tiles non-finite single={single}", flush=True)
+    n, rows = _grid(11, 10, 9)
+    dt = np.float32 if single else np.float64
+    irp, ja, val = _csr(n, rows, np.random.default_rng(6), True)
+    a, desc = _tri_mat(irp, ja, val, True, False, single=single)
+    x = orc.uniform_pm1(50, n).astype(dt)
+    x[n // 2] = np.inf
+    x[n // 3] = np.nan
+    unset = np.uint32(0x7FE5A3C9) if single else np.uint64(0x7FF8A5C3E1D2B497)
+    x[n - 40] = np.array([unset]).view(dt)[0]
+    y = _vec(np.zeros(n, dt), single)
+    for _ in range(2):
+        P.psb_spsm(1.0, a, _vec(x, single), 0.0, y, desc)
+        ref = orc.csr_cssv(irp, ja, val.astype(dt), x)
+        out = y.get_vect()
+        assert np.array_equal(np.isnan(out), np.isnan(ref))
+        ok = ~np.isnan(ref)
+        assert np.array_equal(_bits(out[ok]), _bits(ref[ok]))
+    a.free()
