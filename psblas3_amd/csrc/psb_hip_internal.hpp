@@ -351,6 +351,7 @@ struct HllDev {
   int elem_type;
   int hksz, rows, nzeros, allocsize, noffs, first_index;
   int max_col;          // largest column index stored (x must be this long)
+  int max_width = 0x7fffffff;   // slots of the widest hack (rows in order)
   void* val;            // allocsize entries of elem_type
   int* ja;              // allocsize
   int* hkoffs;          // noffs + 1

@@ -81,6 +81,9 @@ inline int csr_class(int len) {
   return c;
 }
 
+// widest hack of the multi-RHS product that runs column by column
+constexpr int kSpmmWidth = 9;
+
 // ------------------------------------------------------------------ HLL SpMV
 // HK > 0: compile-time hack size (32 or 64); HK == 0: any hksz.  ord: the
 // block order (launch, chunked XCD or plane-tile).
@@ -429,6 +432,129 @@ __global__ __launch_bounds__(kBlock) void k_hll_spmm_pair(int nr, int hksz, int 
         if (row < nr) store_y(yq, row, alpha, a0[q], beta);
         if (row + 1 < nr) store_y(yq, row + 1, alpha, a1[q], beta);
       }
+    }
+  }
+}
+
+// The multi-RHS product of narrow rows (hack width <= W), column by column:
+// each lane keeps the slots of its R rows in registers (byte offsets into a
+// column of x, values) and for every column gathers the W entries, sums in
+// slot order (the bits of k_hll_spmm) and stores y.  The slots of a column
+// run back to back, so the entries that neighbouring slots share (columns
+// r-1, r and r+1 of a stencil) are in L1, where the column groups above came
+// back to a line after 8 to 32 other columns; and no column needs an
+// accumulator of its own.  R = 2 (FP64): the two rows' entries in one 16-byte
+// load on the slots where they are adjacent on every lane (an 8-byte aligned
+// 16-byte load), else two loads.  Bound by its traffic: L = 100, k = 32 moves
+// 1.1 GB (x fetched 3 times past L2) in 195 us, 5.7 TB/s.  Against the column
+// groups, 7-point stencil, vectors past the caches: FP64 L = 100 k = 32 209 -> 195
+// us, L = 130 k = 4 70 -> 62, L = 160 k = 8 205 -> 204; FP32 (R = 1) L = 120 k = 16
+// 138 -> 80 us; FP64 in the caches L = 50 k = 32 31 -> 22 us.  Measured slower:
+// two columns at a time (occupancy; L = 160 k = 8 202 against 192 us in the
+// caches), columns in groups of 4, 8 or 16 with the matrix read again for each
+// (L = 100 k = 32 229, 203 and 196 us), temporal stores of y (204 us).
+template <typename T, int R, int W, bool IDX16>
+__global__ __launch_bounds__(kBlock) void k_hll_spmm_cols(int nr, int hksz, int nlog,
+                                                          const int* __restrict__ hkoffs,
+                                                          const int* __restrict__ ja,
+                                                          const short* __restrict__ res16,
+                                                          const int* __restrict__ base16,
+                                                          const T* __restrict__ val,
+                                                          const T* __restrict__ x, int ldx,
+                                                          T alpha, T beta, T* __restrict__ y,
+                                                          int ldy, int ncols, BlockOrder ord) {
+  const int lb = order_block(ord, nlog);
+  if (lb >= nlog) return;
+  const int row = lb * (R * kBlock) + R * (int)threadIdx.x;
+  const int last = R == 2 ? (nr - 1) & ~1 : nr - 1;
+  const int r = row < last ? row : last;
+  const int hk = r / hksz;
+  const int lane = r - hk * hksz;
+  const int off0 = hkoffs[hk];
+  const int w = (hkoffs[hk + 1] - off0) / hksz;
+  unsigned o[R][W];
+  T v[R][W];
+  unsigned adj = 0;   // slots whose two entries are adjacent on every lane
+#pragma unroll
+  for (int k = 0; k < W; k++) {
+    // past the width: the last slot again, its product dropped; an empty hack
+    // gathers x's first entry and drops it
+    const int jj = k < w ? k : (w > 0 ? w - 1 : 0);
+    const size_t e = (size_t)off0 + (size_t)jj * hksz + lane;
+    int c0 = 0, c1 = 0;
+    vec2<T> vv = {T(0), T(0)};
+    if (w > 0) {
+      if constexpr (R == 2) {
+        if (IDX16) {
+          const int b = r + base16[off0 / hksz + jj];
+          const vec2<short> s = ld_stream(reinterpret_cast<const vec2<short>*>(res16 + e));
+          c0 = b + s.x;
+          c1 = b + 1 + s.y;
+        } else {
+          const vec2<int> s = ld_stream(reinterpret_cast<const vec2<int>*>(ja + e));
+          c0 = s.x - 1;
+          c1 = s.y - 1;
+        }
+        vv = ld_stream(reinterpret_cast<const vec2<T>*>(val + e));
+      } else {
+        c0 = IDX16 ? r + base16[off0 / hksz + jj] + (int)ld_stream(res16 + e)
+                   : ld_stream(ja + e) - 1;
+        vv.x = ld_stream(val + e);
+      }
+    }
+    o[0][k] = (unsigned)c0 * (unsigned)sizeof(T);
+    v[0][k] = vv.x;
+    if constexpr (R == 2) {
+      o[1][k] = (unsigned)c1 * (unsigned)sizeof(T);
+      v[1][k] = vv.y;
+      if (__all(c1 == c0 + 1)) adj |= 1u << k;
+    }
+  }
+  struct __attribute__((packed, aligned(sizeof(T)))) Two {
+    T a, b;
+  };
+  const bool yal = R == 2 && (reinterpret_cast<uintptr_t>(y) & (2 * sizeof(T) - 1)) == 0 &&
+                   (ldy & 1) == 0;
+  for (int q = 0; q < ncols; q++) {
+    const char* xq = reinterpret_cast<const char*>(x + (size_t)q * ldx);
+    T xv[R][W];
+#pragma unroll
+    for (int k = 0; k < W; k++) {
+      if (R == 2 && (adj >> k & 1)) {
+        const Two t = *reinterpret_cast<const Two*>(xq + o[0][k]);
+        xv[0][k] = t.a;
+        xv[R - 1][k] = t.b;
+      } else {
+#pragma unroll
+        for (int i = 0; i < R; i++) xv[i][k] = *reinterpret_cast<const T*>(xq + o[i][k]);
+      }
+    }
+    T acc[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      acc[i] = T(0);
+#pragma unroll
+      for (int k = 0; k < W; k++) {
+        const T t = fma(v[i][k], xv[i][k], acc[i]);
+        acc[i] = k < w ? t : acc[i];
+      }
+    }
+    T* yq = y + (size_t)q * ldy;
+    if (R == 2 && row + 1 < nr && yal) {
+      T r0 = alpha * acc[0], r1 = alpha * acc[R - 1];
+      if (beta != T(0)) {
+        const vec2<T> yo = *reinterpret_cast<const vec2<T>*>(yq + row);
+        r0 = fma(beta, yo.x, r0);
+        r1 = fma(beta, yo.y, r1);
+      }
+      vec2<T> yn;
+      yn.x = r0;
+      yn.y = r1;
+      __builtin_nontemporal_store(yn, reinterpret_cast<vec2<T>*>(yq + row));
+    } else {
+#pragma unroll
+      for (int i = 0; i < R; i++)
+        if (row + i < nr) store_y(yq, row + i, alpha, acc[i], beta);
     }
   }
 }
@@ -1099,6 +1225,12 @@ static int min_index(const int* ja, int64_t n) {
   return n ? m : 1;
 }
 
+static int max_hack_width(const int* hkoffs, int noffs, int hksz) {
+  int w = 0;
+  for (int h = 0; h < noffs; h++) w = std::max(w, (hkoffs[h + 1] - hkoffs[h]) / hksz);
+  return w;
+}
+
 static int check_vectors(const MultiVec* x, const MultiVec* y, int elem_type, int need_x,
                          int need_y) {
   if (!x || !y) return PSB_HIP_INVALID;
@@ -1267,6 +1399,36 @@ static int hll_launch(const HllDev* m, const TV* val, const T* x, T alpha, T bet
   return PSB_HIP_SUCCESS;
 }
 
+// One launch of k_hll_spmm_cols with the smallest W that holds the matrix's
+// widest hack.
+template <typename T, int R>
+static int hll_spmm_cols(const HllDev* m, const T* val, const T* x, int ldx, T alpha, T beta,
+                         T* y, int ldy, int ncols) {
+  const int nlog = grid_for(m->rows, R * kBlock);
+  const BlockOrder o = hll_order(m, true, R * kBlock, nlog);
+  const bool i16 = hll_use_idx16(m);
+  dim3 grid(order_grid(o, nlog)), blk(kBlock);
+  hipStream_t s = ctx().stream;
+#define PSB_SPMMC_CASE(W)                                                                      \
+  do {                                                                                         \
+    if (i16)                                                                                   \
+      hipLaunchKernelGGL((k_hll_spmm_cols<T, R, W, true>), grid, blk, 0, s, m->rows, m->hksz,  \
+                         nlog, m->hkoffs, m->ja, m->res16, m->base16, val, x, ldx, alpha, beta, \
+                         y, ldy, ncols, o);                                                    \
+    else                                                                                       \
+      hipLaunchKernelGGL((k_hll_spmm_cols<T, R, W, false>), grid, blk, 0, s, m->rows, m->hksz, \
+                         nlog, m->hkoffs, m->ja, m->res16, m->base16, val, x, ldx, alpha, beta, \
+                         y, ldy, ncols, o);                                                    \
+  } while (0)
+  if (m->max_width <= 3) PSB_SPMMC_CASE(3);
+  else if (m->max_width <= 5) PSB_SPMMC_CASE(5);
+  else if (m->max_width <= 7) PSB_SPMMC_CASE(7);
+  else PSB_SPMMC_CASE(kSpmmWidth);
+#undef PSB_SPMMC_CASE
+  PSB_HIP_LAUNCH_CHECK();
+  return PSB_HIP_SUCCESS;
+}
+
 template <typename T>
 static int hll_spmm_launch(const HllDev* m, const T* val, const T* x, int ldx, T alpha, T beta,
                            T* y, int ldy, int ncols) {
@@ -1278,6 +1440,20 @@ static int hll_spmm_launch(const HllDev* m, const T* val, const T* x, int ldx, T
       if (rc) return rc;
     }
     return PSB_HIP_SUCCESS;
+  }
+  // narrow rows (stencils of up to 9 points): column by column.  Byte offsets
+  // into a column are 32-bit.  FP32 rows of scattered columns (no 16-bit
+  // offsets) keep the groups of 8 up to 16 columns: every gather is a line of
+  // its own there, and two columns of a slot share the index arithmetic (6
+  // random columns a row, n = 1M, k = 4, 8 and 16: 218, 482 and 1015 us against
+  // 261, 537 and 1162; k = 24 2214 against 1809; FP64 k = 8 693 against 575).
+  const bool scattered = !hll_use_idx16(m);
+  if (m->max_width <= kSpmmWidth && ncols > 1 &&
+      !(scattered && sizeof(T) == 4 && m->hksz % 2 == 0 && ncols <= 16) &&
+      (uint64_t)m->max_col * sizeof(T) <= 0xffffffffull) {
+    if (sizeof(T) == 8 && m->hksz % 2 == 0)
+      return hll_spmm_cols<T, 2>(m, val, x, ldx, alpha, beta, y, ldy, ncols);
+    return hll_spmm_cols<T, 1>(m, val, x, ldx, alpha, beta, y, ldy, ncols);
   }
   hipStream_t s = ctx().stream;
   // two rows per lane, columns in groups of up to 8 inside the launch, up to
@@ -1817,6 +1993,7 @@ int psb_hip_hll_write(void* dmat, const void* val, const int* ja, const int* hko
   if (m->allocsize > 0 && min_index(ja, m->allocsize) < 1)
     return set_error(PSB_HIP_INVALID, __func__, "ja < 1");
   m->max_col = max_index(ja, m->allocsize);
+  m->max_width = max_hack_width(hkoffs, m->noffs, m->hksz);
   size_t es = elem_size(m->elem_type);
   PSB_HIP_CHECK(hipMemcpyAsync(m->val, val, (size_t)m->allocsize * es, hipMemcpyHostToDevice, s));
   PSB_HIP_CHECK(hipMemcpyAsync(m->ja, ja, (size_t)m->allocsize * 4, hipMemcpyHostToDevice, s));
@@ -1885,6 +2062,7 @@ int psb_hip_hll_copy_coo(int nr, int nc, int nza, int hksz, int noffs, int isz, 
   int mn = min_index(ja, nza), mx = max_index(ja, nza);
   if (nza > 0 && (mn < 1 || mx > nc)) return set_error(PSB_HIP_INVALID, __func__, "ja out of range");
   m->max_col = std::max(mx, nr);  // padding of the last hack uses ja = nr
+  m->max_width = max_hack_width(hoffs, noffs, hksz);
   hipStream_t s = ctx().stream;
   PSB_HIP_CHECK(hipStreamSynchronize(s));
   hll_drop_sorted(m);
