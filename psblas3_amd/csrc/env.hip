@@ -48,10 +48,10 @@ static int init_device(int dev) {
   // default priority stream: the library stream every kernel is launched on
   PSB_HIP_CHECK(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
   PSB_HIP_CHECK(hipMalloc(&c.red_partials, sizeof(double) * kRedBlocks * 8));
-  PSB_HIP_CHECK(hipMalloc(&c.red_counter, sizeof(unsigned int) * 64));
+  PSB_HIP_CHECK(hipMalloc(&c.red_counter, sizeof(unsigned int) * 64 * kRedCounter));
   PSB_HIP_CHECK(hipMalloc(&c.red_result, sizeof(double) * 64));
-  PSB_HIP_CHECK(hipMemset(c.red_counter, 0, sizeof(unsigned int) * 64));
-  PSB_HIP_CHECK(hipHostMalloc(&c.host_result, sizeof(double) * 64, hipHostMallocDefault));
+  PSB_HIP_CHECK(hipMemset(c.red_counter, 0, sizeof(unsigned int) * 64 * kRedCounter));
+  PSB_HIP_CHECK(hipHostMalloc(&c.host_result, sizeof(double) * 64, hipHostMallocCoherent));
   void* sp = nullptr;
   PSB_HIP_CHECK(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
   c.scratch = (char*)sp;
