@@ -10,12 +10,14 @@
 // queued after convergence see the flag and return at once, so the iterate
 // and the iteration count are exactly those of the stopping iteration.
 //
-// Reductions: each block of a fused kernel stores its partial sums; a
-// one-block finalisation kernel then adds the partials in index order and
-// updates the scalars (deterministic run to run).  The kernel boundary makes
-// the partials of every XCD visible; a device-scope fence per block would
-// write back the XCD's whole L2 after the fused kernel's stores, which
-// measured 1.4x slower on MI355X.
+// Reductions: each block of a fused kernel stores its partial sums and the
+// launch's last block waits for them, adds them in index order and updates the
+// scalars (deterministic run to run): the finalisations F_* below run at the
+// end of their kernel.  The partials are agent-scope stores and loads, which pass the
+// XCDs' L2s by; a device-scope fence per block would write back the XCD's whole
+// L2 after the fused kernel's stores, which measured 1.4x slower on MI355X.
+// Kernels of more than kFoldGrid blocks leave their partials to a one-block
+// finalisation kernel, whose time does not count beside theirs.
 //
 // CG per iteration:        K_p   p = z | z + beta*p
 //                          K_q   q = A*p, partial p.q        F_q  sigma, alpha
@@ -37,6 +39,12 @@
 namespace psbhip {
 
 constexpr int kMaxGrid = 32768;  // blocks of a fused kernel (partials per reduction)
+// Blocks up to which a fused kernel's finalisation is folded into it: above,
+// the one tail over all partials takes as long as a k_fin launch (FP64 CG at
+// L = 140, 5360 blocks, 44.6 ms folding up to 1024 blocks, 43.9 up to 4096,
+// 43.2 up to 8192; mixed CG at L = 190, 26,800 blocks, 74.2 ms up to 8192 and
+// 16384, 76.6 up to 32768).
+constexpr int kFoldGrid = 8192;
 
 struct KState {
   // scalars of the recurrence
@@ -259,20 +267,10 @@ __device__ __forceinline__ double fin_sum(const double* __restrict__ partials, i
   return r;
 }
 
+// The scalars after a kernel with the sums v (one thread).
 template <int OP, int NP>
-__global__ __launch_bounds__(kFin) void k_fin(KState* st, const double* __restrict__ partials,
-                                              int nb, double* hist,
-                                              const double* __restrict__ aux) {
-  if (OP == FIN_RESTART_CG || OP == FIN_RESTART_BI) {
-    if (st->done) return;
-  } else if (OP != FIN_BNORM && OP != FIN_RU_RESET && OP != FIN_RU_RESET_FIRST) {
-    if (halted(st)) return;
-  }
-  __shared__ double lds[kFin / kWave];
-  double v[NP];
-#pragma unroll
-  for (int p = 0; p < NP; p++) v[p] = fin_sum(partials + p * kMaxGrid, nb, lds);
-  if (threadIdx.x != 0) return;
+__device__ __forceinline__ void fin_apply(KState* st, const double (&v)[NP], double* hist,
+                                          const double* __restrict__ aux) {
   const double v1 = v[NP - 1];  // second partial (NP == 2)
   if (OP == FIN_BNORM) {
     st->bnorm = sqrt(v[0]);
@@ -383,6 +381,89 @@ __global__ __launch_bounds__(kFin) void k_fin(KState* st, const double* __restri
   }
 }
 
+template <int OP, int NP>
+__global__ __launch_bounds__(kFin) void k_fin(KState* st, const double* __restrict__ partials,
+                                              int nb, double* hist,
+                                              const double* __restrict__ aux) {
+  if (OP == FIN_RESTART_CG || OP == FIN_RESTART_BI) {
+    if (st->done) return;
+  } else if (OP != FIN_BNORM && OP != FIN_RU_RESET && OP != FIN_RU_RESET_FIRST) {
+    if (halted(st)) return;
+  }
+  __shared__ double lds[kFin / kWave];
+  double v[NP];
+#pragma unroll
+  for (int p = 0; p < NP; p++) v[p] = fin_sum(partials + p * kMaxGrid, nb, lds);
+  if (threadIdx.x != 0) return;
+  fin_apply<OP, NP>(st, v, hist, aux);
+}
+
+// Where a fused kernel's sums go: the partials of a k_fin launch, or, for a
+// folded finalisation, the fold slots (2 * kFoldGrid doubles that hold
+// kUnsetBits between uses; null: not folded).
+struct Fin {
+  double* partials;
+  double* fold;
+  double* hist;
+};
+
+// polls of a fold slot before the wait is given up (the sum is then NaN)
+constexpr int kFoldPolls = 1 << 22;
+
+// The end of a fused kernel: every block stores its NP partial sums.  Folded,
+// the launch's last block waits for the others' (a slot is there once it holds
+// something else than kUnsetBits: no counter, no fence, and no block but this
+// one waits for a store of its own), adds them in index order, sets the slots
+// back and applies the finalisation.  The wait ends: no other block waits for
+// anything, and this one holds one block's place.
+template <int OP, int NP>
+__device__ __forceinline__ void finish(double (&v)[NP], const Fin& f, KState* st) {
+  typedef unsigned long long U;
+  __shared__ double lds[kBlock / kWave];
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    v[p] = block_sum(v[p], lds);
+    if (threadIdx.x != 0) continue;
+    if (f.fold) {
+      U u = __builtin_bit_cast(U, v[p]);
+      if (u == kUnsetBits) u = 0x7ff8000000000000ull;
+      __hip_atomic_store(reinterpret_cast<U*>(f.fold + p * kFoldGrid + blockIdx.x), u,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      f.partials[p * kMaxGrid + blockIdx.x] = v[p];
+    }
+  }
+  if (!f.fold || blockIdx.x != gridDim.x - 1) return;
+  const int nb = (int)gridDim.x;
+  double t[NP];
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    U* slot = reinterpret_cast<U*>(f.fold + p * kFoldGrid);
+    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = threadIdx.x; b < nb; b += 4 * kBlock) {
+      U u[4];
+      for (int polls = 0;; polls++) {
+        bool all = true;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int i = b + k * kBlock < nb ? b + k * kBlock : b;
+          u[k] = __hip_atomic_load(slot + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          all = all && u[k] != kUnsetBits;
+        }
+        if (all || polls > kFoldPolls) break;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (b + k * kBlock < nb) {
+          a[k] += __builtin_bit_cast(double, u[k]);
+          slot[b + k * kBlock] = kUnsetBits;
+        }
+    }
+    t[p] = block_sum((a[0] + a[1]) + (a[2] + a[3]), lds);
+  }
+  if (threadIdx.x == 0) fin_apply<OP, NP>(st, t, f.hist, nullptr);
+}
+
 // --------------------------------------------------------------- restart / norms
 // r = b - A*x, then (CG) z = d.*r with partials r.r, r.z or (BiCGSTAB) q = r
 // with partial r.r.
@@ -445,7 +526,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_p(int n, const T* __restrict__ z,
 
 template <typename T, class M, int R>
 __global__ __launch_bounds__(kBlock) void k_cg_q(M m, const T* __restrict__ p, T* __restrict__ q,
-                                                 const KState* st, double* partials) {
+                                                 KState* st, Fin f) {
   if (halted(st)) return;
   double v[1] = {0.0};
   // p(row) for the p.q partial comes from the product's own gather at the
@@ -454,26 +535,24 @@ __global__ __launch_bounds__(kBlock) void k_cg_q(M m, const T* __restrict__ p, T
     store_prod(q, row, ax);
     v[0] += (double)xrow * (double)ax;
   })
-  store_partials<1>(v, partials);
+  finish<FIN_CG_Q, 1>(v, f, st);
 }
 
 // a.b partial (the CSR path: the product runs through the CSR kernels)
-template <typename T>
+template <typename T, int OP>
 __global__ __launch_bounds__(kBlock) void k_dot(int n, const T* __restrict__ a,
-                                                const T* __restrict__ b, const KState* st,
-                                                double* partials) {
+                                                const T* __restrict__ b, KState* st, Fin f) {
   if (halted(st)) return;
   double v[1] = {0.0};
   PSB_VEC_LOOP(n, { v[0] += vdot<T>(ldv(a + i), ldv(b + i)); },
                { v[0] += (double)a[i] * (double)b[i]; })
-  store_partials<1>(v, partials);
+  finish<OP, 1>(v, f, st);
 }
 
 // t.t and t.s partials (the CSR path of BiCGSTAB)
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_dot2(int n, const T* __restrict__ t,
-                                                 const T* __restrict__ s, const KState* st,
-                                                 double* partials) {
+                                                 const T* __restrict__ s, KState* st, Fin f) {
   if (halted(st)) return;
   double v[2] = {0.0, 0.0};
   PSB_VEC_LOOP(n,
@@ -486,14 +565,13 @@ __global__ __launch_bounds__(kBlock) void k_dot2(int n, const T* __restrict__ t,
                  v[0] += (double)t[i] * (double)t[i];
                  v[1] += (double)t[i] * (double)s[i];
                })
-  store_partials<2>(v, partials);
+  finish<FIN_BI_T, 2>(v, f, st);
 }
 
-template <typename T>
+template <typename T, int OP>
 __global__ __launch_bounds__(kBlock) void k_cg_x(int n, T* __restrict__ x, T* r,
                                                  const T* __restrict__ p, const T* __restrict__ q,
-                                                 const T* __restrict__ d, T* z, const KState* st,
-                                                 double* partials) {
+                                                 const T* __restrict__ d, T* z, KState* st, Fin f) {
   if (halted(st)) return;
   const T alpha = (T)st->alpha;
   double v[2] = {0.0, 0.0};
@@ -519,7 +597,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_x(int n, T* __restrict__ x, T* r,
                  v[0] += (double)ri * (double)ri;
                  v[1] += (double)ri * (double)zi;
                })
-  store_partials<2>(v, partials);
+  finish<OP, 2>(v, f, st);
 }
 
 // --------------------------------------------------------------- BiCGSTAB kernels
@@ -546,15 +624,14 @@ __global__ __launch_bounds__(kBlock) void k_bi_a(int n, const T* __restrict__ r,
 
 template <typename T, class M, int R>
 __global__ __launch_bounds__(kBlock) void k_bi_v(M m, const T* __restrict__ f, T* __restrict__ v,
-                                                 const T* __restrict__ q, const KState* st,
-                                                 double* partials) {
+                                                 const T* __restrict__ q, KState* st, Fin fin) {
   if (halted(st)) return;
   double s[1] = {0.0};
   PSB_TILE_ROWS(R, m, f, {
     store_prod(v, row, ax);
     s[0] += (double)q[row] * (double)ax;
   })
-  store_partials<1>(s, partials);
+  finish<FIN_BI_V, 1>(s, fin, st);
 }
 
 template <typename T>
@@ -578,8 +655,7 @@ __global__ __launch_bounds__(kBlock) void k_bi_s(int n, const T* __restrict__ r,
 
 template <typename T, class M, int R>
 __global__ __launch_bounds__(kBlock) void k_bi_t(M m, const T* __restrict__ z, T* __restrict__ t,
-                                                 const T* __restrict__ s, const KState* st,
-                                                 double* partials) {
+                                                 const T* __restrict__ s, KState* st, Fin fin) {
   if (halted(st)) return;
   double v[2] = {0.0, 0.0};
   PSB_TILE_ROWS(R, m, z, {
@@ -587,15 +663,14 @@ __global__ __launch_bounds__(kBlock) void k_bi_t(M m, const T* __restrict__ z, T
     v[0] += (double)ax * (double)ax;
     v[1] += (double)ax * (double)s[row];
   })
-  store_partials<2>(v, partials);
+  finish<FIN_BI_T, 2>(v, fin, st);
 }
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_bi_x(int n, T* __restrict__ x, T* __restrict__ r,
                                                  const T* __restrict__ f, const T* __restrict__ z,
                                                  const T* __restrict__ s, const T* __restrict__ t,
-                                                 const T* __restrict__ q, const KState* st,
-                                                 double* partials) {
+                                                 const T* __restrict__ q, KState* st, Fin fin) {
   if (halted(st)) return;
   const T alpha = (T)st->alpha, omega = (T)st->omega;
   double v[2] = {0.0, 0.0};
@@ -615,7 +690,7 @@ __global__ __launch_bounds__(kBlock) void k_bi_x(int n, T* __restrict__ x, T* __
                  v[0] += (double)ri * (double)ri;
                  v[1] += (double)q[i] * (double)ri;
                })
-  store_partials<2>(v, partials);
+  finish<FIN_BI_X, 2>(v, fin, st);
 }
 
 // --------------------------------------------------------------- mixed precision helpers
@@ -645,6 +720,11 @@ __global__ __launch_bounds__(kBlock) void k_d2s_vec(int n, const double* __restr
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_zero(int n, T* __restrict__ a) {
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) a[i] = T(0);
+}
+
+__global__ __launch_bounds__(kBlock) void k_unset(int n, unsigned long long* __restrict__ a) {
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
+    a[i] = kUnsetBits;
 }
 
 // Reliable updates: the FP32 CG step is k_cg_x; its finalisation (FIN_RU_X)
@@ -689,6 +769,7 @@ struct Solver {
   int posted = 0;                // state copies queued so far
   double* partials = nullptr;
   double* hist = nullptr;
+  double* fold = nullptr;        // slots of folded finalisations, kUnsetBits between uses
   std::vector<void*> bufs;
   hipStream_t stream = nullptr;
   // allocation-free mode: device buffers are carved from the library's
@@ -785,11 +866,27 @@ static Mats<T> make_views(Solver& s) {
     else PSB_PRODUCT(KERN, T, HllView<T>, s, g, view, __VA_ARGS__);                         \
   } while (0)
 
+// Whether a fused kernel of nb blocks applies its finalisation itself, and
+// what it is given to do so.  Against a k_fin launch (4.4-4.7 us) after every
+// one of them: FP64 CG at L = 30 2.52 -> 1.95 ms, at L = 100 16.2 -> 14.7 ms,
+// BiCGSTAB at L = 40 3.71 -> 2.85 ms, mixed CG at L = 80 7.65 -> 6.15 ms.  With
+// the last block found by an arrival counter instead (every block waiting for
+// its own stores first) L = 100 took 16.4 ms.
+static bool folds(const Solver& s, int nb) { return s.fold && nb <= kFoldGrid; }
+static Fin fin_args(const Solver& s, int nb) {
+  return Fin{s.partials, folds(s, nb) ? s.fold : nullptr, s.hist};
+}
 // One-block finalisation after a fused kernel launched on nb blocks.
 template <int OP, int NP>
 static void fin(Solver& s, int nb, const double* aux = nullptr) {
   hipLaunchKernelGGL((k_fin<OP, NP>), dim3(1), dim3(kFin), 0, s.stream, s.st, s.partials, nb,
                      s.hist, aux);
+}
+
+// The same where the kernel has not folded it.
+template <int OP, int NP>
+static void fin_after(Solver& s, int nb) {
+  if (!folds(s, nb)) fin<OP, NP>(s, nb);
 }
 
 static int csr_product(Solver& s, const void* x, void* y) {
@@ -836,21 +933,21 @@ static int cg_iter(Solver& s, const Mats<T>& m, T* x, T* r, T* p, T* q, const T*
   const int gs = spmv_grid(n, s.rpl);
   hipLaunchKernelGGL((k_cg_p<T>), gv, blk, 0, s.stream, n, (const T*)z, p, s.st);
   if (s.fmt == FMT_HLL) {
-    PSB_HLL_PRODUCT(k_cg_q, T, s, gs, m.hll, (const T*)p, q, s.st, s.partials);
-    fin<FIN_CG_Q, 1>(s, gs);
+    PSB_HLL_PRODUCT(k_cg_q, T, s, gs, m.hll, (const T*)p, q, s.st, fin_args(s, gs));
+    fin_after<FIN_CG_Q, 1>(s, gs);
   } else if (s.fmt == FMT_ELL) {
-    PSB_PRODUCT(k_cg_q, T, EllView<T>, s, gs, m.ell, (const T*)p, q, s.st, s.partials);
-    fin<FIN_CG_Q, 1>(s, gs);
+    PSB_PRODUCT(k_cg_q, T, EllView<T>, s, gs, m.ell, (const T*)p, q, s.st, fin_args(s, gs));
+    fin_after<FIN_CG_Q, 1>(s, gs);
   } else {
     int rc = csr_product(s, p, q);
     if (rc) return rc;
-    hipLaunchKernelGGL((k_dot<T>), gv, blk, 0, s.stream, n, (const T*)p, (const T*)q, s.st,
-                       s.partials);
-    fin<FIN_CG_Q, 1>(s, gv.x);
+    hipLaunchKernelGGL((k_dot<T, FIN_CG_Q>), gv, blk, 0, s.stream, n, (const T*)p,
+                       (const T*)q, s.st, fin_args(s, gv.x));
+    fin_after<FIN_CG_Q, 1>(s, gv.x);
   }
-  hipLaunchKernelGGL((k_cg_x<T>), gv, blk, 0, s.stream, n, x, r, (const T*)p, (const T*)q, d, z,
-                     s.st, s.partials);
-  fin<FIN_CG_X, 2>(s, gv.x);
+  hipLaunchKernelGGL((k_cg_x<T, FIN_CG_X>), gv, blk, 0, s.stream, n, x, r, (const T*)p,
+                     (const T*)q, d, z, s.st, fin_args(s, gv.x));
+  fin_after<FIN_CG_X, 2>(s, gv.x);
   PSB_HIP_LAUNCH_CHECK();
   return PSB_HIP_SUCCESS;
 }
@@ -865,39 +962,39 @@ static int bi_iter(Solver& s, const Mats<T>& m, T* x, T* r, T* q, T* p, T* v, T*
                      s.st);
   if (s.fmt == FMT_HLL) {
     PSB_HLL_PRODUCT(k_bi_v, T, s, gs, m.hll, (const T*)f, v, (const T*)q, s.st,
-                s.partials);
-    fin<FIN_BI_V, 1>(s, gs);
+                fin_args(s, gs));
+    fin_after<FIN_BI_V, 1>(s, gs);
   } else if (s.fmt == FMT_ELL) {
     PSB_PRODUCT(k_bi_v, T, EllView<T>, s, gs, m.ell, (const T*)f, v, (const T*)q, s.st,
-                s.partials);
-    fin<FIN_BI_V, 1>(s, gs);
+                fin_args(s, gs));
+    fin_after<FIN_BI_V, 1>(s, gs);
   } else {
     int rc = csr_product(s, f, v);
     if (rc) return rc;
-    hipLaunchKernelGGL((k_dot<T>), gv, blk, 0, s.stream, n, (const T*)q, (const T*)v, s.st,
-                       s.partials);
-    fin<FIN_BI_V, 1>(s, gv.x);
+    hipLaunchKernelGGL((k_dot<T, FIN_BI_V>), gv, blk, 0, s.stream, n, (const T*)q,
+                       (const T*)v, s.st, fin_args(s, gv.x));
+    fin_after<FIN_BI_V, 1>(s, gv.x);
   }
   hipLaunchKernelGGL((k_bi_s<T>), gv, blk, 0, s.stream, n, (const T*)r, (const T*)v, d, sv, z,
                      s.st);
   if (s.fmt == FMT_HLL) {
     PSB_HLL_PRODUCT(k_bi_t, T, s, gs, m.hll, (const T*)z, t, (const T*)sv, s.st,
-                s.partials);
-    fin<FIN_BI_T, 2>(s, gs);
+                fin_args(s, gs));
+    fin_after<FIN_BI_T, 2>(s, gs);
   } else if (s.fmt == FMT_ELL) {
     PSB_PRODUCT(k_bi_t, T, EllView<T>, s, gs, m.ell, (const T*)z, t, (const T*)sv, s.st,
-                s.partials);
-    fin<FIN_BI_T, 2>(s, gs);
+                fin_args(s, gs));
+    fin_after<FIN_BI_T, 2>(s, gs);
   } else {
     int rc = csr_product(s, z, t);
     if (rc) return rc;
     hipLaunchKernelGGL((k_dot2<T>), gv, blk, 0, s.stream, n, (const T*)t, (const T*)sv, s.st,
-                       s.partials);
-    fin<FIN_BI_T, 2>(s, gv.x);
+                       fin_args(s, gv.x));
+    fin_after<FIN_BI_T, 2>(s, gv.x);
   }
   hipLaunchKernelGGL((k_bi_x<T>), gv, blk, 0, s.stream, n, x, r, (const T*)f, (const T*)z,
-                     (const T*)sv, (const T*)t, (const T*)q, s.st, s.partials);
-  fin<FIN_BI_X, 2>(s, gv.x);
+                     (const T*)sv, (const T*)t, (const T*)q, s.st, fin_args(s, gv.x));
+  fin_after<FIN_BI_X, 2>(s, gv.x);
   PSB_HIP_LAUNCH_CHECK();
   return PSB_HIP_SUCCESS;
 }
@@ -1036,6 +1133,15 @@ static int describe(Solver& s, int method, int fmt, void* dmat) {
   return PSB_HIP_SUCCESS;
 }
 
+constexpr size_t kFoldBytes = sizeof(double) * 2 * kFoldGrid;
+// by a kernel: a caller may capture the solve
+static int clear_fold(Solver& s) {
+  hipLaunchKernelGGL(k_unset, dim3(stream_grid(2 * kFoldGrid)), dim3(kBlock), 0, s.stream,
+                     2 * kFoldGrid, reinterpret_cast<unsigned long long*>(s.fold));
+  PSB_HIP_LAUNCH_CHECK();
+  return PSB_HIP_SUCCESS;
+}
+
 // State, partials and history buffers plus the host mirror and events
 // (carved from the scratch array and borrowed from the context when
 // s.borrowed is set).
@@ -1053,6 +1159,7 @@ static int setup_state(Solver& s, int itmax) {
     s.ev[1] = ctx().scratch_ev[1];
     return PSB_HIP_SUCCESS;
   }
+  if ((rc = s.alloc((void**)&s.fold, kFoldBytes)) || (rc = clear_fold(s))) return rc;
   PSB_HIP_CHECK(hipHostMalloc((void**)&s.hst, sizeof(KState), hipHostMallocDefault));
   PSB_HIP_CHECK(hipHostMalloc((void**)&s.ring, 2 * sizeof(KState), hipHostMallocDefault));
   for (hipEvent_t& e : s.ev) PSB_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -1151,14 +1258,14 @@ static int mixed_reliable(HllDev* h, const double* b, double* x, const double* d
         hipLaunchKernelGGL((k_cg_p<float>), gv, blk, 0, stream, n, (const float*)z, p, inner.st);
         if (m32.hll.hksz == 64)
           hipLaunchKernelGGL((k_cg_q<float, HllView64<float>, 1>), dim3(gsp), blk, 0, stream,
-                             as64(m32.hll), (const float*)p, q, inner.st, inner.partials);
+                             as64(m32.hll), (const float*)p, q, inner.st, fin_args(inner, gsp));
         else
           hipLaunchKernelGGL((k_cg_q<float, HllView<float>, 1>), dim3(gsp), blk, 0, stream,
-                             m32.hll, (const float*)p, q, inner.st, inner.partials);
-        fin<FIN_CG_Q, 1>(inner, gsp);
-        hipLaunchKernelGGL((k_cg_x<float>), gv, blk, 0, stream, n, x32, r, (const float*)p,
-                           (const float*)q, (const float*)d, z, inner.st, inner.partials);
-        fin<FIN_RU_X, 2>(inner, gv.x);
+                             m32.hll, (const float*)p, q, inner.st, fin_args(inner, gsp));
+        fin_after<FIN_CG_Q, 1>(inner, gsp);
+        hipLaunchKernelGGL((k_cg_x<float, FIN_RU_X>), gv, blk, 0, stream, n, x32, r, (const float*)p,
+                           (const float*)q, (const float*)d, z, inner.st, fin_args(inner, gv.x));
+        fin_after<FIN_RU_X, 2>(inner, gv.x);
       }
       PSB_HIP_LAUNCH_CHECK();
       return post_state(inner);
@@ -1333,6 +1440,11 @@ int psb_hip_krylov_fused_noalloc(int method, int fmt, void* dmat, void* diag, vo
   s.arena = c.scratch;
   s.arena_left = c.scratch_bytes;
   if ((rc = setup_state(s, itmax))) return rc;
+  // the slots of the folded finalisations where the solve leaves room for them
+  // (its own buffers decide what is too large)
+  if (need + align256(kFoldBytes) <= c.scratch_bytes) {
+    if ((rc = s.alloc((void**)&s.fold, kFoldBytes)) || (rc = clear_fold(s))) return rc;
+  }
   return fused_run(__func__, s, diag, bv, xv, eps, itmax, istop, check_every, iter, err, hist);
 }
 
