@@ -7,10 +7,10 @@
 // tiles; the tile table lists (slot, first row) system after system.  Every
 // streaming kernel walks the tile table grid-stride and skips the tiles of
 // systems that are not in the phase it serves; every reduction stores one
-// partial per tile, and a finalisation kernel with one block per slot adds
-// its system's partials in tile order.  A system's arithmetic therefore does
-// not depend on which other systems share the launch: its results are the
-// same alone and in any mix.
+// partial per tile, and the block of a system's last tile waits for the
+// others', adds them in tile order and updates the system's scalars.  A
+// system's arithmetic therefore does not depend on which other systems share
+// the launch: its results are the same alone and in any mix.
 //
 // A step = check_every FP32 iterations of every iterating system, then one
 // transition pass for the systems that asked for one:
@@ -84,14 +84,27 @@ struct BSys {
   float *v, *f, *s, *t;         // BiCGSTAB only
 };
 
+// Bits of a tile entry's slot word: the slot, and whether the tile is its
+// system's last.
+constexpr int kLastTile = 1 << 30;
+constexpr int kSlotMask = kLastTile - 1;
+// Slots up to which the tile kernels finalise by themselves (BTables::fold).
+// The blocks that wait for partials are at most one per system, and only after
+// their own tiles, so the other blocks always find a place: the chip holds at
+// least two of these blocks on each of its 256 CUs.
+constexpr int kFoldSlots = 256;
+// polls of a partial before the wait is given up (the sum is then NaN)
+constexpr int kFoldPolls = 1 << 22;
+
 struct BTables {
-  const int2* __restrict__ tiles;  // (slot, first row)
+  const int2* __restrict__ tiles;  // (slot | kLastTile, first row)
   const int* ntiles;               // device scalar
   const int2* __restrict__ range;  // per slot: first tile, tile count
   const BSys* __restrict__ sys;
   BState* st;
-  double* partials;                // two per tile
+  double* partials;                // two per tile; with fold kUnsetBits between uses
   int tcap;                        // tile table entries (>= kBGrid)
+  int fold;                        // finalise in the tile kernels (no kb_fin launches)
 };
 
 __device__ __forceinline__ bool b_iterating(const BState* s) {
@@ -142,8 +155,8 @@ __device__ __forceinline__ T b_row(const BSys& sy, const T* a, int r, const T* _
     int2 tl_ = (TB).tiles[blockIdx.x];                                   \
     int2 tn_;                                                            \
     for (int t_ = blockIdx.x; t_ < nt_; t_ += gridDim.x, tl_ = tn_) {    \
-      BState* st = (TB).st + tl_.x;                                      \
-      const BSys sy = (TB).sys[tl_.x];                                   \
+      BState* st = (TB).st + (tl_.x & kSlotMask);                        \
+      const BSys sy = (TB).sys[tl_.x & kSlotMask];                       \
       tn_ = (TB).tiles[min(t_ + (int)gridDim.x, (TB).tcap - 1)];         \
       if (!(COND)) continue;                                             \
       const int r0 = tl_.y;                                              \
@@ -151,380 +164,37 @@ __device__ __forceinline__ T b_row(const BSys& sy, const T* a, int r, const T* _
     }                                                                    \
   }
 
-__device__ __forceinline__ void tile_partials(double a, double b, double* partials, int t) {
+// The same for kernels whose body leaves the tile's two sums in a_ and b_:
+// they become the tile's partials, and after its tiles a block that had some
+// system's last one finalises it.
+#define PSB_BATCH_SUMS(TB, OP, COND, ...)                                \
+  {                                                                      \
+    int last_ = 0;                                                       \
+    PSB_BATCH_TILES(TB, COND, {                                          \
+      double a_ = 0.0, b_ = 0.0;                                         \
+      __VA_ARGS__                                                        \
+      tile_partials(a_, b_, TB, t_);                                     \
+      last_ |= tl_.x & kLastTile;                                        \
+    })                                                                   \
+    if ((TB).fold && last_) fold_tiles<OP>(TB);                          \
+  }
+
+__device__ __forceinline__ void tile_partials(double a, double b, const BTables& tb, int t) {
+  typedef unsigned long long U;
   __shared__ double lds[2][kBT / kWave];
   const double sa = block_sum<double, kBT>(a, lds[0]);
   const double sb = block_sum<double, kBT>(b, lds[1]);
-  if (threadIdx.x == 0) {
-    partials[2 * t] = sa;
-    partials[2 * t + 1] = sb;
+  if (threadIdx.x < 2) {
+    double* to = tb.partials + 2 * t + threadIdx.x;
+    const double v = threadIdx.x == 0 ? sa : sb;
+    if (tb.fold) {   // agent scope: the waiting block may sit on another XCD
+      U u = __builtin_bit_cast(U, v);
+      if (u == kUnsetBits) u = 0x7ff8000000000000ull;
+      __hip_atomic_store(reinterpret_cast<U*>(to), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      *to = v;
+    }
   }
-}
-
-// 4 consecutive entries p[0..3] (16-byte aligned); nv < 4: the first nv only
-__device__ __forceinline__ void ld4(const float* p, int nv, float (&a)[4]) {
-  if (nv == 4) {
-    const v16<float> t = ldv(p);
-    a[0] = t[0]; a[1] = t[1]; a[2] = t[2]; a[3] = t[3];
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; k++) a[k] = k < nv ? p[k] : 0.0f;
-  }
-}
-__device__ __forceinline__ void st4(float* p, int nv, const float (&a)[4]) {
-  if (nv == 4) {
-    v16<float> t;
-    t[0] = a[0]; t[1] = a[1]; t[2] = a[2]; t[3] = a[3];
-    stv(p, t);
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-      if (k < nv) p[k] = a[k];
-  }
-}
-__device__ __forceinline__ void ld4(const double* p, int nv, double (&a)[4]) {
-  if (nv == 4) {
-    const v16<double> t0 = ldv(p), t1 = ldv(p + 2);
-    a[0] = t0[0]; a[1] = t0[1]; a[2] = t1[0]; a[3] = t1[1];
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; k++) a[k] = k < nv ? p[k] : 0.0;
-  }
-}
-__device__ __forceinline__ void st4(double* p, int nv, const double (&a)[4]) {
-  if (nv == 4) {
-    v16<double> t0, t1;
-    t0[0] = a[0]; t0[1] = a[1]; t1[0] = a[2]; t1[1] = a[3];
-    stv(p, t0);
-    stv(p + 2, t1);
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-      if (k < nv) p[k] = a[k];
-  }
-}
-
-// first row and count (0..4) of this thread's 4 rows in an elementwise tile
-#define PSB_QUAD(I, NV)                                                  \
-  const int I = r0 + 4 * (int)threadIdx.x;                               \
-  const int NV = sy.n - I < 4 ? (sy.n - I > 0 ? sy.n - I : 0) : 4;
-
-// ------------------------------------------------------------------ CG iteration
-__global__ __launch_bounds__(kBT) void kb_cg_p(BTables tb) {
-  PSB_BATCH_TILES(tb, b_iterating(st), {
-    PSB_QUAD(i, nv)
-    if (nv > 0) {
-      float z[4], p[4];
-      ld4(sy.z + i, nv, z);
-      if (st->it == 0) {
-        st4(sy.p + i, nv, z);
-      } else {
-        ld4(sy.p + i, nv, p);
-        const float beta = (float)st->beta;
-_Pragma("unroll")
-        for (int k = 0; k < 4; k++) p[k] = z[k] + beta * p[k];
-        st4(sy.p + i, nv, p);
-      }
-    }
-  })
-}
-
-// Product kernels: 4 rows per thread (rows r0 + k*kBT + thread, k = 0..3,
-// each wavefront walking 4 whole hacks of the tile), so a block's descriptor
-// loads and reduction serve the whole tile with kBT threads and 4 times as
-// many blocks fit a CU as with one row per thread.
-__global__ __launch_bounds__(kBT) void kb_cg_q(BTables tb) {
-  PSB_BATCH_TILES(tb, b_iterating(st), {
-    float ax[4];
-_Pragma("unroll")
-    for (int k = 0; k < 4; k++) {
-      const int i = r0 + k * kBT + (int)threadIdx.x;
-      ax[k] = b_row<float>(sy, sy.a32, i < sy.n ? i : sy.n - 1, sy.p);
-    }
-    double pq = 0.0;
-_Pragma("unroll")
-    for (int k = 0; k < 4; k++) {
-      const int i = r0 + k * kBT + (int)threadIdx.x;
-      if (i < sy.n) {
-        sy.q[i] = ax[k];
-        pq += (double)sy.p[i] * (double)ax[k];
-      }
-    }
-    tile_partials(pq, 0.0, tb.partials, t_);
-  })
-}
-
-__global__ __launch_bounds__(kBT) void kb_cg_x(BTables tb) {
-  PSB_BATCH_TILES(tb, b_iterating(st), {
-    PSB_QUAD(i, nv)
-    double rr = 0.0, rz = 0.0;
-    if (nv > 0) {
-      const float alpha = (float)st->alpha;
-      float x[4], p[4], r[4], q[4], z[4];
-      ld4(sy.x32 + i, nv, x);
-      ld4(sy.p + i, nv, p);
-      ld4(sy.r + i, nv, r);
-      ld4(sy.q + i, nv, q);
-      if (sy.d32) ld4(sy.d32 + i, nv, z);
-_Pragma("unroll")
-      for (int k = 0; k < 4; k++) {
-        x[k] = x[k] + alpha * p[k];
-        r[k] = r[k] - alpha * q[k];
-        z[k] = sy.d32 ? z[k] * r[k] : r[k];
-        rr += (double)r[k] * (double)r[k];
-        rz += (double)r[k] * (double)z[k];
-      }
-      st4(sy.x32 + i, nv, x);
-      st4(sy.r + i, nv, r);
-      st4(sy.z + i, nv, z);
-    }
-    tile_partials(rr, rz, tb.partials, t_);
-  })
-}
-
-// ------------------------------------------------------------------ BiCGSTAB iteration
-__global__ __launch_bounds__(kBT) void kb_bi_a(BTables tb) {
-  PSB_BATCH_TILES(tb, b_iterating(st), {
-    PSB_QUAD(i, nv)
-    if (nv > 0) {
-      float r[4], p[4], v[4], f[4];
-      ld4(sy.r + i, nv, r);
-      if (st->it != 0) {
-        ld4(sy.p + i, nv, p);
-        ld4(sy.v + i, nv, v);
-        const float beta = (float)st->beta, momega = (float)(-st->omega);
-_Pragma("unroll")
-        for (int k = 0; k < 4; k++) p[k] = r[k] + beta * (momega * v[k] + p[k]);
-      } else {
-_Pragma("unroll")
-        for (int k = 0; k < 4; k++) p[k] = r[k];
-      }
-      st4(sy.p + i, nv, p);
-      if (sy.d32) {
-        ld4(sy.d32 + i, nv, f);
-_Pragma("unroll")
-        for (int k = 0; k < 4; k++) f[k] = f[k] * p[k];
-        st4(sy.f + i, nv, f);
-      } else {
-        st4(sy.f + i, nv, p);
-      }
-    }
-  })
-}
-
-__global__ __launch_bounds__(kBT) void kb_bi_v(BTables tb) {
-  PSB_BATCH_TILES(tb, b_iterating(st), {
-    float ax[4];
-_Pragma("unroll")
-    for (int k = 0; k < 4; k++) {
-      const int i = r0 + k * kBT + (int)threadIdx.x;
-      ax[k] = b_row<float>(sy, sy.a32, i < sy.n ? i : sy.n - 1, sy.f);
-    }
-    double qv = 0.0;
-_Pragma("unroll")
-    for (int k = 0; k < 4; k++) {
-      const int i = r0 + k * kBT + (int)threadIdx.x;
-      if (i < sy.n) {
-        sy.v[i] = ax[k];
-        qv += (double)sy.q[i] * (double)ax[k];
-      }
-    }
-    tile_partials(qv, 0.0, tb.partials, t_);
-  })
-}
-
-__global__ __launch_bounds__(kBT) void kb_bi_s(BTables tb) {
-  PSB_BATCH_TILES(tb, b_iterating(st), {
-    PSB_QUAD(i, nv)
-    if (nv > 0) {
-      float v[4], r[4], z[4];
-      ld4(sy.v + i, nv, v);
-      ld4(sy.r + i, nv, r);
-      const float malpha = (float)(-st->alpha);
-_Pragma("unroll")
-      for (int k = 0; k < 4; k++) r[k] = malpha * v[k] + r[k];   // s
-      st4(sy.s + i, nv, r);
-      if (sy.d32) {
-        ld4(sy.d32 + i, nv, z);
-_Pragma("unroll")
-        for (int k = 0; k < 4; k++) z[k] = z[k] * r[k];
-        st4(sy.z + i, nv, z);
-      } else {
-        st4(sy.z + i, nv, r);
-      }
-    }
-  })
-}
-
-__global__ __launch_bounds__(kBT) void kb_bi_t(BTables tb) {
-  PSB_BATCH_TILES(tb, b_iterating(st), {
-    float ax[4];
-_Pragma("unroll")
-    for (int k = 0; k < 4; k++) {
-      const int i = r0 + k * kBT + (int)threadIdx.x;
-      ax[k] = b_row<float>(sy, sy.a32, i < sy.n ? i : sy.n - 1, sy.z);
-    }
-    double tt = 0.0, ts = 0.0;
-_Pragma("unroll")
-    for (int k = 0; k < 4; k++) {
-      const int i = r0 + k * kBT + (int)threadIdx.x;
-      if (i < sy.n) {
-        sy.t[i] = ax[k];
-        tt += (double)ax[k] * (double)ax[k];
-        ts += (double)ax[k] * (double)sy.s[i];
-      }
-    }
-    tile_partials(tt, ts, tb.partials, t_);
-  })
-}
-
-__global__ __launch_bounds__(kBT) void kb_bi_x(BTables tb) {
-  PSB_BATCH_TILES(tb, b_iterating(st), {
-    PSB_QUAD(i, nv)
-    double rr = 0.0, qr = 0.0;
-    if (nv > 0) {
-      const float alpha = (float)st->alpha, omega = (float)st->omega;
-      float x[4], z[4], f[4], t[4], s4[4], q[4];
-      ld4(sy.x32 + i, nv, x);
-      ld4(sy.z + i, nv, z);
-      ld4(sy.f + i, nv, f);
-      ld4(sy.t + i, nv, t);
-      ld4(sy.s + i, nv, s4);
-      ld4(sy.q + i, nv, q);
-_Pragma("unroll")
-      for (int k = 0; k < 4; k++) {
-        x[k] = omega * z[k] + (alpha * f[k] + x[k]);
-        s4[k] = -omega * t[k] + s4[k];   // r
-        rr += (double)s4[k] * (double)s4[k];
-        qr += (double)q[k] * (double)s4[k];
-      }
-      st4(sy.x32 + i, nv, x);
-      st4(sy.r + i, nv, s4);
-    }
-    tile_partials(rr, qr, tb.partials, t_);
-  })
-}
-
-// ------------------------------------------------------------------ transitions
-// x64 += scale * x32 (residual replacement: scale 1; restarted refinement:
-// ||r64|| of the finished cycle), x32 = 0.  A newly admitted system only
-// clears x32.
-__global__ __launch_bounds__(kBT) void kb_accum(BTables tb, int unit_scale) {
-  PSB_BATCH_TILES(tb, b_transiting(st), {
-    PSB_QUAD(i, nv)
-    if (nv > 0) {
-      float x32[4];
-      // a recurrence that ended on a non-finite residual norm leaves its
-      // iterate out (st->rr: the norm after its last iteration)
-      if (st->phase != BP_INIT && isfinite(st->rr)) {
-        const double scale = unit_scale ? 1.0 : st->ref;
-        double x[4];
-        ld4(sy.x + i, nv, x);
-        ld4(sy.x32 + i, nv, x32);
-_Pragma("unroll")
-        for (int k = 0; k < 4; k++) x[k] = x[k] + scale * (double)x32[k];
-        st4(sy.x + i, nv, x);
-      }
-_Pragma("unroll")
-      for (int k = 0; k < 4; k++) x32[k] = 0.0f;
-      st4(sy.x32 + i, nv, x32);
-    }
-  })
-}
-
-// r64 = b - A64 x64 with partials r64.r64 and b.b (FP64)
-__global__ __launch_bounds__(kBT) void kb_res(BTables tb) {
-  PSB_BATCH_TILES(tb, b_transiting(st), {
-    double ax[4];
-_Pragma("unroll")
-    for (int k = 0; k < 4; k++) {
-      const int i = r0 + k * kBT + (int)threadIdx.x;
-      ax[k] = b_row<double>(sy, sy.a64, i < sy.n ? i : sy.n - 1, sy.x);
-    }
-    double rr = 0.0, bb = 0.0;
-_Pragma("unroll")
-    for (int k = 0; k < 4; k++) {
-      const int i = r0 + k * kBT + (int)threadIdx.x;
-      if (i < sy.n) {
-        const double bi = sy.b[i];
-        const double ri = bi - ax[k];
-        sy.r64[i] = ri;
-        rr += ri * ri;
-        bb += bi * bi;
-      }
-    }
-    tile_partials(rr, bb, tb.partials, t_);
-  })
-}
-
-// CG: r = (float) r64, z = d.*r, partial r.z
-__global__ __launch_bounds__(kBT) void kb_cg_reset(BTables tb) {
-  PSB_BATCH_TILES(tb, b_transiting(st), {
-    PSB_QUAD(i, nv)
-    double rz = 0.0;
-    if (nv > 0) {
-      double r64[4];
-      float r[4], z[4];
-      ld4(sy.r64 + i, nv, r64);
-      if (sy.d32) ld4(sy.d32 + i, nv, z);
-_Pragma("unroll")
-      for (int k = 0; k < 4; k++) {
-        r[k] = (float)r64[k];
-        z[k] = sy.d32 ? z[k] * r[k] : r[k];
-        rz += (double)r[k] * (double)z[k];
-      }
-      st4(sy.r + i, nv, r);
-      st4(sy.z + i, nv, z);
-    }
-    tile_partials(rz, 0.0, tb.partials, t_);
-  })
-}
-
-// BiCGSTAB: r = q = (float)(r64 / ||r64||), partial r.r
-__global__ __launch_bounds__(kBT) void kb_bi_restart(BTables tb) {
-  PSB_BATCH_TILES(tb, b_transiting(st), {
-    PSB_QUAD(i, nv)
-    double rr = 0.0;
-    if (nv > 0) {
-      const double inv = 1.0 / st->rnorm;
-      double r64[4];
-      float r[4];
-      ld4(sy.r64 + i, nv, r64);
-_Pragma("unroll")
-      for (int k = 0; k < 4; k++) {
-        r[k] = (float)(r64[k] * inv);
-        rr += (double)r[k] * (double)r[k];
-      }
-      st4(sy.r + i, nv, r);
-      st4(sy.q + i, nv, r);
-    }
-    tile_partials(rr, 0.0, tb.partials, t_);
-  })
-}
-
-// BiCGSTAB with residual replacement: r = (float) r64; a newly admitted or
-// broken-down system also takes q = r.  Partial q.r.
-__global__ __launch_bounds__(kBT) void kb_biru_reset(BTables tb) {
-  PSB_BATCH_TILES(tb, b_transiting(st), {
-    PSB_QUAD(i, nv)
-    double qr = 0.0;
-    if (nv > 0) {
-      const bool fresh = st->phase != BP_TRANS;
-      double r64[4];
-      float r[4], q[4];
-      ld4(sy.r64 + i, nv, r64);
-      if (!fresh) ld4(sy.q + i, nv, q);
-_Pragma("unroll")
-      for (int k = 0; k < 4; k++) {
-        r[k] = (float)r64[k];
-        if (fresh) q[k] = r[k];
-        qr += (double)q[k] * (double)r[k];
-      }
-      st4(sy.r + i, nv, r);
-      if (fresh) st4(sy.q + i, nv, q);
-    }
-    tile_partials(qr, 0.0, tb.partials, t_);
-  })
 }
 
 // ------------------------------------------------------------------ per-system finalisation
@@ -533,22 +203,13 @@ enum BFin {
   BF_BIRU_RESET
 };
 
+__host__ __device__ constexpr bool fin_transiting(int op) {
+  return op == BF_RES || op == BF_CG_RESET || op == BF_BI_RESTART || op == BF_BIRU_RESET;
+}
+
+// A system's scalars after a kernel with the sums a and b (one thread).
 template <int OP>
-__global__ __launch_bounds__(kBT) void kb_fin(BTables tb) {
-  BState* st = tb.st + blockIdx.x;
-  const bool trans =
-      OP == BF_RES || OP == BF_CG_RESET || OP == BF_BI_RESTART || OP == BF_BIRU_RESET;
-  if (trans ? !b_transiting(st) : !b_iterating(st)) return;
-  const int2 rg = tb.range[blockIdx.x];
-  double a = 0.0, b = 0.0;
-  for (int k = threadIdx.x; k < rg.y; k += kBT) {
-    a += tb.partials[2 * (rg.x + k)];
-    b += tb.partials[2 * (rg.x + k) + 1];
-  }
-  __shared__ double lds[2][kBT / kWave];
-  a = block_sum<double, kBT>(a, lds[0]);
-  b = block_sum<double, kBT>(b, lds[1]);
-  if (threadIdx.x != 0) return;
+__device__ __forceinline__ void fin_apply(BState* st, double a, double b) {
   // A zero or non-finite denominator or scalar is a breakdown: the FP32
   // recurrence stops before its vectors take the value, the transition
   // keeps the last finite iterate and restarts from the FP64 residual.  (An
@@ -684,6 +345,436 @@ __global__ __launch_bounds__(kBT) void kb_fin(BTables tb) {
   }
 }
 
+// One block per slot: the finalisation of engines with more than kFoldSlots
+// slots.
+template <int OP>
+__global__ __launch_bounds__(kBT) void kb_fin(BTables tb) {
+  BState* st = tb.st + blockIdx.x;
+  if (fin_transiting(OP) ? !b_transiting(st) : !b_iterating(st)) return;
+  const int2 rg = tb.range[blockIdx.x];
+  double a = 0.0, b = 0.0;
+  for (int k = threadIdx.x; k < rg.y; k += kBT) {
+    a += tb.partials[2 * (rg.x + k)];
+    b += tb.partials[2 * (rg.x + k) + 1];
+  }
+  __shared__ double lds[2][kBT / kWave];
+  a = block_sum<double, kBT>(a, lds[0]);
+  b = block_sum<double, kBT>(b, lds[1]);
+  if (threadIdx.x == 0) fin_apply<OP>(st, a, b);
+}
+
+// The finalisation of the systems whose last tile is one of this block's: waits
+// for the partials of the system's other tiles (each is there once it holds
+// something else than kUnsetBits), sets them back, adds them as kb_fin does.
+// The wait ends: every block stores its tiles' partials before it waits, and
+// the waiting ones leave room for the others (kFoldSlots).
+template <int OP>
+__device__ __forceinline__ void fold_tiles(const BTables& tb) {
+  typedef unsigned long long U;
+  __shared__ double lds[2][kBT / kWave];
+  const int nt = *tb.ntiles;
+  for (int t = blockIdx.x; t < nt; t += gridDim.x) {
+    const int2 tl = tb.tiles[t];
+    if (!(tl.x & kLastTile)) continue;
+    BState* st = tb.st + (tl.x & kSlotMask);
+    if (fin_transiting(OP) ? !b_transiting(st) : !b_iterating(st)) continue;
+    const int2 rg = tb.range[tl.x & kSlotMask];
+    double a = 0.0, b = 0.0;
+    for (int k = threadIdx.x; k < rg.y; k += kBT) {
+      U* p = reinterpret_cast<U*>(tb.partials) + 2 * (size_t)(rg.x + k);
+      U ua, ub;
+      int polls = 0;
+      do {
+        ua = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        ub = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      } while ((ua == kUnsetBits || ub == kUnsetBits) && ++polls < kFoldPolls);
+      p[0] = kUnsetBits;
+      p[1] = kUnsetBits;
+      a += __builtin_bit_cast(double, ua);
+      b += __builtin_bit_cast(double, ub);
+    }
+    a = block_sum<double, kBT>(a, lds[0]);
+    b = block_sum<double, kBT>(b, lds[1]);
+    if (threadIdx.x == 0) fin_apply<OP>(st, a, b);
+  }
+}
+
+// 4 consecutive entries p[0..3] (16-byte aligned); nv < 4: the first nv only
+__device__ __forceinline__ void ld4(const float* p, int nv, float (&a)[4]) {
+  if (nv == 4) {
+    const v16<float> t = ldv(p);
+    a[0] = t[0]; a[1] = t[1]; a[2] = t[2]; a[3] = t[3];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; k++) a[k] = k < nv ? p[k] : 0.0f;
+  }
+}
+__device__ __forceinline__ void st4(float* p, int nv, const float (&a)[4]) {
+  if (nv == 4) {
+    v16<float> t;
+    t[0] = a[0]; t[1] = a[1]; t[2] = a[2]; t[3] = a[3];
+    stv(p, t);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (k < nv) p[k] = a[k];
+  }
+}
+__device__ __forceinline__ void ld4(const double* p, int nv, double (&a)[4]) {
+  if (nv == 4) {
+    const v16<double> t0 = ldv(p), t1 = ldv(p + 2);
+    a[0] = t0[0]; a[1] = t0[1]; a[2] = t1[0]; a[3] = t1[1];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; k++) a[k] = k < nv ? p[k] : 0.0;
+  }
+}
+__device__ __forceinline__ void st4(double* p, int nv, const double (&a)[4]) {
+  if (nv == 4) {
+    v16<double> t0, t1;
+    t0[0] = a[0]; t0[1] = a[1]; t1[0] = a[2]; t1[1] = a[3];
+    stv(p, t0);
+    stv(p + 2, t1);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (k < nv) p[k] = a[k];
+  }
+}
+
+// first row and count (0..4) of this thread's 4 rows in an elementwise tile
+#define PSB_QUAD(I, NV)                                                  \
+  const int I = r0 + 4 * (int)threadIdx.x;                               \
+  const int NV = sy.n - I < 4 ? (sy.n - I > 0 ? sy.n - I : 0) : 4;
+
+// ------------------------------------------------------------------ CG iteration
+__global__ __launch_bounds__(kBT) void kb_cg_p(BTables tb) {
+  PSB_BATCH_TILES(tb, b_iterating(st), {
+    PSB_QUAD(i, nv)
+    if (nv > 0) {
+      float z[4], p[4];
+      ld4(sy.z + i, nv, z);
+      if (st->it == 0) {
+        st4(sy.p + i, nv, z);
+      } else {
+        ld4(sy.p + i, nv, p);
+        const float beta = (float)st->beta;
+_Pragma("unroll")
+        for (int k = 0; k < 4; k++) p[k] = z[k] + beta * p[k];
+        st4(sy.p + i, nv, p);
+      }
+    }
+  })
+}
+
+// Product kernels: 4 rows per thread (rows r0 + k*kBT + thread, k = 0..3,
+// each wavefront walking 4 whole hacks of the tile), so a block's descriptor
+// loads and reduction serve the whole tile with kBT threads and 4 times as
+// many blocks fit a CU as with one row per thread.
+__global__ __launch_bounds__(kBT) void kb_cg_q(BTables tb) {
+  PSB_BATCH_SUMS(tb, BF_CG_Q, b_iterating(st), {
+    float ax[4];
+_Pragma("unroll")
+    for (int k = 0; k < 4; k++) {
+      const int i = r0 + k * kBT + (int)threadIdx.x;
+      ax[k] = b_row<float>(sy, sy.a32, i < sy.n ? i : sy.n - 1, sy.p);
+    }
+    double pq = 0.0;
+_Pragma("unroll")
+    for (int k = 0; k < 4; k++) {
+      const int i = r0 + k * kBT + (int)threadIdx.x;
+      if (i < sy.n) {
+        sy.q[i] = ax[k];
+        pq += (double)sy.p[i] * (double)ax[k];
+      }
+    }
+    a_ = pq;
+  })
+}
+
+__global__ __launch_bounds__(kBT) void kb_cg_x(BTables tb) {
+  PSB_BATCH_SUMS(tb, BF_CG_X, b_iterating(st), {
+    PSB_QUAD(i, nv)
+    double rr = 0.0, rz = 0.0;
+    if (nv > 0) {
+      const float alpha = (float)st->alpha;
+      float x[4], p[4], r[4], q[4], z[4];
+      ld4(sy.x32 + i, nv, x);
+      ld4(sy.p + i, nv, p);
+      ld4(sy.r + i, nv, r);
+      ld4(sy.q + i, nv, q);
+      if (sy.d32) ld4(sy.d32 + i, nv, z);
+_Pragma("unroll")
+      for (int k = 0; k < 4; k++) {
+        x[k] = x[k] + alpha * p[k];
+        r[k] = r[k] - alpha * q[k];
+        z[k] = sy.d32 ? z[k] * r[k] : r[k];
+        rr += (double)r[k] * (double)r[k];
+        rz += (double)r[k] * (double)z[k];
+      }
+      st4(sy.x32 + i, nv, x);
+      st4(sy.r + i, nv, r);
+      st4(sy.z + i, nv, z);
+    }
+    a_ = rr;
+    b_ = rz;
+  })
+}
+
+// ------------------------------------------------------------------ BiCGSTAB iteration
+__global__ __launch_bounds__(kBT) void kb_bi_a(BTables tb) {
+  PSB_BATCH_TILES(tb, b_iterating(st), {
+    PSB_QUAD(i, nv)
+    if (nv > 0) {
+      float r[4], p[4], v[4], f[4];
+      ld4(sy.r + i, nv, r);
+      if (st->it != 0) {
+        ld4(sy.p + i, nv, p);
+        ld4(sy.v + i, nv, v);
+        const float beta = (float)st->beta, momega = (float)(-st->omega);
+_Pragma("unroll")
+        for (int k = 0; k < 4; k++) p[k] = r[k] + beta * (momega * v[k] + p[k]);
+      } else {
+_Pragma("unroll")
+        for (int k = 0; k < 4; k++) p[k] = r[k];
+      }
+      st4(sy.p + i, nv, p);
+      if (sy.d32) {
+        ld4(sy.d32 + i, nv, f);
+_Pragma("unroll")
+        for (int k = 0; k < 4; k++) f[k] = f[k] * p[k];
+        st4(sy.f + i, nv, f);
+      } else {
+        st4(sy.f + i, nv, p);
+      }
+    }
+  })
+}
+
+__global__ __launch_bounds__(kBT) void kb_bi_v(BTables tb) {
+  PSB_BATCH_SUMS(tb, BF_BI_V, b_iterating(st), {
+    float ax[4];
+_Pragma("unroll")
+    for (int k = 0; k < 4; k++) {
+      const int i = r0 + k * kBT + (int)threadIdx.x;
+      ax[k] = b_row<float>(sy, sy.a32, i < sy.n ? i : sy.n - 1, sy.f);
+    }
+    double qv = 0.0;
+_Pragma("unroll")
+    for (int k = 0; k < 4; k++) {
+      const int i = r0 + k * kBT + (int)threadIdx.x;
+      if (i < sy.n) {
+        sy.v[i] = ax[k];
+        qv += (double)sy.q[i] * (double)ax[k];
+      }
+    }
+    a_ = qv;
+  })
+}
+
+__global__ __launch_bounds__(kBT) void kb_bi_s(BTables tb) {
+  PSB_BATCH_TILES(tb, b_iterating(st), {
+    PSB_QUAD(i, nv)
+    if (nv > 0) {
+      float v[4], r[4], z[4];
+      ld4(sy.v + i, nv, v);
+      ld4(sy.r + i, nv, r);
+      const float malpha = (float)(-st->alpha);
+_Pragma("unroll")
+      for (int k = 0; k < 4; k++) r[k] = malpha * v[k] + r[k];   // s
+      st4(sy.s + i, nv, r);
+      if (sy.d32) {
+        ld4(sy.d32 + i, nv, z);
+_Pragma("unroll")
+        for (int k = 0; k < 4; k++) z[k] = z[k] * r[k];
+        st4(sy.z + i, nv, z);
+      } else {
+        st4(sy.z + i, nv, r);
+      }
+    }
+  })
+}
+
+__global__ __launch_bounds__(kBT) void kb_bi_t(BTables tb) {
+  PSB_BATCH_SUMS(tb, BF_BI_T, b_iterating(st), {
+    float ax[4];
+_Pragma("unroll")
+    for (int k = 0; k < 4; k++) {
+      const int i = r0 + k * kBT + (int)threadIdx.x;
+      ax[k] = b_row<float>(sy, sy.a32, i < sy.n ? i : sy.n - 1, sy.z);
+    }
+    double tt = 0.0, ts = 0.0;
+_Pragma("unroll")
+    for (int k = 0; k < 4; k++) {
+      const int i = r0 + k * kBT + (int)threadIdx.x;
+      if (i < sy.n) {
+        sy.t[i] = ax[k];
+        tt += (double)ax[k] * (double)ax[k];
+        ts += (double)ax[k] * (double)sy.s[i];
+      }
+    }
+    a_ = tt;
+    b_ = ts;
+  })
+}
+
+template <int OP>
+__global__ __launch_bounds__(kBT) void kb_bi_x(BTables tb) {
+  PSB_BATCH_SUMS(tb, OP, b_iterating(st), {
+    PSB_QUAD(i, nv)
+    double rr = 0.0, qr = 0.0;
+    if (nv > 0) {
+      const float alpha = (float)st->alpha, omega = (float)st->omega;
+      float x[4], z[4], f[4], t[4], s4[4], q[4];
+      ld4(sy.x32 + i, nv, x);
+      ld4(sy.z + i, nv, z);
+      ld4(sy.f + i, nv, f);
+      ld4(sy.t + i, nv, t);
+      ld4(sy.s + i, nv, s4);
+      ld4(sy.q + i, nv, q);
+_Pragma("unroll")
+      for (int k = 0; k < 4; k++) {
+        x[k] = omega * z[k] + (alpha * f[k] + x[k]);
+        s4[k] = -omega * t[k] + s4[k];   // r
+        rr += (double)s4[k] * (double)s4[k];
+        qr += (double)q[k] * (double)s4[k];
+      }
+      st4(sy.x32 + i, nv, x);
+      st4(sy.r + i, nv, s4);
+    }
+    a_ = rr;
+    b_ = qr;
+  })
+}
+
+// ------------------------------------------------------------------ transitions
+// x64 += scale * x32 (residual replacement: scale 1; restarted refinement:
+// ||r64|| of the finished cycle), x32 = 0.  A newly admitted system only
+// clears x32.
+__global__ __launch_bounds__(kBT) void kb_accum(BTables tb, int unit_scale) {
+  PSB_BATCH_TILES(tb, b_transiting(st), {
+    PSB_QUAD(i, nv)
+    if (nv > 0) {
+      float x32[4];
+      // a recurrence that ended on a non-finite residual norm leaves its
+      // iterate out (st->rr: the norm after its last iteration)
+      if (st->phase != BP_INIT && isfinite(st->rr)) {
+        const double scale = unit_scale ? 1.0 : st->ref;
+        double x[4];
+        ld4(sy.x + i, nv, x);
+        ld4(sy.x32 + i, nv, x32);
+_Pragma("unroll")
+        for (int k = 0; k < 4; k++) x[k] = x[k] + scale * (double)x32[k];
+        st4(sy.x + i, nv, x);
+      }
+_Pragma("unroll")
+      for (int k = 0; k < 4; k++) x32[k] = 0.0f;
+      st4(sy.x32 + i, nv, x32);
+    }
+  })
+}
+
+// r64 = b - A64 x64 with partials r64.r64 and b.b (FP64)
+__global__ __launch_bounds__(kBT) void kb_res(BTables tb) {
+  PSB_BATCH_SUMS(tb, BF_RES, b_transiting(st), {
+    double ax[4];
+_Pragma("unroll")
+    for (int k = 0; k < 4; k++) {
+      const int i = r0 + k * kBT + (int)threadIdx.x;
+      ax[k] = b_row<double>(sy, sy.a64, i < sy.n ? i : sy.n - 1, sy.x);
+    }
+    double rr = 0.0, bb = 0.0;
+_Pragma("unroll")
+    for (int k = 0; k < 4; k++) {
+      const int i = r0 + k * kBT + (int)threadIdx.x;
+      if (i < sy.n) {
+        const double bi = sy.b[i];
+        const double ri = bi - ax[k];
+        sy.r64[i] = ri;
+        rr += ri * ri;
+        bb += bi * bi;
+      }
+    }
+    a_ = rr;
+    b_ = bb;
+  })
+}
+
+// CG: r = (float) r64, z = d.*r, partial r.z
+__global__ __launch_bounds__(kBT) void kb_cg_reset(BTables tb) {
+  PSB_BATCH_SUMS(tb, BF_CG_RESET, b_transiting(st), {
+    PSB_QUAD(i, nv)
+    double rz = 0.0;
+    if (nv > 0) {
+      double r64[4];
+      float r[4], z[4];
+      ld4(sy.r64 + i, nv, r64);
+      if (sy.d32) ld4(sy.d32 + i, nv, z);
+_Pragma("unroll")
+      for (int k = 0; k < 4; k++) {
+        r[k] = (float)r64[k];
+        z[k] = sy.d32 ? z[k] * r[k] : r[k];
+        rz += (double)r[k] * (double)z[k];
+      }
+      st4(sy.r + i, nv, r);
+      st4(sy.z + i, nv, z);
+    }
+    a_ = rz;
+  })
+}
+
+// BiCGSTAB: r = q = (float)(r64 / ||r64||), partial r.r
+__global__ __launch_bounds__(kBT) void kb_bi_restart(BTables tb) {
+  PSB_BATCH_SUMS(tb, BF_BI_RESTART, b_transiting(st), {
+    PSB_QUAD(i, nv)
+    double rr = 0.0;
+    if (nv > 0) {
+      const double inv = 1.0 / st->rnorm;
+      double r64[4];
+      float r[4];
+      ld4(sy.r64 + i, nv, r64);
+_Pragma("unroll")
+      for (int k = 0; k < 4; k++) {
+        r[k] = (float)(r64[k] * inv);
+        rr += (double)r[k] * (double)r[k];
+      }
+      st4(sy.r + i, nv, r);
+      st4(sy.q + i, nv, r);
+    }
+    a_ = rr;
+  })
+}
+
+// BiCGSTAB with residual replacement: r = (float) r64; a newly admitted or
+// broken-down system also takes q = r.  Partial q.r.
+__global__ __launch_bounds__(kBT) void kb_biru_reset(BTables tb) {
+  PSB_BATCH_SUMS(tb, BF_BIRU_RESET, b_transiting(st), {
+    PSB_QUAD(i, nv)
+    double qr = 0.0;
+    if (nv > 0) {
+      const bool fresh = st->phase != BP_TRANS;
+      double r64[4];
+      float r[4], q[4];
+      ld4(sy.r64 + i, nv, r64);
+      if (!fresh) ld4(sy.q + i, nv, q);
+_Pragma("unroll")
+      for (int k = 0; k < 4; k++) {
+        r[k] = (float)r64[k];
+        if (fresh) q[k] = r[k];
+        qr += (double)q[k] * (double)r[k];
+      }
+      st4(sy.r + i, nv, r);
+      if (fresh) st4(sy.q + i, nv, q);
+    }
+    a_ = qr;
+  })
+}
+
+__global__ __launch_bounds__(kBT) void kb_unset(int64_t n, unsigned long long* __restrict__ a) {
+  for (int64_t i = (int64_t)blockIdx.x * kBT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBT)
+    a[i] = kUnsetBits;
+}
+
 __global__ __launch_bounds__(kBT) void kb_fill(double* __restrict__ x, int n, double v) {
   for (int i = blockIdx.x * kBT + threadIdx.x; i < n; i += gridDim.x * kBT) x[i] = v;
 }
@@ -716,6 +807,7 @@ struct Batch {
   int method = 0, nslots = 0, check_every = 8;
   double delta = 1e-2, inner_eps = 1e-4;
   bool use_graph = true;
+  bool fold = false;                          // the tile kernels finalise (kFoldSlots)
   hipStream_t stream = nullptr;
   char* arena = nullptr;
   size_t arena_bytes = 0;
@@ -751,6 +843,7 @@ static BTables tables(const Batch& B) {
   t.st = B.st;
   t.partials = B.partials;
   t.tcap = B.tmax;
+  t.fold = B.fold ? 1 : 0;
   return t;
 }
 
@@ -797,37 +890,44 @@ static void enqueue_step(Batch& B) {
   const BTables tb = tables(B);
   dim3 g(kBGrid), blk(kBT), gs(B.nslots);
   hipStream_t s = B.stream;
+  auto fin = [&](void (*kernel)(BTables)) {
+    if (!B.fold) hipLaunchKernelGGL(kernel, gs, blk, 0, s, tb);
+  };
   for (int k = 0; k < B.check_every; k++) {
     if (B.method == 0) {
       hipLaunchKernelGGL(kb_cg_p, g, blk, 0, s, tb);
       hipLaunchKernelGGL(kb_cg_q, g, blk, 0, s, tb);
-      hipLaunchKernelGGL(kb_fin<BF_CG_Q>, gs, blk, 0, s, tb);
+      fin(kb_fin<BF_CG_Q>);
       hipLaunchKernelGGL(kb_cg_x, g, blk, 0, s, tb);
-      hipLaunchKernelGGL(kb_fin<BF_CG_X>, gs, blk, 0, s, tb);
+      fin(kb_fin<BF_CG_X>);
     } else {
       hipLaunchKernelGGL(kb_bi_a, g, blk, 0, s, tb);
       hipLaunchKernelGGL(kb_bi_v, g, blk, 0, s, tb);
-      hipLaunchKernelGGL(kb_fin<BF_BI_V>, gs, blk, 0, s, tb);
+      fin(kb_fin<BF_BI_V>);
       hipLaunchKernelGGL(kb_bi_s, g, blk, 0, s, tb);
       hipLaunchKernelGGL(kb_bi_t, g, blk, 0, s, tb);
-      hipLaunchKernelGGL(kb_fin<BF_BI_T>, gs, blk, 0, s, tb);
-      hipLaunchKernelGGL(kb_bi_x, g, blk, 0, s, tb);
-      if (B.method == 1) hipLaunchKernelGGL(kb_fin<BF_BI_X>, gs, blk, 0, s, tb);
-      else hipLaunchKernelGGL(kb_fin<BF_BIRU_X>, gs, blk, 0, s, tb);
+      fin(kb_fin<BF_BI_T>);
+      if (B.method == 1) {
+        hipLaunchKernelGGL(kb_bi_x<BF_BI_X>, g, blk, 0, s, tb);
+        fin(kb_fin<BF_BI_X>);
+      } else {
+        hipLaunchKernelGGL(kb_bi_x<BF_BIRU_X>, g, blk, 0, s, tb);
+        fin(kb_fin<BF_BIRU_X>);
+      }
     }
   }
   hipLaunchKernelGGL(kb_accum, g, blk, 0, s, tb, B.method == 1 ? 0 : 1);
   hipLaunchKernelGGL(kb_res, g, blk, 0, s, tb);
-  hipLaunchKernelGGL(kb_fin<BF_RES>, gs, blk, 0, s, tb);
+  fin(kb_fin<BF_RES>);
   if (B.method == 0) {
     hipLaunchKernelGGL(kb_cg_reset, g, blk, 0, s, tb);
-    hipLaunchKernelGGL(kb_fin<BF_CG_RESET>, gs, blk, 0, s, tb);
+    fin(kb_fin<BF_CG_RESET>);
   } else if (B.method == 2) {
     hipLaunchKernelGGL(kb_biru_reset, g, blk, 0, s, tb);
-    hipLaunchKernelGGL(kb_fin<BF_BIRU_RESET>, gs, blk, 0, s, tb);
+    fin(kb_fin<BF_BIRU_RESET>);
   } else {
     hipLaunchKernelGGL(kb_bi_restart, g, blk, 0, s, tb);
-    hipLaunchKernelGGL(kb_fin<BF_BI_RESTART>, gs, blk, 0, s, tb);
+    fin(kb_fin<BF_BI_RESTART>);
   }
 }
 
@@ -843,7 +943,7 @@ static int upload(Batch& B) {
       const int nk = sl.live ? (B.sys_h[k].n + kTileRows - 1) / kTileRows : 0;
       if (nt + nk > B.tmax) return set_error(PSB_HIP_RUNTIME, "batch", "tile table overflow");
       S.range[k] = make_int2(nt, nk);
-      for (int j = 0; j < nk; j++) S.tiles[nt + j] = make_int2(k, j * kTileRows);
+      for (int j = 0; j < nk; j++) S.tiles[nt + j] = make_int2(k | (j == nk - 1 ? kLastTile : 0), j * kTileRows);
       nt += nk;
     }
     *S.ntiles = nt;
@@ -958,6 +1058,15 @@ int psb_hip_batch_create(void** batch, int method, int max_systems, int64_t aren
     destroy(B);
     return set_error(e == hipErrorOutOfMemory ? PSB_HIP_OUTOFMEM : PSB_HIP_RUNTIME, __func__,
                      hipGetErrorString(e));
+  }
+  B->fold = max_systems <= kFoldSlots;
+  if (B->fold) {
+    hipLaunchKernelGGL(kb_unset, dim3(stream_grid(2 * (int64_t)B->tmax)), dim3(kBT), 0, B->stream,
+                       2 * (int64_t)B->tmax, (unsigned long long*)B->partials);
+    if (hipGetLastError() != hipSuccess) {
+      destroy(B);
+      return set_error(PSB_HIP_RUNTIME, __func__, "kb_unset");
+    }
   }
   // every slot starts finished (no tiles, skipped by every kernel)
   std::vector<BState> idle(max_systems);
