@@ -59,6 +59,7 @@ struct KState {
   int done;       // stop test satisfied (or itmax reached)
   int breakdown;  // 1: restart requested; 2: residual replacement requested
   int istop;
+  int left;       // a resident launch did not come to run (res_enter)
 };
 
 // --------------------------------------------------------------- views
@@ -693,6 +694,542 @@ __global__ __launch_bounds__(kBlock) void k_bi_x(int n, T* __restrict__ x, T* __
   finish<FIN_BI_X, 2>(v, fin, st);
 }
 
+// --------------------------------------------------------------- resident solvers
+// CG and BiCGSTAB of systems small enough that the chip's threads hold their
+// vectors and matrix: one launch runs kResIters iterations on one to four rows
+// a thread.  Between blocks go only the vector that the product gathers (p; f
+// and z for BiCGSTAB) and the partial sums, as agent-scope stores and loads of
+// entries that hold the unset pattern until they are there.  Nothing else may
+// read those entries: a plain load leaves its line in the XCD's L2, where
+// later agent-scope loads would find it unchanged.
+//
+// The launches per step are bound by the launches where the system is small (a
+// dependent one costs 5 us; three an iteration of CG) and by the matrix and the
+// vectors going through memory where it is large.  Here a CG iteration is two
+// sums over the blocks and one exchange, 2 us each; above 262144 rows the
+// chain of a thread's rows, each waiting for its exchanged entries, adds to it.
+// An iteration of CG, 7-point, FP64 (launches per step -> resident): 27 000
+// rows 16 -> 7.7 us, 262 144 rows 20 -> 9.0, 1 000 000 rows 37 -> 25;
+// BiCGSTAB, 262 144 rows 36 -> 16.
+//
+// Blocks wait for one another, so all of them have to be on the chip: the grid
+// is at most what it holds, and before anything is changed the blocks agree
+// that all have arrived (res_enter); where that takes over a tenth of a second
+// (another process has the chip) they agree to leave, and the solve goes on
+// with the launches per step.  After that no block waits for anything but
+// blocks that run.
+constexpr int kResGrid = 256;     // blocks: one per CU, and the sums' slots
+constexpr int kResSlots = 8;      // slots of a row in registers
+constexpr int kResIters = 48;     // iterations of a launch (its vectors are loaded and stored once)
+// polls of an entry before the wait is given up (it then counts as NaN and the
+// recurrence breaks down); a poll takes under a microsecond, a real wait tens
+constexpr int kResPolls = 1 << 20;
+
+struct ResCtl {
+  unsigned int arrived;    // blocks of all launches so far
+  unsigned int decision;   // 2 * launch + 1: go, + 2: leave
+  unsigned int sums;       // sums over the blocks so far (which slots come next)
+};
+
+template <typename T>
+struct ResArgs {
+  KState* st;
+  ResCtl* ctl;
+  double* slots;           // [4][2][kResGrid], unset between uses
+  T* xb[2];                // exchanged entries, unset between uses
+  T *x, *r, *p, *z, *v, *q;
+  const T* d;
+  double* hist;
+  int iters;
+  unsigned int launch;     // 1, 2, ... of the solve
+};
+
+// Whether all blocks of the launch run together (see above).  Every block
+// arrives in every launch, so the count tells.
+__device__ __forceinline__ bool res_enter(ResCtl* c, unsigned int launch, KState* st) {
+  __shared__ int go;
+  if (threadIdx.x == 0) {
+    __hip_atomic_fetch_add(&c->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    go = 0;
+    if (!halted(st)) {
+      const unsigned int yes = 2 * launch + 1, no = yes + 1;
+      const long long t0 = wall_clock64();   // 100 MHz
+      for (;;) {
+        unsigned int d = __hip_atomic_load(&c->decision, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+        if (d == yes || d == no) {
+          go = d == yes;
+          break;
+        }
+        const bool all = __hip_atomic_load(&c->arrived, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT) == launch * gridDim.x;
+        if (all || wall_clock64() - t0 > 10000000)
+          __hip_atomic_compare_exchange_strong(&c->decision, &d, all ? yes : no, __ATOMIC_RELAXED,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if (!go && blockIdx.x == 0) st->left = 1;
+    }
+  }
+  __syncthreads();
+  return go != 0;
+}
+
+// Sums over all blocks, the same bits in each.  Slots rotate through four
+// sets: once a block has seen everybody's values of sum j, everybody has done
+// with those of j - 1, and it sets its own of that set back for j + 3.  WAIT:
+// every earlier store of the block (entries and slots set back) arrives before
+// its values do; the sums after a product wait, where those stores are long on
+// their way, and of any two sums in a row at least one does, which is what the
+// slots need.
+template <int NT, int NP, bool WAIT>
+__device__ __forceinline__ void res_sum(double (&v)[NP], double* slots, unsigned int j) {
+  typedef unsigned long long U;
+  __shared__ double lds[NP][NT / kWave];
+  __shared__ double tot[NP][kResGrid / kWave];
+  if (WAIT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int wid = threadIdx.x >> 6;
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    const double w = wave_sum(v[p]);
+    if ((threadIdx.x & 63) == 0) lds[p][wid] = w;
+  }
+  __syncthreads();
+  U* now = reinterpret_cast<U*>(slots) + (size_t)(j % 4) * 2 * kResGrid;
+  U* old = reinterpret_cast<U*>(slots) + (size_t)((j + 3) % 4) * 2 * kResGrid;
+  if ((int)threadIdx.x < NP) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < NT / kWave; k++) s += lds[threadIdx.x][k];
+    __hip_atomic_store(now + threadIdx.x * kResGrid + blockIdx.x,
+                       __builtin_bit_cast(U, set_value(s)), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  }
+  static_assert(NT >= kResGrid, "a thread per slot");
+  if ((int)threadIdx.x < kResGrid) {
+    double t[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) t[p] = 0.0;
+    if (threadIdx.x < gridDim.x)
+      for (int polls = 0; polls < kResPolls; polls++) {
+        bool all = true;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          t[p] = ld_agent(reinterpret_cast<const double*>(now) + p * kResGrid + threadIdx.x);
+          all = all && !is_unset(t[p]);
+        }
+        if (all) break;
+      }
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const double w = wave_sum(t[p]);
+      if ((threadIdx.x & 63) == 0) tot[p][wid] = w;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 2)
+    __hip_atomic_store(old + threadIdx.x * kResGrid + blockIdx.x, MarkBits<double>::unset,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    v[p] = 0.0;
+#pragma unroll
+    for (int k = 0; k < kResGrid / kWave; k++) v[p] += tot[p][k];
+  }
+}
+
+// At the start of a launch: the slots of the last sum before it are still set.
+__device__ __forceinline__ void res_slots_back(double* slots, unsigned int j) {
+  if (threadIdx.x < 2)
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(slots) +
+                           ((size_t)((j + 3) % 4) * 2 + threadIdx.x) * kResGrid + blockIdx.x,
+                       MarkBits<double>::unset, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Where a row's slots are.
+template <typename T>
+struct ResRow {
+  const short* pe;   // 16-bit offsets (and pb their bases), or null
+  const int* pb;
+  const int* pj;
+  const T* pv;
+  int stride, w;
+};
+template <typename T, int HK>
+__device__ __forceinline__ ResRow<T> res_row(const HllView<T, HK>& m, int r) {
+  ResRow<T> o;
+  o.stride = HK > 0 ? HK : m.hksz;
+  const int hk = r / o.stride, lane = r - hk * o.stride, off0 = m.hkoffs[hk];
+  o.w = (m.hkoffs[hk + 1] - off0) / o.stride;
+  o.pe = m.res16 ? m.res16 + off0 + lane : nullptr;
+  o.pb = m.res16 ? m.base16 + off0 / o.stride : nullptr;
+  o.pj = m.ja + off0 + lane;
+  o.pv = m.val + off0 + lane;
+  return o;
+}
+template <typename T>
+__device__ __forceinline__ ResRow<T> res_row(const EllView<T>& m, int r) {
+  ResRow<T> o;
+  o.stride = m.pitch;
+  o.w = m.nzm;
+  o.pe = m.res16 ? m.res16 + r : nullptr;
+  o.pb = m.res16 ? m.base16 + (size_t)(r >> 6) * m.nzm : nullptr;
+  o.pj = m.ja + r;
+  o.pv = m.val + r;
+  return o;
+}
+template <typename T>
+__device__ __forceinline__ int res_col(const ResRow<T>& o, int r, int j) {
+  return o.pe ? r + o.pb[j] + (int)o.pe[(size_t)j * o.stride] : o.pj[(size_t)j * o.stride] - 1;
+}
+
+// acc += v[k] x[r0 + c[k]] for k < w in slot order (the bits of slot_dot), x
+// exchanged: the block's own rows [r0, r0 + rows) from xs in LDS, the others
+// polled in xb.  c[k] for k >= w is some row of the block.
+template <typename T>
+__device__ __forceinline__ T res_group(const int (&c)[kResSlots], const T (&v)[kResSlots], int w,
+                                       int r0, int rows, const T* xs, const T* xb, T acc) {
+  const char* xr = reinterpret_cast<const char*>(xb + r0);
+  // l: opaque, or the compiler keeps every slot's addresses and masks over the
+  // iterations and spills them.  Named scalars: an array that the loop below
+  // reads became one tuple of registers, copied and waited for at every load.
+#define PSB_RES_8(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7)
+#define PSB_RES_OUT(k)                                                                       \
+  int l##k = c[k];                                                                           \
+  asm volatile("" : "+v"(l##k));                                                             \
+  T x##k = T(0);                                                                             \
+  if ((unsigned)l##k >= (unsigned)rows)                                                      \
+    x##k = ld_agent(reinterpret_cast<const T*>(xr + l##k * (int)sizeof(T)));
+#define PSB_RES_OWN(k) \
+  if ((unsigned)l##k < (unsigned)rows) x##k = xs[l##k];
+#define PSB_RES_UNSET(k) || is_unset(x##k)
+#define PSB_RES_AGAIN(k) \
+  if (is_unset(x##k)) x##k = ld_agent(reinterpret_cast<const T*>(xr + l##k * (int)sizeof(T)));
+#define PSB_RES_FMA(k)                    \
+  {                                       \
+    const T t = fma(v[k], x##k, acc);     \
+    acc = k < w ? t : acc;                \
+  }
+  static_assert(kResSlots == 8, "PSB_RES_8");
+  PSB_RES_8(PSB_RES_OUT)
+  PSB_RES_8(PSB_RES_OWN)
+  for (int polls = 0; polls < kResPolls; polls++) {
+    if (!(false PSB_RES_8(PSB_RES_UNSET))) break;
+    PSB_RES_8(PSB_RES_AGAIN)
+  }
+  PSB_RES_8(PSB_RES_FMA)
+#undef PSB_RES_8
+#undef PSB_RES_OUT
+#undef PSB_RES_OWN
+#undef PSB_RES_UNSET
+#undef PSB_RES_AGAIN
+#undef PSB_RES_FMA
+  return acc;
+}
+
+// A thread's rows r0 + k*NT + t, k < RPT, of the matrix: the first kResSlots
+// slots of each in registers for the whole launch (a 7-point stencil's all),
+// the others read in every product (one row a thread only).  Columns are kept
+// relative to r0.  C16: four rows of FP64 leave no room for 32-bit columns, so
+// 16-bit offsets are kept, and in LDS (bases) what a wavefront's 64 rows add to
+// them (res16 storage of ELL or of hacks of a multiple of 64 rows).
+template <typename T, class M, int NT, int RPT, bool C16>
+struct ResRows {
+  T v[RPT][kResSlots];
+  int c[RPT][C16 ? kResSlots / 2 : kResSlots];
+  int w[RPT];
+  int* bases;   // of the wavefront, [RPT][kResSlots]
+
+  __device__ __forceinline__ void load(const M& m, int r0, int rows) {
+#pragma unroll
+    for (int k = 0; k < RPT; k++) {
+      const int t = k * NT + (int)threadIdx.x;
+      w[k] = 0;
+      if (t >= rows) continue;
+      const int r = r0 + t;
+      const ResRow<T> o = res_row(m, r);
+      w[k] = o.w;
+#pragma unroll
+      for (int j = 0; j < kResSlots; j++) {
+        const int jj = j < o.w ? j : 0;
+        v[k][j] = j < o.w ? o.pv[(size_t)jj * o.stride] : T(0);
+        if constexpr (C16) {
+          const int e = j < o.w ? (int)(unsigned short)o.pe[(size_t)jj * o.stride] : 0;
+          c[k][j / 2] = j % 2 ? c[k][j / 2] | e << 16 : e;
+          bases[k * kResSlots + j] = k * NT + (j < o.w ? o.pb[jj] : 0);
+        } else {
+          c[k][j] = (j < o.w ? res_col(o, r, jj) : r) - r0;
+        }
+      }
+    }
+  }
+
+  // row k's product with x (res_group)
+  __device__ __forceinline__ T dot(const M& m, int k, int r0, int rows, const T* xs,
+                                   const T* xb) const {
+    if constexpr (C16) {
+      int cc[kResSlots];
+#pragma unroll
+      for (int j = 0; j < kResSlots; j += 2) {
+        int e = c[k][j / 2];
+        asm volatile("" : "+v"(e));   // or the sums are kept, and spilled
+        cc[j] = (int)threadIdx.x + bases[k * kResSlots + j] + (int)(short)e;
+        cc[j + 1] = (int)threadIdx.x + bases[k * kResSlots + j + 1] + (e >> 16);
+      }
+      return res_group<T>(cc, v[k], w[k], r0, rows, xs, xb, T(0));
+    } else {
+      T acc = res_group<T>(c[k], v[k], w[k], r0, rows, xs, xb, T(0));
+      if constexpr (RPT == 1) {
+        if (w[k] > kResSlots) {
+          const int r = r0 + (int)threadIdx.x;
+          const ResRow<T> o = res_row(m, r);
+          for (int j = kResSlots; j < o.w; j += kResSlots) {
+            T vv[kResSlots];
+            int cc[kResSlots];
+#pragma unroll
+            for (int i = 0; i < kResSlots; i++) {
+              const int jj = j + i < o.w ? j + i : o.w - 1;
+              cc[i] = res_col(o, r, jj) - r0;
+              vv[i] = o.pv[(size_t)jj * o.stride];
+            }
+            acc = res_group<T>(cc, vv, o.w - j, r0, rows, xs, xb, acc);
+          }
+        }
+      }
+      return acc;
+    }
+  }
+};
+
+// A vector of which a thread only touches its own rows: registers, or LDS
+// where a thread has several rows.
+template <typename T, int NT, int RPT>
+struct ResVec {
+  T* lds;
+  T reg[RPT > 1 ? 1 : RPT];
+  __device__ __forceinline__ T& operator[](int k) {
+    if constexpr (RPT > 1) return lds[k * NT + threadIdx.x];
+    else return reg[k];
+  }
+};
+#define PSB_RES_VEC(name)                             \
+  __shared__ T name##_lds[RPT > 1 ? NT * RPT : 1];    \
+  ResVec<T, NT, RPT> name;                            \
+  name.lds = name##_lds
+
+// The rows of thread t of a block: r0 + k*NT + t, k < RPT.
+#define PSB_RES_ROWS _Pragma("unroll") for (int k = 0; k < RPT; k++)
+
+template <typename T, class M, int NT, int RPT, bool C16, int OP>
+__global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
+  __shared__ T ps[NT * RPT];
+  __shared__ KState S;
+  if (!res_enter(a.ctl, a.launch, a.st)) return;
+  const int n = m.nr, r0 = blockIdx.x * (NT * RPT);
+  const int rows = min(NT * RPT, n - r0);
+  unsigned int j = a.ctl->sums;
+  if (threadIdx.x == 0) S = *a.st;
+  res_slots_back(a.slots, j);
+  __shared__ int bases[C16 ? NT / kWave * RPT * kResSlots : 1];
+  ResRows<T, M, NT, RPT, C16> mr;
+  mr.bases = bases + (C16 ? (int)threadIdx.x / kWave * RPT * kResSlots : 0);
+  mr.load(m, r0, rows);
+  PSB_RES_VEC(x);
+  PSB_RES_VEC(r);
+  PSB_RES_VEC(d);
+  PSB_RES_ROWS {
+    const int t = k * NT + (int)threadIdx.x, i = r0 + t;
+    const bool in = t < rows;
+    x[k] = in ? a.x[i] : T(0);
+    r[k] = in ? a.r[i] : T(0);
+    d[k] = in && a.d ? a.d[i] : T(1);
+    ps[t] = in ? a.p[i] : T(0);
+  }
+  __syncthreads();
+  double* hist = blockIdx.x == 0 ? a.hist : nullptr;
+  for (int it = 0; it < a.iters && !halted(&S); it++) {
+    T* xb = a.xb[it & 1];
+    const bool first = S.it == 0;
+    const T beta = (T)S.beta;
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      const T z = a.d ? d[k] * r[k] : r[k];
+      const T p = set_value(first ? z : z + beta * ps[t]);
+      if (t < rows) st_agent(xb + r0 + t, p);
+      ps[t] = p;
+    }
+    __syncthreads();
+    T q[RPT];
+    double s[1] = {0.0};
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      q[k] = T(0);
+      if (t < rows) {
+        q[k] = mr.dot(m, k, r0, rows, ps, xb);
+        s[0] += (double)ps[t] * (double)q[k];
+      }
+    }
+    res_sum<NT, 1, true>(s, a.slots, j++);
+    PSB_RES_ROWS {   // every block has its product: the entries go back
+      const int t = k * NT + (int)threadIdx.x;
+      if (t < rows) st_agent(xb + r0 + t, __builtin_bit_cast(T, MarkBits<T>::unset));
+    }
+    if (threadIdx.x == 0) fin_apply<FIN_CG_Q, 1>(&S, s, hist, nullptr);
+    __syncthreads();
+    if (halted(&S)) break;
+    const T alpha = (T)S.alpha;
+    double w[2] = {0.0, 0.0};
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      x[k] = x[k] + alpha * ps[t];
+      const T rk = r[k] - alpha * q[k];
+      r[k] = rk;
+      const T z = a.d ? d[k] * rk : rk;
+      if (t < rows) {
+        w[0] += (double)rk * (double)rk;
+        w[1] += (double)rk * (double)z;
+      }
+    }
+    res_sum<NT, 2, false>(w, a.slots, j++);
+    if (threadIdx.x == 0) fin_apply<OP, 2>(&S, w, hist, nullptr);
+    __syncthreads();
+  }
+  PSB_RES_ROWS {
+    const int t = k * NT + (int)threadIdx.x, i = r0 + t;
+    if (t < rows) {
+      a.x[i] = x[k];
+      a.r[i] = r[k];
+      a.p[i] = ps[t];
+      if (a.d) a.z[i] = d[k] * r[k];
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *a.st = S;
+    a.ctl->sums = j;
+  }
+}
+
+template <typename T, class M, int NT, int RPT>
+__global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
+  __shared__ T ps[NT * RPT];
+  __shared__ KState S;
+  if (!res_enter(a.ctl, a.launch, a.st)) return;
+  const int n = m.nr, r0 = blockIdx.x * (NT * RPT);
+  const int rows = min(NT * RPT, n - r0);
+  unsigned int j = a.ctl->sums;
+  if (threadIdx.x == 0) S = *a.st;
+  res_slots_back(a.slots, j);
+  ResRows<T, M, NT, RPT, false> mr;
+  mr.load(m, r0, rows);
+  PSB_RES_VEC(x);
+  PSB_RES_VEC(p);
+  PSB_RES_VEC(q);
+  PSB_RES_VEC(d);
+  T r[RPT], v[RPT];
+  PSB_RES_ROWS {
+    const int i = r0 + k * NT + (int)threadIdx.x;
+    const bool in = i < n;
+    x[k] = in ? a.x[i] : T(0);
+    r[k] = in ? a.r[i] : T(0);
+    p[k] = in ? a.p[i] : T(0);
+    v[k] = in ? a.v[i] : T(0);
+    q[k] = in ? a.q[i] : T(0);
+    d[k] = in && a.d ? a.d[i] : T(1);
+  }
+  __syncthreads();
+  double* hist = blockIdx.x == 0 ? a.hist : nullptr;
+  const T gone = __builtin_bit_cast(T, MarkBits<T>::unset);
+  for (int it = 0; it < a.iters && !halted(&S); it++) {
+    const bool first = S.it == 0;
+    const T beta = (T)S.beta, momega = (T)(-S.omega);
+    T f[RPT], t_[RPT], s[RPT], z[RPT];
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      const T pk = first ? r[k] : r[k] + beta * (momega * v[k] + p[k]);
+      p[k] = pk;
+      f[k] = set_value(a.d ? d[k] * pk : pk);
+      if (t < rows) {
+        st_agent(a.xb[0] + r0 + t, f[k]);
+        ps[t] = f[k];
+      }
+    }
+    __syncthreads();
+    double c[1] = {0.0};
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      v[k] = T(0);
+      if (t < rows) {
+        v[k] = mr.dot(m, k, r0, rows, ps, a.xb[0]);
+        c[0] += (double)q[k] * (double)v[k];
+      }
+    }
+    res_sum<NT, 1, true>(c, a.slots, j++);
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      if (t < rows) st_agent(a.xb[0] + r0 + t, gone);
+    }
+    if (threadIdx.x == 0) fin_apply<FIN_BI_V, 1>(&S, c, hist, nullptr);
+    __syncthreads();
+    if (halted(&S)) break;
+    const T alpha = (T)S.alpha, malpha = (T)(-S.alpha);
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      s[k] = malpha * v[k] + r[k];
+      z[k] = set_value(a.d ? d[k] * s[k] : s[k]);
+      if (t < rows) {
+        st_agent(a.xb[1] + r0 + t, z[k]);
+        ps[t] = z[k];
+      }
+    }
+    __syncthreads();
+    double w[2] = {0.0, 0.0};
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      t_[k] = T(0);
+      if (t < rows) {
+        t_[k] = mr.dot(m, k, r0, rows, ps, a.xb[1]);
+        w[0] += (double)t_[k] * (double)t_[k];
+        w[1] += (double)t_[k] * (double)s[k];
+      }
+    }
+    res_sum<NT, 2, true>(w, a.slots, j++);
+    PSB_RES_ROWS {
+      const int t = k * NT + (int)threadIdx.x;
+      if (t < rows) st_agent(a.xb[1] + r0 + t, gone);
+    }
+    if (threadIdx.x == 0) fin_apply<FIN_BI_T, 2>(&S, w, hist, nullptr);
+    __syncthreads();
+    if (halted(&S)) break;
+    const T omega = (T)S.omega;
+    w[0] = w[1] = 0.0;
+    PSB_RES_ROWS {
+      x[k] = omega * z[k] + (alpha * f[k] + x[k]);
+      r[k] = -omega * t_[k] + s[k];
+      if (k * NT + (int)threadIdx.x < rows) {
+        w[0] += (double)r[k] * (double)r[k];
+        w[1] += (double)q[k] * (double)r[k];
+      }
+    }
+    res_sum<NT, 2, false>(w, a.slots, j++);
+    if (threadIdx.x == 0) fin_apply<FIN_BI_X, 2>(&S, w, hist, nullptr);
+    __syncthreads();
+  }
+  PSB_RES_ROWS {
+    const int i = r0 + k * NT + (int)threadIdx.x;
+    if (i < n) {
+      a.x[i] = x[k];
+      a.r[i] = r[k];
+      a.p[i] = p[k];
+      a.v[i] = v[k];
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *a.st = S;
+    a.ctl->sums = j;
+  }
+}
+#undef PSB_RES_ROWS
+#undef PSB_RES_VEC
+
 // --------------------------------------------------------------- mixed precision helpers
 // r32 = (float)(r * inv), inv = 1/||r|| read from device
 __global__ __launch_bounds__(kBlock) void k_to_single(int n, const double* __restrict__ r,
@@ -720,6 +1257,12 @@ __global__ __launch_bounds__(kBlock) void k_d2s_vec(int n, const double* __restr
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_zero(int n, T* __restrict__ a) {
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) a[i] = T(0);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_mark(int n, T* __restrict__ a) {
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
+    a[i] = __builtin_bit_cast(T, MarkBits<T>::unset);
 }
 
 __global__ __launch_bounds__(kBlock) void k_unset(int n, unsigned long long* __restrict__ a) {
@@ -770,6 +1313,12 @@ struct Solver {
   double* partials = nullptr;
   double* hist = nullptr;
   double* fold = nullptr;        // slots of folded finalisations, kUnsetBits between uses
+  // resident iterations (k_res_cg, k_res_bi): control block, sum slots, exchanged
+  // entries (null: launches per step)
+  ResCtl* rctl = nullptr;
+  double* rslots = nullptr;
+  void* rx[2] = {nullptr, nullptr};
+  unsigned int launches = 0;
   std::vector<void*> bufs;
   hipStream_t stream = nullptr;
   // allocation-free mode: device buffers are carved from the library's
@@ -812,6 +1361,40 @@ static size_t solve_bytes(int method, int n, int etype, int itmax) {
          align256(sizeof(double) * ((size_t)itmax + 2)) + (method == 0 ? 4 : 8) * vec;
 }
 static_assert(3 * sizeof(KState) <= kScratchHostBytes, "host mirror + ring in the pinned block");
+
+constexpr size_t kFoldBytes = sizeof(double) * 2 * kFoldGrid;
+constexpr size_t kResSlotBytes = sizeof(double) * 4 * 2 * kResGrid;
+
+static size_t resident_bytes(int n, int etype) {
+  return 256 + align256(kResSlotBytes) + 2 * align256(elem_size(etype) * (size_t)n);
+}
+
+// Rows per thread of a resident solve of n rows in blocks of nt threads, 0
+// where the solve takes launches per step: CSR, more rows than threads hold
+// (four rows each for CG and two for BiCGSTAB), several rows a thread wider
+// than the registers hold or, four of FP64, not in 16-bit storage (ResRows),
+// fewer CUs than blocks, or buffers that the allocation-free entry point could
+// not hold (both entry points choose alike).
+static int resident_rows(const Solver& s, int itmax, int* nt) {
+  if (s.fmt == FMT_CSR || s.n <= 0) return 0;
+  if ((s.fmt == FMT_HLL ? ((HllDev*)s.mat)->max_col : ((EllDev*)s.mat)->max_col) > s.n) return 0;
+  if (solve_bytes(s.method, s.n, s.etype, itmax) + align256(kFoldBytes) +
+          resident_bytes(s.n, s.etype) > kScratchBytes)
+    return 0;
+  *nt = s.n <= 256 * kResGrid ? 256 : 1024;
+  const int most = s.method == 0 ? 4 : 2;
+  int rpt = 1;
+  while ((s.n + *nt * rpt - 1) / (*nt * rpt) > kResGrid) rpt *= 2;
+  if (rpt > most || (s.n + *nt * rpt - 1) / (*nt * rpt) > ctx().num_cus) return 0;
+  const HllDev* h = (const HllDev*)s.mat;
+  const EllDev* e = (const EllDev*)s.mat;
+  const bool hll = s.fmt == FMT_HLL;
+  if (rpt > 1 && (hll ? h->max_width : e->nzm) > kResSlots) return 0;
+  if (rpt == 4 && s.etype == PSB_HIP_TYPE_DOUBLE &&
+      !(hll ? hll_use_idx16(h) && h->hksz % 64 == 0 : ell_use_idx16(e)))
+    return 0;
+  return rpt;
+}
 
 template <typename T>
 struct Mats {
@@ -999,6 +1582,63 @@ static int bi_iter(Solver& s, const Mats<T>& m, T* x, T* r, T* q, T* p, T* v, T*
   return PSB_HIP_SUCCESS;
 }
 
+// One launch of up to iters resident iterations (OP: FIN_CG_X or FIN_RU_X for
+// CG, FIN_BI_X for BiCGSTAB).
+template <typename T, int OP, class M>
+static int resident_launch(Solver& s, const M& m, ResArgs<T> a, int nt, int rpt) {
+  a.launch = ++s.launches;
+  const int grid = (s.n + nt * rpt - 1) / (nt * rpt);
+#define PSB_RES(NT, RPT)                                                                         \
+  do {                                                                                           \
+    if constexpr (OP == FIN_BI_X)                                                                \
+      hipLaunchKernelGGL((k_res_bi<T, M, NT, RPT>), dim3(grid), dim3(NT), 0, s.stream, m, a);    \
+    else                                                                                         \
+      hipLaunchKernelGGL((k_res_cg<T, M, NT, RPT, (sizeof(T) == 8 && RPT == 4), OP>), dim3(grid), \
+                         dim3(NT), 0, s.stream, m, a);                                           \
+  } while (0)
+  if (nt == 256) PSB_RES(256, 1);
+  else if (rpt == 1) PSB_RES(1024, 1);
+  else if (rpt == 2) PSB_RES(1024, 2);
+  else if constexpr (OP != FIN_BI_X) PSB_RES(1024, 4);
+#undef PSB_RES
+  PSB_HIP_LAUNCH_CHECK();
+  return PSB_HIP_SUCCESS;
+}
+
+template <typename T, int OP>
+static int resident_batch(Solver& s, const Mats<T>& m, const ResArgs<T>& a, int nt, int rpt) {
+  if (s.fmt == FMT_HLL && m.hll.hksz == 64)
+    return resident_launch<T, OP>(s, as64(m.hll), a, nt, rpt);
+  if (s.fmt == FMT_HLL) return resident_launch<T, OP>(s, m.hll, a, nt, rpt);
+  return resident_launch<T, OP>(s, m.ell, a, nt, rpt);
+}
+
+// The buffers of a resident solve; every entry starts unset.
+template <typename T>
+static int resident_setup(Solver& s, ResArgs<T>* a) {
+  int rc = s.alloc((void**)&s.rctl, sizeof(ResCtl));
+  if (!rc) rc = s.alloc((void**)&s.rslots, kResSlotBytes);
+  for (int k = 0; k < 2 && !rc; k++) rc = s.alloc(&s.rx[k], sizeof(T) * (size_t)s.n);
+  if (rc) return rc;
+  static_assert(sizeof(ResCtl) == 3 * sizeof(unsigned int), "cleared as words");
+  hipLaunchKernelGGL((k_zero<unsigned int>), dim3(1), dim3(kBlock), 0, s.stream, 3,
+                     (unsigned int*)s.rctl);
+  hipLaunchKernelGGL((k_mark<double>), dim3(stream_grid(8 * kResGrid)), dim3(kBlock), 0, s.stream,
+                     8 * kResGrid, s.rslots);
+  for (int k = 0; k < 2; k++)
+    hipLaunchKernelGGL((k_mark<T>), dim3(stream_grid(s.n)), dim3(kBlock), 0, s.stream, s.n,
+                       (T*)s.rx[k]);
+  PSB_HIP_LAUNCH_CHECK();
+  *a = ResArgs<T>{};
+  a->st = s.st;
+  a->ctl = s.rctl;
+  a->slots = s.rslots;
+  a->xb[0] = (T*)s.rx[0];
+  a->xb[1] = (T*)s.rx[1];
+  a->hist = s.hist;
+  return PSB_HIP_SUCCESS;
+}
+
 static int read_state(Solver& s) {
   PSB_HIP_CHECK(hipMemcpyAsync(s.hst, s.st, sizeof(KState), hipMemcpyDeviceToHost, s.stream));
   PSB_HIP_CHECK(hipStreamSynchronize(s.stream));
@@ -1024,7 +1664,7 @@ static int post_state(Solver& s) {
 static int prev_halted(Solver& s, bool* halted) {
   const int k = (s.posted - 2) & 1;
   PSB_HIP_CHECK(hipEventSynchronize(s.ev[k]));
-  *halted = s.ring[k].done != 0 || s.ring[k].breakdown != 0;
+  *halted = s.ring[k].done != 0 || s.ring[k].breakdown != 0 || s.ring[k].left != 0;
   return PSB_HIP_SUCCESS;
 }
 
@@ -1061,10 +1701,17 @@ static int solve(Solver& s, const T* b, T* x, const T* d, double eps, int itmax,
   int rc = bnorm<T>(s, b);
   if (rc) return rc;
   if (check_every < 1) check_every = 8;
+  ResArgs<T> ra;
+  int rnt = 0;
+  int rpt = resident_rows(s, itmax, &rnt);   // 0: launches per step
+  if (rpt && (rc = resident_setup<T>(s, &ra))) return rc;
+  bool fresh = true;   // the recurrence starts from b - A x
   for (;;) {
     // restart: r = b - A x (and the first z / rho); without a preconditioner
     // the vectors it would only copy are aliased (z = r, f = p, z = s)
-    if (s.method == 0) {
+    if (!fresh) {
+      fresh = true;
+    } else if (s.method == 0) {
       T* z = d ? w[3] : w[0];
       rc = restart<T>(s, m, b, x, w[0], nullptr, d, z, 0);
     } else {
@@ -1072,6 +1719,25 @@ static int solve(Solver& s, const T* b, T* x, const T* d, double eps, int itmax,
     }
     if (rc) return rc;
     auto batch = [&]() -> int {
+      if (rpt) {
+        ra.x = x;
+        ra.r = w[0];
+        ra.d = d;
+        ra.iters = check_every > kResIters ? check_every : kResIters;
+        if (s.method == 0) {
+          ra.p = w[1];
+          ra.z = d ? w[3] : w[0];
+          const int rk = resident_batch<T, FIN_CG_X>(s, m, ra, rnt, rpt);
+          if (rk) return rk;
+        } else {
+          ra.q = w[1];
+          ra.p = w[2];
+          ra.v = w[3];
+          const int rk = resident_batch<T, FIN_BI_X>(s, m, ra, rnt, rpt);
+          if (rk) return rk;
+        }
+        return post_state(s);
+      }
       for (int k = 0; k < check_every; k++) {
         int rk;
         if (s.method == 0) {
@@ -1095,6 +1761,12 @@ static int solve(Solver& s, const T* b, T* x, const T* d, double eps, int itmax,
     }
     if ((rc = read_state(s))) return rc;
     if (s.hst->done) break;
+    if (s.hst->left) {   // the chip was not free: go on from here with launches per step
+      rpt = 0;
+      s.hst->left = 0;
+      PSB_HIP_CHECK(hipMemcpyAsync(s.st, s.hst, sizeof(KState), hipMemcpyHostToDevice, s.stream));
+      fresh = s.hst->breakdown != 0;
+    }
     // breakdown: restart unless the iteration budget is spent
     if (s.hst->itx >= itmax) break;
     s.hst->breakdown = 0;
@@ -1133,7 +1805,6 @@ static int describe(Solver& s, int method, int fmt, void* dmat) {
   return PSB_HIP_SUCCESS;
 }
 
-constexpr size_t kFoldBytes = sizeof(double) * 2 * kFoldGrid;
 // by a kernel: a caller may capture the solve
 static int clear_fold(Solver& s) {
   hipLaunchKernelGGL(k_unset, dim3(stream_grid(2 * kFoldGrid)), dim3(kBlock), 0, s.stream,
@@ -1251,9 +1922,24 @@ static int mixed_reliable(HllDev* h, const double* b, double* x, const double* d
   if (check_every < 1) check_every = 8;
   dim3 gv(vec_grid<float>(n));
   const int gsp = spmv_grid(n, inner.rpl);
+  ResArgs<float> ra;
+  int rnt = 0;
+  int rpt = resident_rows(inner, inner_itmax, &rnt);   // 0: launches per step
+  if (rpt && (rc = resident_setup<float>(inner, &ra))) return rc;
   while (!conv) {
     // queue FP32 iterations until a replacement (or breakdown) is requested
     auto batch = [&]() -> int {
+      if (rpt) {
+        ra.x = x32;
+        ra.r = r;
+        ra.p = p;
+        ra.z = z;
+        ra.d = d;
+        ra.iters = check_every > kResIters ? check_every : kResIters;
+        const int rk = resident_batch<float, FIN_RU_X>(inner, m32, ra, rnt, rpt);
+        if (rk) return rk;
+        return post_state(inner);
+      }
       for (int k = 0; k < check_every; k++) {
         hipLaunchKernelGGL((k_cg_p<float>), gv, blk, 0, stream, n, (const float*)z, p, inner.st);
         if (m32.hll.hksz == 64)
@@ -1278,6 +1964,13 @@ static int mixed_reliable(HllDev* h, const double* b, double* x, const double* d
       if ((rc = prev_halted(inner, &stop))) return rc;
     }
     if ((rc = read_state(inner))) return rc;
+    if (inner.hst->left) {   // the chip was not free: go on with launches per step
+      rpt = 0;
+      inner.hst->left = 0;
+      PSB_HIP_CHECK(hipMemcpyAsync(inner.st, inner.hst, sizeof(KState), hipMemcpyHostToDevice,
+                                   stream));
+      if (!inner.hst->breakdown) continue;
+    }
     // replacement: x += x32 in FP64, r = b - A x in FP64
     hipLaunchKernelGGL(k_ru_accum, gs, blk, 0, stream, n, x, x32);
     PSB_HIP_LAUNCH_CHECK();

@@ -272,6 +272,59 @@ __device__ __forceinline__ void grid_reduce(double v, double* partials, unsigned
   }
 }
 
+// ------------------------------------------------------------------ entries that say whether they are there
+// The bit pattern of an entry that is not there yet: a quiet NaN with a payload
+// of its own.  A computed NaN with exactly these bits is stored as the default
+// NaN instead.  Blocks that wait for one another's entries poll the entries
+// themselves: no flag, no fence.
+template <typename T>
+struct MarkBits;
+template <>
+struct MarkBits<double> {
+  typedef unsigned long long U;
+  static constexpr U unset = 0x7ff8a5c3e1d2b497ull, nan = 0x7ff8000000000000ull;
+};
+template <>
+struct MarkBits<float> {
+  typedef unsigned int U;
+  static constexpr U unset = 0x7fe5a3c9u, nan = 0x7fc00000u;
+};
+template <typename T>
+__device__ __forceinline__ bool is_unset(T v) {
+  return __builtin_bit_cast(typename MarkBits<T>::U, v) == MarkBits<T>::unset;
+}
+template <typename T>
+__device__ __forceinline__ T set_value(T v) {   // v, never the unset pattern
+  typedef typename MarkBits<T>::U U;
+  const U u = __builtin_bit_cast(U, v);
+  return __builtin_bit_cast(T, u == MarkBits<T>::unset ? MarkBits<T>::nan : u);
+}
+// agent-scope (all XCDs) and workgroup-scope (LDS) accesses of one entry
+template <typename T>
+__device__ __forceinline__ T ld_agent(const T* p) {
+  typedef typename MarkBits<T>::U U;
+  return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const U*>(p), __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT));
+}
+template <typename T>
+__device__ __forceinline__ void st_agent(T* p, T v) {
+  typedef typename MarkBits<T>::U U;
+  __hip_atomic_store(reinterpret_cast<U*>(p), __builtin_bit_cast(U, v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T ld_lds(const T* p) {
+  typedef typename MarkBits<T>::U U;
+  return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const U*>(p), __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+template <typename T>
+__device__ __forceinline__ void st_lds(T* p, T v) {
+  typedef typename MarkBits<T>::U U;
+  __hip_atomic_store(reinterpret_cast<U*>(p), __builtin_bit_cast(U, v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // XCD-aware block index: blocks are dispatched round-robin over the 8 XCDs;
 // remap so that each XCD works on a contiguous range of the logical grid,
 // keeping neighbouring rows (and the x entries they gather) in one L2.

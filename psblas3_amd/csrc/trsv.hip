@@ -28,7 +28,7 @@
 // staged in LDS, so a step costs LDS traffic and arithmetic only.  A row's
 // dependencies outside its tile (its halo) are polled from the solution array
 // itself, which starts out filled with one NaN bit pattern that no solve
-// stores (tri_unset): an entry is ready once it holds anything else, so a
+// stores (is_unset): an entry is ready once it holds anything else, so a
 // value needs no flag and no fence (8- or 4-byte agent-scope loads and
 // stores).  Three wavefronts of the workgroup poll while the fourth solves.
 // Workgroups take their tiles by a ticket, in an order where a tile depends
@@ -204,60 +204,9 @@ __global__ __launch_bounds__(kBlock) void k_trsv_level(int p0, int count,
   y[p] = DIV ? r / dv[p] : r;
 }
 
-// The bit pattern of a solution entry that is not there yet: a quiet NaN with
-// a payload of its own.  A computed NaN with exactly these bits is stored as
-// the default NaN instead.
-template <typename T>
-struct TriBits;
-template <>
-struct TriBits<double> {
-  typedef unsigned long long U;
-  static constexpr U unset = 0x7ff8a5c3e1d2b497ull, nan = 0x7ff8000000000000ull;
-};
-template <>
-struct TriBits<float> {
-  typedef unsigned int U;
-  static constexpr U unset = 0x7fe5a3c9u, nan = 0x7fc00000u;
-};
-template <typename T>
-__device__ __forceinline__ bool tri_unset(T v) {
-  return __builtin_bit_cast(typename TriBits<T>::U, v) == TriBits<T>::unset;
-}
-template <typename T>
-__device__ __forceinline__ T tri_value(T v) {   // v, never the unset pattern
-  typedef typename TriBits<T>::U U;
-  const U u = __builtin_bit_cast(U, v);
-  return __builtin_bit_cast(T, u == TriBits<T>::unset ? TriBits<T>::nan : u);
-}
-// agent-scope (all XCDs) and workgroup-scope (LDS) accesses of one entry
-template <typename T>
-__device__ __forceinline__ T ld_agent(const T* p) {
-  typedef typename TriBits<T>::U U;
-  return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const U*>(p), __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT));
-}
-template <typename T>
-__device__ __forceinline__ void st_agent(T* p, T v) {
-  typedef typename TriBits<T>::U U;
-  __hip_atomic_store(reinterpret_cast<U*>(p), __builtin_bit_cast(U, v), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ T ld_lds(const T* p) {
-  typedef typename TriBits<T>::U U;
-  return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const U*>(p), __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_WORKGROUP));
-}
-template <typename T>
-__device__ __forceinline__ void st_lds(T* p, T v) {
-  typedef typename TriBits<T>::U U;
-  __hip_atomic_store(reinterpret_cast<U*>(p), __builtin_bit_cast(U, v), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_tri_unset(int64_t n, T* __restrict__ sol) {
-  const T u = __builtin_bit_cast(T, TriBits<T>::unset);
+  const T u = __builtin_bit_cast(T, MarkBits<T>::unset);
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * kBlock)
     sol[i] = u;
@@ -321,7 +270,7 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
   int2* steps = reinterpret_cast<int2*>(at);
   at += lds16(sizeof(int2) * (size_t)t.nstep);
   uint16_t* ed = reinterpret_cast<uint16_t*>(at);
-  const T unset = __builtin_bit_cast(T, TriBits<T>::unset);
+  const T unset = __builtin_bit_cast(T, MarkBits<T>::unset);
 
   for (int p = threadIdx.x; p < t.nrow; p += kTileThreads) {
     const int r = trow[t.row0 + p];
@@ -352,10 +301,10 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
     int src = h < t.nhalo ? thalo[t.halo0 + h] : 0;
     bool open = lane < kFirst;
     while (__any(h < t.nhalo)) {
-      if (!open) open = !tri_unset(ld_lds(ys + t.nrow));
+      if (!open) open = !is_unset(ld_lds(ys + t.nrow));
       if (open && h < t.nhalo) {
         const T v = ld_agent(sol + src);
-        if (!tri_unset(v)) {
+        if (!is_unset(v)) {
           st_lds(ys + t.nrow + h, v);
           h += kPollers;
           if (h < t.nhalo) src = thalo[t.halo0 + h];
@@ -365,7 +314,7 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
       }
       if (++polls > kTilePolls) {
         for (; h < t.nhalo; h += kPollers)
-          st_lds(ys + t.nrow + h, __builtin_bit_cast(T, TriBits<T>::nan));
+          st_lds(ys + t.nrow + h, __builtin_bit_cast(T, MarkBits<T>::nan));
       }
     }
   } else {
@@ -397,7 +346,7 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
       for (;;) {
         bool ready = true;
 #pragma unroll
-        for (int k = 0; k < WR; k++) ready = ready && !tri_unset(yk[k]);
+        for (int k = 0; k < WR; k++) ready = ready && !is_unset(yk[k]);
         if (__all(ready)) break;
         __builtin_amdgcn_s_sleep(1);
         read(dep, yk);
@@ -440,7 +389,7 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
       }
       T r = RUN ? acc : cur.xi - acc;
       if (DIV) r = r / cur.dv;
-      r = tri_value(r);
+      r = set_value(r);
       if (lane < cur.cnt) {
         st_lds(ys + cur.roff + lane, r);
         st_agent(sol + cur.row, r);
