@@ -709,7 +709,7 @@ __global__ __launch_bounds__(kBlock) void k_bi_x(int n, T* __restrict__ x, T* __
 // sums over the blocks and one exchange, 2 us each; above 262144 rows the
 // chain of a thread's rows, each waiting for its exchanged entries, adds to it.
 // An iteration of CG, 7-point, FP64 (launches per step -> resident): 27 000
-// rows 16 -> 7.7 us, 262 144 rows 20 -> 9.0, 1 000 000 rows 37 -> 25;
+// rows 16 -> 7.7 us, 262 144 rows 20 -> 9.0, 1 000 000 rows 37 -> 22;
 // BiCGSTAB, 262 144 rows 36 -> 16.
 //
 // Blocks wait for one another, so all of them have to be on the chip: the grid
@@ -885,27 +885,31 @@ __device__ __forceinline__ int res_col(const ResRow<T>& o, int r, int j) {
 // acc += v[k] x[r0 + c[k]] for k < w in slot order (the bits of slot_dot), x
 // exchanged: the block's own rows [r0, r0 + rows) from xs in LDS, the others
 // polled in xb.  c[k] for k >= w is some row of the block.
-template <typename T>
-__device__ __forceinline__ T res_group(const int (&c)[kResSlots], const T (&v)[kResSlots], int w,
-                                       int r0, int rows, const T* xs, const T* xb, T acc) {
+template <typename T, int W>
+__device__ __forceinline__ T res_group(const int (&c)[W], const T (&v)[W], int w, int r0, int rows,
+                                       const T* xs, const T* xb, T acc) {
   const char* xr = reinterpret_cast<const char*>(xb + r0);
   // l: opaque, or the compiler keeps every slot's addresses and masks over the
   // iterations and spills them.  Named scalars: an array that the loop below
   // reads became one tuple of registers, copied and waited for at every load.
 #define PSB_RES_8(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7)
-#define PSB_RES_OUT(k)                                                                       \
-  int l##k = c[k];                                                                           \
-  asm volatile("" : "+v"(l##k));                                                             \
-  T x##k = T(0);                                                                             \
-  if ((unsigned)l##k >= (unsigned)rows)                                                      \
-    x##k = ld_agent(reinterpret_cast<const T*>(xr + l##k * (int)sizeof(T)));
+#define PSB_RES_OUT(k)                                                            \
+  int l##k = 0;                                                                   \
+  T x##k = T(0);                                                                  \
+  if constexpr (k < W) {                                                          \
+    l##k = c[k];                                                                  \
+    asm volatile("" : "+v"(l##k));                                                \
+    if ((unsigned)l##k >= (unsigned)rows)                                         \
+      x##k = ld_agent(reinterpret_cast<const T*>(xr + l##k * (int)sizeof(T)));    \
+  }
 #define PSB_RES_OWN(k) \
-  if ((unsigned)l##k < (unsigned)rows) x##k = xs[l##k];
-#define PSB_RES_UNSET(k) || is_unset(x##k)
-#define PSB_RES_AGAIN(k) \
-  if (is_unset(x##k)) x##k = ld_agent(reinterpret_cast<const T*>(xr + l##k * (int)sizeof(T)));
+  if (k < W && (unsigned)l##k < (unsigned)rows) x##k = xs[l##k];
+#define PSB_RES_UNSET(k) || (k < W && is_unset(x##k))
+#define PSB_RES_AGAIN(k)          \
+  if (k < W && is_unset(x##k))    \
+    x##k = ld_agent(reinterpret_cast<const T*>(xr + l##k * (int)sizeof(T)));
 #define PSB_RES_FMA(k)                    \
-  {                                       \
+  if constexpr (k < W) {                  \
     const T t = fma(v[k], x##k, acc);     \
     acc = k < w ? t : acc;                \
   }
@@ -926,18 +930,18 @@ __device__ __forceinline__ T res_group(const int (&c)[kResSlots], const T (&v)[k
   return acc;
 }
 
-// A thread's rows r0 + k*NT + t, k < RPT, of the matrix: the first kResSlots
-// slots of each in registers for the whole launch (a 7-point stencil's all),
+// A thread's rows r0 + k*NT + t, k < RPT, of the matrix: the first W slots of
+// each in registers for the whole launch (a 7-point stencil's all),
 // the others read in every product (one row a thread only).  Columns are kept
 // relative to r0.  C16: four rows of FP64 leave no room for 32-bit columns, so
 // 16-bit offsets are kept, and in LDS (bases) what a wavefront's 64 rows add to
 // them (res16 storage of ELL or of hacks of a multiple of 64 rows).
-template <typename T, class M, int NT, int RPT, bool C16>
+template <typename T, class M, int NT, int RPT, int W, bool C16>
 struct ResRows {
-  T v[RPT][kResSlots];
-  int c[RPT][C16 ? kResSlots / 2 : kResSlots];
+  T v[RPT][W];
+  int c[RPT][C16 ? (W + 1) / 2 : W];
   int w[RPT];
-  int* bases;   // of the wavefront, [RPT][kResSlots]
+  int* bases;   // of the wavefront, [RPT][W]
 
   __device__ __forceinline__ void load(const M& m, int r0, int rows) {
 #pragma unroll
@@ -949,13 +953,13 @@ struct ResRows {
       const ResRow<T> o = res_row(m, r);
       w[k] = o.w;
 #pragma unroll
-      for (int j = 0; j < kResSlots; j++) {
+      for (int j = 0; j < W; j++) {
         const int jj = j < o.w ? j : 0;
         v[k][j] = j < o.w ? o.pv[(size_t)jj * o.stride] : T(0);
         if constexpr (C16) {
           const int e = j < o.w ? (int)(unsigned short)o.pe[(size_t)jj * o.stride] : 0;
           c[k][j / 2] = j % 2 ? c[k][j / 2] | e << 16 : e;
-          bases[k * kResSlots + j] = k * NT + (j < o.w ? o.pb[jj] : 0);
+          bases[k * W + j] = k * NT + (j < o.w ? o.pb[jj] : 0);
         } else {
           c[k][j] = (j < o.w ? res_col(o, r, jj) : r) - r0;
         }
@@ -967,31 +971,31 @@ struct ResRows {
   __device__ __forceinline__ T dot(const M& m, int k, int r0, int rows, const T* xs,
                                    const T* xb) const {
     if constexpr (C16) {
-      int cc[kResSlots];
+      int cc[W];
 #pragma unroll
-      for (int j = 0; j < kResSlots; j += 2) {
+      for (int j = 0; j < W; j += 2) {
         int e = c[k][j / 2];
         asm volatile("" : "+v"(e));   // or the sums are kept, and spilled
-        cc[j] = (int)threadIdx.x + bases[k * kResSlots + j] + (int)(short)e;
-        cc[j + 1] = (int)threadIdx.x + bases[k * kResSlots + j + 1] + (e >> 16);
+        cc[j] = (int)threadIdx.x + bases[k * W + j] + (int)(short)e;
+        if (j + 1 < W) cc[j + 1] = (int)threadIdx.x + bases[k * W + j + 1] + (e >> 16);
       }
-      return res_group<T>(cc, v[k], w[k], r0, rows, xs, xb, T(0));
+      return res_group<T, W>(cc, v[k], w[k], r0, rows, xs, xb, T(0));
     } else {
-      T acc = res_group<T>(c[k], v[k], w[k], r0, rows, xs, xb, T(0));
+      T acc = res_group<T, W>(c[k], v[k], w[k], r0, rows, xs, xb, T(0));
       if constexpr (RPT == 1) {
-        if (w[k] > kResSlots) {
+        if (w[k] > W) {
           const int r = r0 + (int)threadIdx.x;
           const ResRow<T> o = res_row(m, r);
-          for (int j = kResSlots; j < o.w; j += kResSlots) {
-            T vv[kResSlots];
-            int cc[kResSlots];
+          for (int j = W; j < o.w; j += W) {
+            T vv[W];
+            int cc[W];
 #pragma unroll
-            for (int i = 0; i < kResSlots; i++) {
+            for (int i = 0; i < W; i++) {
               const int jj = j + i < o.w ? j + i : o.w - 1;
               cc[i] = res_col(o, r, jj) - r0;
               vv[i] = o.pv[(size_t)jj * o.stride];
             }
-            acc = res_group<T>(cc, vv, o.w - j, r0, rows, xs, xb, acc);
+            acc = res_group<T, W>(cc, vv, o.w - j, r0, rows, xs, xb, acc);
           }
         }
       }
@@ -1019,7 +1023,7 @@ struct ResVec {
 // The rows of thread t of a block: r0 + k*NT + t, k < RPT.
 #define PSB_RES_ROWS _Pragma("unroll") for (int k = 0; k < RPT; k++)
 
-template <typename T, class M, int NT, int RPT, bool C16, int OP>
+template <typename T, class M, int NT, int RPT, int W, bool C16, int OP>
 __global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
   __shared__ T ps[NT * RPT];
   __shared__ KState S;
@@ -1029,9 +1033,9 @@ __global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
   unsigned int j = a.ctl->sums;
   if (threadIdx.x == 0) S = *a.st;
   res_slots_back(a.slots, j);
-  __shared__ int bases[C16 ? NT / kWave * RPT * kResSlots : 1];
-  ResRows<T, M, NT, RPT, C16> mr;
-  mr.bases = bases + (C16 ? (int)threadIdx.x / kWave * RPT * kResSlots : 0);
+  __shared__ int bases[C16 ? NT / kWave * RPT * W : 1];
+  ResRows<T, M, NT, RPT, W, C16> mr;
+  mr.bases = bases + (C16 ? (int)threadIdx.x / kWave * RPT * W : 0);
   mr.load(m, r0, rows);
   PSB_RES_VEC(x);
   PSB_RES_VEC(r);
@@ -1108,7 +1112,7 @@ __global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
   }
 }
 
-template <typename T, class M, int NT, int RPT>
+template <typename T, class M, int NT, int RPT, int W>
 __global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
   __shared__ T ps[NT * RPT];
   __shared__ KState S;
@@ -1118,7 +1122,7 @@ __global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
   unsigned int j = a.ctl->sums;
   if (threadIdx.x == 0) S = *a.st;
   res_slots_back(a.slots, j);
-  ResRows<T, M, NT, RPT, false> mr;
+  ResRows<T, M, NT, RPT, W, false> mr;
   mr.load(m, r0, rows);
   PSB_RES_VEC(x);
   PSB_RES_VEC(p);
@@ -1369,6 +1373,11 @@ static size_t resident_bytes(int n, int etype) {
   return 256 + align256(kResSlotBytes) + 2 * align256(elem_size(etype) * (size_t)n);
 }
 
+// Slots of the widest row.
+static int res_width(const Solver& s) {
+  return s.fmt == FMT_HLL ? ((HllDev*)s.mat)->max_width : ((EllDev*)s.mat)->nzm;
+}
+
 // Rows per thread of a resident solve of n rows in blocks of nt threads, 0
 // where the solve takes launches per step: CSR, more rows than threads hold
 // (four rows each for CG and two for BiCGSTAB), several rows a thread wider
@@ -1389,7 +1398,7 @@ static int resident_rows(const Solver& s, int itmax, int* nt) {
   const HllDev* h = (const HllDev*)s.mat;
   const EllDev* e = (const EllDev*)s.mat;
   const bool hll = s.fmt == FMT_HLL;
-  if (rpt > 1 && (hll ? h->max_width : e->nzm) > kResSlots) return 0;
+  if (rpt > 1 && res_width(s) > kResSlots) return 0;
   if (rpt == 4 && s.etype == PSB_HIP_TYPE_DOUBLE &&
       !(hll ? hll_use_idx16(h) && h->hksz % 64 == 0 : ell_use_idx16(e)))
     return 0;
@@ -1588,18 +1597,25 @@ template <typename T, int OP, class M>
 static int resident_launch(Solver& s, const M& m, ResArgs<T> a, int nt, int rpt) {
   a.launch = ++s.launches;
   const int grid = (s.n + nt * rpt - 1) / (nt * rpt);
-#define PSB_RES(NT, RPT)                                                                         \
-  do {                                                                                           \
-    if constexpr (OP == FIN_BI_X)                                                                \
-      hipLaunchKernelGGL((k_res_bi<T, M, NT, RPT>), dim3(grid), dim3(NT), 0, s.stream, m, a);    \
-    else                                                                                         \
-      hipLaunchKernelGGL((k_res_cg<T, M, NT, RPT, (sizeof(T) == 8 && RPT == 4), OP>), dim3(grid), \
-                         dim3(NT), 0, s.stream, m, a);                                           \
+#define PSB_RES(NT, RPT, W)                                                                        \
+  do {                                                                                             \
+    if constexpr (OP == FIN_BI_X)                                                                  \
+      hipLaunchKernelGGL((k_res_bi<T, M, NT, RPT, W>), dim3(grid), dim3(NT), 0, s.stream, m, a);   \
+    else                                                                                           \
+      hipLaunchKernelGGL((k_res_cg<T, M, NT, RPT, W, (sizeof(T) == 8 && RPT == 4), OP>),           \
+                         dim3(grid), dim3(NT), 0, s.stream, m, a);                                 \
   } while (0)
-  if (nt == 256) PSB_RES(256, 1);
-  else if (rpt == 1) PSB_RES(1024, 1);
-  else if (rpt == 2) PSB_RES(1024, 2);
-  else if constexpr (OP != FIN_BI_X) PSB_RES(1024, 4);
+  // seven slots where that is all of a row and registers are short: an
+  // iteration of CG at 1 000 000 rows 25.0 -> 21.6 us
+  const bool w7 = res_width(s) <= 7;
+  if (nt == 256) PSB_RES(256, 1, 8);
+  else if (rpt == 1) PSB_RES(1024, 1, 8);
+  else if (rpt == 2 && w7) PSB_RES(1024, 2, 7);
+  else if (rpt == 2) PSB_RES(1024, 2, 8);
+  else if constexpr (OP != FIN_BI_X) {
+    if (w7) PSB_RES(1024, 4, 7);
+    else PSB_RES(1024, 4, 8);
+  }
 #undef PSB_RES
   PSB_HIP_LAUNCH_CHECK();
   return PSB_HIP_SUCCESS;

@@ -15,39 +15,43 @@ MOLDS = {"HLG": P.psb_d_hip_hlg_sparse_mat, "HLG32": lambda: P.psb_d_hip_hlg_spa
          "ELG": P.psb_d_hip_elg_sparse_mat}
 
 
-def _system(n, mold, spd):
-    """Diagonally dominant: a tridiagonal part and, in every row but the first
-    rows, far entries that reach other blocks (nine of them in some rows, so
-    that a row has more than one group of slots)."""
+def _system(n, mold, spd, wide):
+    """Diagonally dominant: a tridiagonal part, entries that reach other blocks
+    (a third of the matrix away; 9973 rows away in the largest, whose columns
+    are to fit in 16 bits), and two rows of 5 + wide slots."""
     if n == 1:
         return P.matrix_from_coo(1, 1, np.array([1], np.int32), np.array([1], np.int32),
                                  np.array([2.0]), mold=mold)
     i = np.arange(n, dtype=np.int32)
     rows, cols, vals = [i], [i], [6.0 + 0.1 * (i % 7)]
-    for o, w in ((1, 1.0), (max(2, n // 3), 0.5)):
+    for o, w in ((1, 1.0), (max(2, n // 3 if n <= 524288 else 9973), 0.5)):
         if o < n:
             rows += [i[o:], i[:-o]]
             cols += [i[:-o], i[o:]]
             vals += [np.full(n - o, -w), np.full(n - o, -w if spd else -0.6 * w)]
-    if n > 64:
-        c = np.arange(7, dtype=np.int32) * 7 + 3
-        r = np.array([n - 1, n // 2 + 3], np.int32)
-        R, C = (a.ravel() for a in np.meshgrid(r, c, indexing="ij"))
-        rows += [R, C]
-        cols += [C, R]
-        vals += [np.full(R.size, -0.1), np.full(R.size, -0.1)]
+    if n > 256:
+        r = np.array([n - 1, n // 2 + 3], np.int32).repeat(wide)
+        c = r - 7 * np.tile(np.arange(1, wide + 1, dtype=np.int32), 2)
+        rows += [r, c]
+        cols += [c, r]
+        vals += [np.full(r.size, -0.1), np.full(r.size, -0.1)]
     ia, ja, v = (np.concatenate(a) for a in (rows, cols, vals))
     return P.matrix_from_coo(n, n, ia.astype(np.int32) + 1, ja.astype(np.int32) + 1, v, mold=mold)
 
 
-@pytest.mark.parametrize("fmt,n", [("HLG", 1), ("HLG", 257), ("ELG", 1000), ("HLG", 65536),
-                                   ("HLG", 65537), ("HLG32", 100001), ("ELG", 262144),
-                                   ("HLG", 262145), ("HLG", 524289), ("ELG", 1048576),
-                                   ("HLG", 1048577)])
+# wide: rows of more slots than the registers hold where a thread has one row,
+# of seven and of eight where it has several
+@pytest.mark.parametrize("fmt,n,wide", [("HLG", 1, 0), ("HLG", 257, 4), ("ELG", 1000, 12),
+                                        ("HLG", 65536, 12), ("HLG", 65537, 20),
+                                        ("HLG32", 100001, 3), ("ELG", 262144, 4),
+                                        ("HLG", 262145, 2), ("ELG", 300000, 3),
+                                        ("HLG", 524288, 3), ("HLG", 524289, 2),
+                                        ("ELG", 700001, 3), ("HLG", 1048576, 2),
+                                        ("HLG", 1048577, 2)])
 @pytest.mark.parametrize("method", ["CG", "BICGSTAB"])
-def test_resident_follows_reference_sequence(gpu, orc, fmt, n, method):
-    print(f"[gpu] case resident {fmt} n={n} {method}", flush=True)
-    a = _system(n, MOLDS[fmt](), method == "CG")
+def test_resident_follows_reference_sequence(gpu, orc, fmt, n, wide, method):
+    print(f"[gpu] case resident {fmt} n={n} wide={wide} {method}", flush=True)
+    a = _system(n, MOLDS[fmt](), method == "CG", wide)
     desc = P.psb_cdall(nl=n)
     for ptype in ("DIAG", "NONE"):
         prec = P.psb_dprec_type(ptype).build(a, desc)
