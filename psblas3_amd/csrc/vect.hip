@@ -190,10 +190,11 @@ __global__ __launch_bounds__(kBlock) void k_abs(int n, T alpha, const T* x, T* y
 // Reductions.  op: 0 dot, 1 sum of squares, 2 max |x|, 3 sum |x|, 4 scaled
 // sum of squares (x/scale)^2 with scale read from device memory.  Accumulated
 // in FP64.  VEC: 16-byte loads, four vectors per input in flight and four
-// sums per thread (both inputs 16-byte aligned); else entry by entry.  Against
-// entry by entry with one sum, a fence and one arrival counter: FP64 dot of
-// 1M entries 16.4 -> 7.3 us, nrm2 14.6 -> 5.6 us, FP32 dot of 3M 27.4 -> 6.8 us;
-// small sizes are bound by the arrivals and the tail over the partials.
+// sums per thread (both inputs 16-byte aligned, over 65536 entries); else a
+// thread's entries in order.  Against entry by entry, a fence and one arrival
+// counter: FP64 dot of 1M entries 16.4 -> 7.3 us, nrm2 14.6 -> 5.6 us, FP32 dot
+// of 3M 27.4 -> 6.8 us.  Small sizes are bound by the arrivals and the tail over
+// the partials.
 template <typename T, int OP>
 __device__ __forceinline__ void red_step(double& acc, T xi, T yi, double inv) {
   const double a = (double)xi;
@@ -212,33 +213,51 @@ __global__ __launch_bounds__(kBlock) void k_reduce(int n, const T* __restrict__ 
                                                    double* result, double* host_result) {
   constexpr int V = VEC ? 16 / (int)sizeof(T) : 1, U = 4;
   const int stride = gridDim.x * kBlock, t0 = blockIdx.x * kBlock + threadIdx.x;
-  const int nv = n / V;
   double acc[U] = {};
   double inv = 1.0;
   if (OP == 4) inv = 1.0 / *scale_p;
-  typedef T vec __attribute__((ext_vector_type(V)));
-  int64_t k = t0;
-  for (; k + (U - 1) * (int64_t)stride < nv; k += U * (int64_t)stride) {
-    vec a[U], b[U];
+  if constexpr (VEC) {
+    const int nv = n / V;
+    typedef T vec __attribute__((ext_vector_type(V)));
+    int64_t k = t0;
+    for (; k + (U - 1) * (int64_t)stride < nv; k += U * (int64_t)stride) {
+      vec a[U], b[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      a[u] = reinterpret_cast<const vec*>(x)[k + u * (int64_t)stride];
-      b[u] = OP == 0 ? reinterpret_cast<const vec*>(y)[k + u * (int64_t)stride] : a[u];
+      for (int u = 0; u < U; u++) {
+        a[u] = reinterpret_cast<const vec*>(x)[k + u * (int64_t)stride];
+        b[u] = OP == 0 ? reinterpret_cast<const vec*>(y)[k + u * (int64_t)stride] : a[u];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int e = 0; e < V; e++) red_step<T, OP>(acc[u], a[u][e], b[u][e], inv);
     }
+    for (; k < nv; k += stride) {
+      const vec a = reinterpret_cast<const vec*>(x)[k];
+      const vec b = OP == 0 ? reinterpret_cast<const vec*>(y)[k] : a;
 #pragma unroll
-    for (int u = 0; u < U; u++)
+      for (int e = 0; e < V; e++) red_step<T, OP>(acc[0], a[e], b[e], inv);
+    }
+    if (blockIdx.x == 0)
+      for (int i = nv * V + threadIdx.x; i < n; i += kBlock)
+        red_step<T, OP>(acc[1], x[i], y[i], inv);
+  } else {
+    // one sum in entry order; eight loads (red_grid's entries a thread) on their
+    // way at a time, the last ones past the end at the last entry
+    constexpr int G = 8;
+    for (int64_t k = t0; k < n; k += G * (int64_t)stride) {
+      T a[G], b[G];
 #pragma unroll
-      for (int e = 0; e < V; e++) red_step<T, OP>(acc[u], a[u][e], b[u][e], inv);
+      for (int u = 0; u < G; u++) {
+        const int64_t i = k + u * (int64_t)stride < n ? k + u * (int64_t)stride : n - 1;
+        a[u] = x[i];
+        b[u] = OP == 0 ? y[i] : a[u];
+      }
+#pragma unroll
+      for (int u = 0; u < G; u++)
+        if (k + u * (int64_t)stride < n) red_step<T, OP>(acc[0], a[u], b[u], inv);
+    }
   }
-  for (; k < nv; k += stride) {
-    const vec a = reinterpret_cast<const vec*>(x)[k];
-    const vec b = OP == 0 ? reinterpret_cast<const vec*>(y)[k] : a;
-#pragma unroll
-    for (int e = 0; e < V; e++) red_step<T, OP>(acc[0], a[e], b[e], inv);
-  }
-  if (V > 1 && blockIdx.x == 0)
-    for (int i = nv * V + threadIdx.x; i < n; i += kBlock)
-      red_step<T, OP>(acc[1], x[i], y[i], inv);
   if (OP == 2)
     grid_reduce<true>(fmax(fmax(acc[0], acc[1]), fmax(acc[2], acc[3])), partials, counter, result,
                       host_result);
@@ -302,7 +321,11 @@ static int launch_reduce(int n, const T* x, const T* y, const double* scale_p, i
   Context& c = ctx();
   int g = red_grid(n);
   reinterpret_cast<volatile unsigned long long*>(c.host_result)[slot] = kUnsetBits;
-  const bool vec = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+  // Up to 65536 entries (32 blocks) the arrivals bound both forms alike (a CG
+  // step's vector operations at 4096 34.2-35.0 us, at 65536 34.8-35.6, either
+  // way), and single loads keep a thread's entries in one sum in order.
+  const bool vec = n > 65536 &&
+      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
   if (vec)
     hipLaunchKernelGGL((k_reduce<T, OP, true>), dim3(g), dim3(kBlock), 0, c.stream, n, x, y,
                        scale_p, c.red_partials, c.red_counter + (size_t)slot * kRedCounter, c.red_result + slot,

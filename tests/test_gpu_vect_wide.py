@@ -18,8 +18,8 @@ def _vec(a):
     return (P.psb_s_hip_vect() if a.dtype == np.float32 else P.psb_d_hip_vect()).bld(a)
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 2047, 2049, 1024 * 2048 - 1, 1024 * 2048 + 3,
-                               3 * 1024 * 2048 + 1])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 2047, 2049, 65536, 65537, 1024 * 2048 - 1,
+                               1024 * 2048 + 3, 3 * 1024 * 2048 + 1])
 @pytest.mark.parametrize("dt", [np.float64, np.float32], ids=["f64", "f32"])
 def test_sizes(gpu, orc, n, dt):
     print(f"[gpu] case vector ops n={n} {np.dtype(dt).name}", flush=True)
