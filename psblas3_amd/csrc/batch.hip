@@ -365,7 +365,8 @@ __global__ __launch_bounds__(kBT) void kb_fin(BTables tb) {
 
 // The finalisation of the systems whose last tile is one of this block's: waits
 // for the partials of the system's other tiles (each is there once it holds
-// something else than kUnsetBits), sets them back, adds them as kb_fin does.
+// something else than kUnsetBits), sets them back (tiles of one system, and of
+// neighbouring ones, share lines: st_unset), adds them as kb_fin does.
 // The wait ends: every block stores its tiles' partials before it waits, and
 // the waiting ones leave room for the others (kFoldSlots).
 template <int OP>
@@ -388,8 +389,8 @@ __device__ __forceinline__ void fold_tiles(const BTables& tb) {
         ua = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         ub = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       } while ((ua == kUnsetBits || ub == kUnsetBits) && ++polls < kFoldPolls);
-      p[0] = kUnsetBits;
-      p[1] = kUnsetBits;
+      st_unset(p);
+      st_unset(p + 1);
       a += __builtin_bit_cast(double, ua);
       b += __builtin_bit_cast(double, ub);
     }

@@ -457,7 +457,7 @@ __device__ __forceinline__ void finish(double (&v)[NP], const Fin& f, KState* st
       for (int k = 0; k < 4; k++)
         if (b + k * kBlock < nb) {
           a[k] += __builtin_bit_cast(double, u[k]);
-          slot[b + k * kBlock] = kUnsetBits;
+          st_unset(slot + b + k * kBlock);
         }
     }
     t[p] = block_sum((a[0] + a[1]) + (a[2] + a[3]), lds);

@@ -215,6 +215,13 @@ __device__ __forceinline__ void st_host(double* p, double v) {
                      __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// A slot that blocks poll, set back to "not there".  At agent scope as every
+// access of such a slot: a plain access leaves its 128-byte line in the XCD's
+// L2, where the polls of the slots beside it would find it unchanged.
+__device__ __forceinline__ void st_unset(unsigned long long* p) {
+  __hip_atomic_store(p, kUnsetBits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Grid reduction by the last block to arrive: every block stores its partial,
 // the last one adds (MAX: takes the maximum of) the partials in index order,
 // stores the result on the device and for the host, and re-arms the counters.

@@ -65,3 +65,30 @@ def test_more_tiles_than_blocks(gpu, orc):
         one = xs[0] if one is None else one
         assert all(np.array_equal(one, x) for x in xs)
         eng.free()
+
+
+@pytest.mark.parametrize("order", [(0, 1), (1, 0), (0, 0, 0, 1, 0, 1)])
+def test_partials_that_share_lines(gpu, orc, order):
+    """Systems of more than 64 tiles (two wavefronts poll) whose partials do not
+    start on a line, beside systems of one tile: eight tiles' partials share a
+    128-byte line, between the wavefronts of one block and between blocks."""
+    print(f"[gpu] case batch fold shared lines {order}", flush=True)
+    big = orc.gen_aniso2d(259, 0.5)       # 66 tiles, the last one of 521 rows
+    systems = _systems(orc)[:1]
+    a = P.matrix_from_coo(big.nr, big.nc, big.ia, big.ja, big.val,
+                          mold=P.psb_d_hip_hlg_sparse_mat(64))
+    systems.append((a, P.psb_dprec_type("DIAG").build(a, P.psb_cdall(nl=big.nr)),
+                    orc.uniform_pm1(7, big.nr)))
+    ref = None
+    for slots in (8, 257):
+        eng = P.psb_hip_batch("CG", max_systems=slots, arena_bytes=64 << 20)
+        ids = [eng.register(a, p) for a, p, _ in systems]
+        jobs = [(ids[k], P.vect_from(systems[k][2]), P.psb_d_hip_vect().all(len(systems[k][2])))
+                for k in order]
+        res = eng.solve(jobs, eps=1e-6, itmax=400)
+        got = [(r["iterations"], r["status"], x.get_vect()) for r, (_, _, x) in zip(res, jobs)]
+        if ref is None:
+            ref = got
+        for (i0, s0, x0), (i1, s1, x1) in zip(ref, got):
+            assert i0 == i1 and s0 == s1 and np.array_equal(x0, x1)
+        eng.free()
