@@ -106,7 +106,7 @@ struct TriLevels {
   uint16_t* tdep = nullptr;     // LDS slot of the entry's dependency
   int2* tstep = nullptr;        // {first row | rows << 16, first entry | width << 16}
   int* thalo = nullptr;         // rows of earlier tiles the tile reads
-  T* sol = nullptr;             // two solution arrays of n entries
+  T* sol = nullptr;             // two solution arrays, sol_stride entries apart
   unsigned long long* ticket = nullptr;
 };
 
@@ -212,6 +212,16 @@ __global__ __launch_bounds__(kBlock) void k_tri_unset(int64_t n, T* __restrict__
     sol[i] = u;
 }
 
+// Entries from one solution array to the other: n rounded up to whole 128-byte
+// lines.  A solve polls one array while it sets the other back with plain
+// stores, and a plain access leaves its line in the XCD's L2, where polls of
+// entries in the same line would find it unchanged.
+template <typename T>
+inline size_t sol_stride(int n) {
+  constexpr size_t line = 128 / sizeof(T);
+  return ((size_t)n + line - 1) / line * line;
+}
+
 // LDS of a tile, in this order (each part 16-byte aligned): solution slots
 // (rows, halo, a zero slot), entry values, diagonals, rows, steps, entry
 // slots.  The host's tile_lds adds up the same parts.
@@ -246,7 +256,7 @@ struct TileStep {
 // form subtracts +0); W == 0: the step's own width.  Rows sum in CSR order.
 template <typename T, int W, bool DIV, bool RUN>
 __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
-    int n, int ntiles, const TriTile* __restrict__ tiles, const int* __restrict__ trow,
+    size_t stride, int ntiles, const TriTile* __restrict__ tiles, const int* __restrict__ trow,
     const T* __restrict__ tdv, const T* __restrict__ tval, const uint16_t* __restrict__ tdep,
     const int2* __restrict__ tstep, const int* __restrict__ thalo, T* sol2,
     unsigned long long* ticket, const T* x, const T* __restrict__ scale, T alpha, T beta, T* y) {
@@ -257,8 +267,8 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
   // a launch draws exactly ntiles tickets, so all of its tickets share one epoch
   const unsigned long long epoch = my / (unsigned)ntiles;
   const TriTile t = tiles[(int)(my - epoch * (unsigned)ntiles)];
-  T* sol = sol2 + (epoch & 1 ? (size_t)n : 0);
-  T* next = sol2 + (epoch & 1 ? 0 : (size_t)n);
+  T* sol = sol2 + (epoch & 1 ? stride : 0);    // no line of one in the other: sol_stride
+  T* next = sol2 + (epoch & 1 ? 0 : stride);
   T* ys = reinterpret_cast<T*>(lds);
   char* at = lds + lds16(sizeof(T) * (size_t)(t.nrow + t.nhalo + 1));
   T* ev = reinterpret_cast<T*>(at);
@@ -746,9 +756,9 @@ static int plan_tiles(TriLevels<V>& T, bool lower, const int* irp, const int* ja
   const unsigned long long zero = 0;
   rc = upload(&T.ticket, &zero, 1);
   if (rc) return rc;
-  PSB_HIP_CHECK(hipMalloc((void**)&T.sol, sizeof(V) * 2 * (size_t)n));
-  hipLaunchKernelGGL((k_tri_unset<V>), dim3(stream_grid(2 * (int64_t)n)), dim3(kBlock), 0, s,
-                     2 * (int64_t)n, T.sol);
+  const int64_t nsol = 2 * (int64_t)sol_stride<V>(n);
+  PSB_HIP_CHECK(hipMalloc((void**)&T.sol, sizeof(V) * (size_t)nsol));
+  hipLaunchKernelGGL((k_tri_unset<V>), dim3(stream_grid(nsol)), dim3(kBlock), 0, s, nsol, T.sol);
   PSB_HIP_LAUNCH_CHECK();
   PSB_HIP_CHECK(hipStreamSynchronize(s));   // the host vectors go out of scope
   T.width = width;
@@ -765,7 +775,7 @@ static int solve_tiles_t(const TriLevels<V>& T, const V* x, const V* scale, V al
                          hipStream_t s) {
 #define PSB_TILE_LAUNCH(W)                                                                    \
   hipLaunchKernelGGL((k_trsv_tiles<V, W, DIV, RUN>), dim3(T.ntiles), dim3(kTileThreads), T.lds, \
-                     s, T.n, T.ntiles, T.tiles, T.trow, T.tdv, T.tval, T.tdep, T.tstep, T.thalo, \
+                     s, sol_stride<V>(T.n), T.ntiles, T.tiles, T.trow, T.tdv, T.tval, T.tdep, T.tstep, T.thalo, \
                      T.sol, T.ticket, x, scale, alpha, beta, y)
   switch (T.width) {
     case 2: PSB_TILE_LAUNCH(2); break;

@@ -99,3 +99,24 @@ def test_tiles_nonfinite(gpu, orc, single):
         ok = ~np.isnan(ref)
         assert np.array_equal(_bits(out[ok]), _bits(ref[ok]))
     a.free()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(9, 9, 9), (25, 24, 1), (17, 15, 9), (41, 41, 5)])
+@pytest.mark.parametrize("single", [False, True], ids=["f64", "f32"])
+def test_tiles_ragged_arrays(gpu, orc, nx, ny, nz, single):
+    """Row counts that do not fill the last line of a solution array, the last
+    tile reading rows beside its own: twenty solves in turn in both arrays."""
+    print(f"[gpu] case trsv tiles ragged {nx}x{ny}x{nz} single={single}", flush=True)
+    n, rows = _grid(nx, ny, nz)
+    dt = np.float32 if single else np.float64
+    assert n * np.dtype(dt).itemsize % 128 != 0
+    for lower in (True, False):
+        irp, ja, val = _csr(n, rows, np.random.default_rng(8), lower)
+        a, desc = _tri_mat(irp, ja, val, lower, False, single=single)
+        x = orc.uniform_pm1(60, n).astype(dt)
+        ref = orc.csr_cssv(irp, ja, val.astype(dt), x, lower=lower)
+        for k in range(20):
+            y = _vec(np.zeros(n, dt), single)
+            P.psb_spsm(1.0, a, _vec(x, single), 0.0, y, desc)
+            assert np.array_equal(_bits(y.get_vect()), _bits(ref)), k
+        a.free()
