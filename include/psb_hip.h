@@ -74,6 +74,14 @@ int psb_hip_get_device_name(char *buf, int len);
 double psb_hip_memory_peak_bandwidth(void);
 /* cudaSync (cuda/cuda_util.h:69): wait for all work on the library stream */
 int psb_hip_device_sync(void);
+/* Kernels whose workgroups wait for one another's values (triangular solves,
+   fused solvers, batch engine) give a wait up after a bounded number of polls,
+   seconds in all.  The kernel then ends with NaN for what did not come, and the
+   next call that brings a result to the host (a vector, buffer or scalar, a
+   solver's state, psb_hip_device_sync) returns PSB_HIP_RUNTIME.  This call sets
+   the polls of every later launch, for tests of that way out; 0 (default): each
+   kernel's own bound.  Returns the previous value. */
+int psb_hip_set_wait_polls(int polls);
 /* psb_cudaGetStream: the library stream as an opaque hipStream_t */
 void *psb_hip_get_stream(void);
 /* Last error text (for the host mirror's error messages). */

@@ -64,6 +64,7 @@ _SIGS = {
     "psb_hip_get_device_name": (i32, [C.c_char_p, i32]),
     "psb_hip_memory_peak_bandwidth": (f64, []),
     "psb_hip_device_sync": (i32, []),
+    "psb_hip_set_wait_polls": (i32, [i32]),
     "psb_hip_get_stream": (vp, []),
     "psb_hip_last_error": (C.c_char_p, []),
     "psb_hip_timer_start": (i32, []),

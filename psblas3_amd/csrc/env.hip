@@ -4,6 +4,7 @@
 // cuda/psb_cuda_env_mod.F90:43-174.
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 
@@ -31,6 +32,20 @@ int set_error(int code, const char* where, const char* what) {
   return code;
 }
 
+static std::atomic<int> g_wait_polls{0};   // psb_hip_set_wait_polls
+
+Waits waits(int polls) {
+  const int set = g_wait_polls.load(std::memory_order_relaxed);
+  return Waits{set > 0 ? set : polls, g_ctx.gave_up};
+}
+
+int check_waits(const char* who) {
+  if (__atomic_exchange_n(g_ctx.gave_up, 0u, __ATOMIC_RELAXED) == 0) return PSB_HIP_SUCCESS;
+  return set_error(PSB_HIP_RUNTIME, who,
+                   "a wait between workgroups of this call or one before it ran out: the results "
+                   "since the last synchronisation are not valid");
+}
+
 static int init_device(int dev) {
   std::lock_guard<std::mutex> lock(g_init_mutex);
   Context& c = g_ctx;
@@ -52,6 +67,8 @@ static int init_device(int dev) {
   PSB_HIP_CHECK(hipMalloc(&c.red_result, sizeof(double) * 64));
   PSB_HIP_CHECK(hipMemset(c.red_counter, 0, sizeof(unsigned int) * 64 * kRedCounter));
   PSB_HIP_CHECK(hipHostMalloc(&c.host_result, sizeof(double) * 64, hipHostMallocCoherent));
+  PSB_HIP_CHECK(hipHostMalloc(&c.gave_up, sizeof(unsigned int), hipHostMallocCoherent));
+  *c.gave_up = 0;
   void* sp = nullptr;
   PSB_HIP_CHECK(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
   c.scratch = (char*)sp;
@@ -166,6 +183,7 @@ int psb_hip_exit(void) {
   hipFree(c.red_counter);
   hipFree(c.red_result);
   hipHostFree(c.host_result);
+  hipHostFree(c.gave_up);
   hipHostFree(c.scratch_host);
   for (hipEvent_t e : c.scratch_ev) hipEventDestroy(e);
   hipEventDestroy(g_ev_start);
@@ -236,7 +254,11 @@ int psb_hip_device_sync(void) {
   int rc = ensure_init();
   if (rc) return rc;
   PSB_HIP_CHECK(hipStreamSynchronize(g_ctx.stream));
-  return PSB_HIP_SUCCESS;
+  return check_waits(__func__);
+}
+
+int psb_hip_set_wait_polls(int polls) {
+  return g_wait_polls.exchange(polls > 0 ? polls : 0, std::memory_order_relaxed);
 }
 
 void* psb_hip_get_stream(void) {
@@ -354,7 +376,7 @@ int psb_hip_read_buffer(void* host, const void* dptr, int64_t nbytes) {
   if (nbytes <= 0) return PSB_HIP_SUCCESS;
   PSB_HIP_CHECK(hipMemcpyAsync(host, dptr, (size_t)nbytes, hipMemcpyDeviceToHost, g_ctx.stream));
   PSB_HIP_CHECK(hipStreamSynchronize(g_ctx.stream));
-  return PSB_HIP_SUCCESS;
+  return check_waits(__func__);
 }
 
 }  // extern "C"

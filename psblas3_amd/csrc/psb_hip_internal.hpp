@@ -42,6 +42,7 @@ struct Context {
   unsigned int* red_counter = nullptr;  // 64 x kRedCounter words, zero between uses
   double* red_result = nullptr;         // 64 result slots
   double* host_result = nullptr;        // pinned and coherent, 64 slots (st_host)
+  unsigned int* gave_up = nullptr;      // pinned and coherent: a wait ran out (Waits)
   // the allocation-free solver's workspace: the device address of the
   // file-scope scratch array on this context's device (looked up at init),
   // a pinned host block for its state read-backs and two events
@@ -61,6 +62,14 @@ int ensure_init();                      // lazily initialises device 0
     int rc_ = ::psbhip::ensure_init(); \
     if (rc_) return rc_;           \
   } while (0)
+
+// ------------------------------------------------------------------ waits between workgroups
+struct Waits;
+// the library stream's waits: polls unless psb_hip_set_wait_polls says otherwise
+Waits waits(int polls);
+// after a synchronisation: PSB_HIP_RUNTIME (once) if a wait of a kernel before
+// it was given up
+int check_waits(const char* who);
 
 // ------------------------------------------------------------------ vectors
 // Device multivector, the counterpart of cuda/vectordev.h:39-52.
@@ -220,6 +229,18 @@ __device__ __forceinline__ void st_host(double* p, double v) {
 // L2, where the polls of the slots beside it would find it unchanged.
 __device__ __forceinline__ void st_unset(unsigned long long* p) {
   __hip_atomic_store(p, kUnsetBits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Every wait of a workgroup for another one's values is bounded: past its polls
+// it is given up, the value counts as NaN, the kernel ends, and this word in
+// pinned coherent host memory says so.  The next call that brings a result to
+// the host fails (check_waits).
+struct Waits {
+  int polls;
+  unsigned int* gave_up;
+};
+__device__ __forceinline__ void give_up(const Waits& w) {
+  __hip_atomic_store(w.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Grid reduction by the last block to arrive: every block stores its partial,

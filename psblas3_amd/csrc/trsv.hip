@@ -76,8 +76,11 @@ constexpr int kTileEntries = 2048;
 constexpr int kTileHalo = 1024;
 constexpr size_t kTileLds = (size_t)64 << 10;
 constexpr int kTileThreads = 256;
-// polls of a halo entry before the wait is given up (the entry then counts
-// as NaN); a poll takes about a microsecond, a real wait far fewer
+// polls of memory by a wavefront before its halo entries are given up (they
+// then count as NaN, and the next call that brings a result to the host fails);
+// a poll takes about a microsecond.  A tile waits for those whose workgroups
+// run beside it: at most 2048 of them, of 512 steps of 0.26 us, one after
+// another, are 0.3 s.
 constexpr int kTilePolls = 1 << 23;
 
 // A tile: its rows at positions row0 .. row0+nrow-1 of the tile-ordered
@@ -259,7 +262,8 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
     size_t stride, int ntiles, const TriTile* __restrict__ tiles, const int* __restrict__ trow,
     const T* __restrict__ tdv, const T* __restrict__ tval, const uint16_t* __restrict__ tdep,
     const int2* __restrict__ tstep, const int* __restrict__ thalo, T* sol2,
-    unsigned long long* ticket, const T* x, const T* __restrict__ scale, T alpha, T beta, T* y) {
+    unsigned long long* ticket, const T* x, const T* __restrict__ scale, T alpha, T beta, T* y,
+    Waits waits) {
   extern __shared__ __align__(16) char lds[];
   __shared__ unsigned long long my;
   if (threadIdx.x == 0) my = atomicAdd(ticket, 1ull);
@@ -312,7 +316,8 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
     bool open = lane < kFirst;
     while (__any(h < t.nhalo)) {
       if (!open) open = !is_unset(ld_lds(ys + t.nrow));
-      if (open && h < t.nhalo) {
+      const bool look = open && h < t.nhalo;
+      if (look) {
         const T v = ld_agent(sol + src);
         if (!is_unset(v)) {
           st_lds(ys + t.nrow + h, v);
@@ -322,7 +327,8 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
       } else {
         __builtin_amdgcn_s_sleep(2);
       }
-      if (++polls > kTilePolls) {
+      if (__any(look) && ++polls > waits.polls) {
+        give_up(waits);
         for (; h < t.nhalo; h += kPollers)
           st_lds(ys + t.nrow + h, __builtin_bit_cast(T, MarkBits<T>::nan));
       }
@@ -776,7 +782,7 @@ static int solve_tiles_t(const TriLevels<V>& T, const V* x, const V* scale, V al
 #define PSB_TILE_LAUNCH(W)                                                                    \
   hipLaunchKernelGGL((k_trsv_tiles<V, W, DIV, RUN>), dim3(T.ntiles), dim3(kTileThreads), T.lds, \
                      s, sol_stride<V>(T.n), T.ntiles, T.tiles, T.trow, T.tdv, T.tval, T.tdep, T.tstep, T.thalo, \
-                     T.sol, T.ticket, x, scale, alpha, beta, y)
+                     T.sol, T.ticket, x, scale, alpha, beta, y, waits(kTilePolls))
   switch (T.width) {
     case 2: PSB_TILE_LAUNCH(2); break;
     case 3: PSB_TILE_LAUNCH(3); break;

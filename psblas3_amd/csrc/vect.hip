@@ -356,7 +356,7 @@ static int fetch_results(int nslots, double* out) {
     }
     out[k] = c.host_result[k];
   }
-  return PSB_HIP_SUCCESS;
+  return check_waits("reduction");
 }
 
 // Slots of one batch of column reductions (host_result and red_result hold 64).
@@ -495,7 +495,7 @@ int psb_hip_mv_read_r2(void* mv, void* host, int ld) {
                                  (size_t)v->size * es, (size_t)v->count, hipMemcpyDeviceToHost,
                                  ctx().stream));
   PSB_HIP_CHECK(hipStreamSynchronize(ctx().stream));
-  return PSB_HIP_SUCCESS;
+  return check_waits(__func__);
 }
 
 int psb_hip_mv_write(void* mv, const void* host) { return psb_hip_mv_write_r2(mv, host, MV(mv)->size); }
@@ -522,7 +522,7 @@ int psb_hip_mv_read_first(void* mv, int first, int n, void* host) {
   PSB_HIP_CHECK(hipMemcpyAsync(host, (char*)v->v + (size_t)(first - 1) * es, (size_t)n * es,
                                hipMemcpyDeviceToHost, ctx().stream));
   PSB_HIP_CHECK(hipStreamSynchronize(ctx().stream));
-  return PSB_HIP_SUCCESS;
+  return check_waits(__func__);
 }
 
 int psb_hip_mv_setscal_d(double val, int first, int last, int index_base, void* x) {
