@@ -80,7 +80,8 @@ int psb_hip_device_sync(void);
    next call that brings a result to the host (a vector, buffer or scalar, a
    solver's state, psb_hip_device_sync) returns PSB_HIP_RUNTIME.  This call sets
    the polls of every later launch, for tests of that way out; 0 (default): each
-   kernel's own bound.  Returns the previous value. */
+   kernel's own bound; negative: every wait is given up at once.  Returns the
+   previous value. */
 int psb_hip_set_wait_polls(int polls);
 /* psb_cudaGetStream: the library stream as an opaque hipStream_t */
 void *psb_hip_get_stream(void);

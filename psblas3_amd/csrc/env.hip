@@ -36,7 +36,7 @@ static std::atomic<int> g_wait_polls{0};   // psb_hip_set_wait_polls
 
 Waits waits(int polls) {
   const int set = g_wait_polls.load(std::memory_order_relaxed);
-  return Waits{set > 0 ? set : polls, g_ctx.gave_up};
+  return Waits{set == 0 ? polls : (set > 0 ? set : 0), g_ctx.gave_up};
 }
 
 int check_waits(const char* who) {
@@ -258,7 +258,7 @@ int psb_hip_device_sync(void) {
 }
 
 int psb_hip_set_wait_polls(int polls) {
-  return g_wait_polls.exchange(polls > 0 ? polls : 0, std::memory_order_relaxed);
+  return g_wait_polls.exchange(polls, std::memory_order_relaxed);
 }
 
 void* psb_hip_get_stream(void) {

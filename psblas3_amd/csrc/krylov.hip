@@ -406,9 +406,11 @@ struct Fin {
   double* partials;
   double* fold;
   double* hist;
+  Waits waits;
 };
 
-// polls of a fold slot before the wait is given up (the sum is then NaN)
+// polls of fold slots before the wait is given up (the sum is then NaN and the
+// solve fails)
 constexpr int kFoldPolls = 1 << 22;
 
 // The end of a fused kernel: every block stores its NP partial sums.  Folded,
@@ -451,7 +453,11 @@ __device__ __forceinline__ void finish(double (&v)[NP], const Fin& f, KState* st
           u[k] = __hip_atomic_load(slot + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           all = all && u[k] != kUnsetBits;
         }
-        if (all || polls > kFoldPolls) break;
+        if (all && f.waits.polls > 0) break;
+        if (polls >= f.waits.polls) {
+          give_up(f.waits);
+          break;
+        }
       }
 #pragma unroll
       for (int k = 0; k < 4; k++)
@@ -721,8 +727,9 @@ __global__ __launch_bounds__(kBlock) void k_bi_x(int n, T* __restrict__ x, T* __
 constexpr int kResGrid = 256;     // blocks: one per CU, and the sums' slots
 constexpr int kResSlots = 8;      // slots of a row in registers
 constexpr int kResIters = 48;     // iterations of a launch (its vectors are loaded and stored once)
-// polls of an entry before the wait is given up (it then counts as NaN and the
-// recurrence breaks down); a poll takes under a microsecond, a real wait tens
+// polls of an entry before the wait is given up (it then counts as NaN, the
+// recurrence breaks down and the solve fails); a poll takes under a microsecond,
+// a real wait tens
 constexpr int kResPolls = 1 << 20;
 
 struct ResCtl {
@@ -742,6 +749,7 @@ struct ResArgs {
   double* hist;
   int iters;
   unsigned int launch;     // 1, 2, ... of the solve
+  Waits waits;
 };
 
 // Whether all blocks of the launch run together (see above).  Every block
@@ -780,9 +788,12 @@ __device__ __forceinline__ bool res_enter(ResCtl* c, unsigned int launch, KState
 // every earlier store of the block (entries and slots set back) arrives before
 // its values do; the sums after a product wait, where those stores are long on
 // their way, and of any two sums in a row at least one does, which is what the
-// slots need.
+// slots need.  lost: set where the wait is given up after most polls; kept to the
+// kernel's end (storing give_up's word here made an iteration of BiCGSTAB at
+// L = 64 18.5 us instead of 17.4).
 template <int NT, int NP, bool WAIT>
-__device__ __forceinline__ void res_sum(double (&v)[NP], double* slots, unsigned int j) {
+__device__ __forceinline__ void res_sum(double (&v)[NP], double* slots, unsigned int j, int most,
+                                        bool& lost) {
   typedef unsigned long long U;
   __shared__ double lds[NP][NT / kWave];
   __shared__ double tot[NP][kResGrid / kWave];
@@ -809,16 +820,19 @@ __device__ __forceinline__ void res_sum(double (&v)[NP], double* slots, unsigned
     double t[NP];
 #pragma unroll
     for (int p = 0; p < NP; p++) t[p] = 0.0;
-    if (threadIdx.x < gridDim.x)
-      for (int polls = 0; polls < kResPolls; polls++) {
-        bool all = true;
+    if (threadIdx.x < gridDim.x) {
+      bool all;
+      int polls = 0;
+      do {
+        all = true;
 #pragma unroll
         for (int p = 0; p < NP; p++) {
           t[p] = ld_agent(reinterpret_cast<const double*>(now) + p * kResGrid + threadIdx.x);
           all = all && !is_unset(t[p]);
         }
-        if (all) break;
-      }
+      } while (!all && ++polls < most);
+      lost = lost || !all || most == 0;
+    }
 #pragma unroll
     for (int p = 0; p < NP; p++) {
       const double w = wave_sum(t[p]);
@@ -887,7 +901,7 @@ __device__ __forceinline__ int res_col(const ResRow<T>& o, int r, int j) {
 // polled in xb.  c[k] for k >= w is some row of the block.
 template <typename T, int W>
 __device__ __forceinline__ T res_group(const int (&c)[W], const T (&v)[W], int w, int r0, int rows,
-                                       const T* xs, const T* xb, T acc) {
+                                       const T* xs, const T* xb, T acc, bool& lost) {
   const char* xr = reinterpret_cast<const char*>(xb + r0);
   // l: opaque, or the compiler keeps every slot's addresses and masks over the
   // iterations and spills them.  Named scalars: an array that the loop below
@@ -916,10 +930,12 @@ __device__ __forceinline__ T res_group(const int (&c)[W], const T (&v)[W], int w
   static_assert(kResSlots == 8, "PSB_RES_8");
   PSB_RES_8(PSB_RES_OUT)
   PSB_RES_8(PSB_RES_OWN)
-  for (int polls = 0; polls < kResPolls; polls++) {
+  int polls = 0;
+  for (; polls < kResPolls; polls++) {
     if (!(false PSB_RES_8(PSB_RES_UNSET))) break;
     PSB_RES_8(PSB_RES_AGAIN)
   }
+  lost = lost || polls == kResPolls;
   PSB_RES_8(PSB_RES_FMA)
 #undef PSB_RES_8
 #undef PSB_RES_OUT
@@ -969,7 +985,7 @@ struct ResRows {
 
   // row k's product with x (res_group)
   __device__ __forceinline__ T dot(const M& m, int k, int r0, int rows, const T* xs,
-                                   const T* xb) const {
+                                   const T* xb, bool& lost) const {
     if constexpr (C16) {
       int cc[W];
 #pragma unroll
@@ -979,9 +995,9 @@ struct ResRows {
         cc[j] = (int)threadIdx.x + bases[k * W + j] + (int)(short)e;
         if (j + 1 < W) cc[j + 1] = (int)threadIdx.x + bases[k * W + j + 1] + (e >> 16);
       }
-      return res_group<T, W>(cc, v[k], w[k], r0, rows, xs, xb, T(0));
+      return res_group<T, W>(cc, v[k], w[k], r0, rows, xs, xb, T(0), lost);
     } else {
-      T acc = res_group<T, W>(c[k], v[k], w[k], r0, rows, xs, xb, T(0));
+      T acc = res_group<T, W>(c[k], v[k], w[k], r0, rows, xs, xb, T(0), lost);
       if constexpr (RPT == 1) {
         if (w[k] > W) {
           const int r = r0 + (int)threadIdx.x;
@@ -995,7 +1011,7 @@ struct ResRows {
               cc[i] = res_col(o, r, jj) - r0;
               vv[i] = o.pv[(size_t)jj * o.stride];
             }
-            acc = res_group<T, W>(cc, vv, o.w - j, r0, rows, xs, xb, acc);
+            acc = res_group<T, W>(cc, vv, o.w - j, r0, rows, xs, xb, acc, lost);
           }
         }
       }
@@ -1027,6 +1043,7 @@ template <typename T, class M, int NT, int RPT, int W, bool C16, int OP>
 __global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
   __shared__ T ps[NT * RPT];
   __shared__ KState S;
+  bool lost = false;   // a wait was given up (res_sum, res_group)
   if (!res_enter(a.ctl, a.launch, a.st)) return;
   const int n = m.nr, r0 = blockIdx.x * (NT * RPT);
   const int rows = min(NT * RPT, n - r0);
@@ -1068,11 +1085,11 @@ __global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
       const int t = k * NT + (int)threadIdx.x;
       q[k] = T(0);
       if (t < rows) {
-        q[k] = mr.dot(m, k, r0, rows, ps, xb);
+        q[k] = mr.dot(m, k, r0, rows, ps, xb, lost);
         s[0] += (double)ps[t] * (double)q[k];
       }
     }
-    res_sum<NT, 1, true>(s, a.slots, j++);
+    res_sum<NT, 1, true>(s, a.slots, j++, a.waits.polls, lost);
     PSB_RES_ROWS {   // every block has its product: the entries go back
       const int t = k * NT + (int)threadIdx.x;
       if (t < rows) st_agent(xb + r0 + t, __builtin_bit_cast(T, MarkBits<T>::unset));
@@ -1093,7 +1110,7 @@ __global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
         w[1] += (double)rk * (double)z;
       }
     }
-    res_sum<NT, 2, false>(w, a.slots, j++);
+    res_sum<NT, 2, false>(w, a.slots, j++, a.waits.polls, lost);
     if (threadIdx.x == 0) fin_apply<OP, 2>(&S, w, hist, nullptr);
     __syncthreads();
   }
@@ -1110,12 +1127,14 @@ __global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
     *a.st = S;
     a.ctl->sums = j;
   }
+  if (lost) give_up(a.waits);
 }
 
 template <typename T, class M, int NT, int RPT, int W>
 __global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
   __shared__ T ps[NT * RPT];
   __shared__ KState S;
+  bool lost = false;   // a wait was given up (res_sum, res_group)
   if (!res_enter(a.ctl, a.launch, a.st)) return;
   const int n = m.nr, r0 = blockIdx.x * (NT * RPT);
   const int rows = min(NT * RPT, n - r0);
@@ -1162,11 +1181,11 @@ __global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
       const int t = k * NT + (int)threadIdx.x;
       v[k] = T(0);
       if (t < rows) {
-        v[k] = mr.dot(m, k, r0, rows, ps, a.xb[0]);
+        v[k] = mr.dot(m, k, r0, rows, ps, a.xb[0], lost);
         c[0] += (double)q[k] * (double)v[k];
       }
     }
-    res_sum<NT, 1, true>(c, a.slots, j++);
+    res_sum<NT, 1, true>(c, a.slots, j++, a.waits.polls, lost);
     PSB_RES_ROWS {
       const int t = k * NT + (int)threadIdx.x;
       if (t < rows) st_agent(a.xb[0] + r0 + t, gone);
@@ -1190,12 +1209,12 @@ __global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
       const int t = k * NT + (int)threadIdx.x;
       t_[k] = T(0);
       if (t < rows) {
-        t_[k] = mr.dot(m, k, r0, rows, ps, a.xb[1]);
+        t_[k] = mr.dot(m, k, r0, rows, ps, a.xb[1], lost);
         w[0] += (double)t_[k] * (double)t_[k];
         w[1] += (double)t_[k] * (double)s[k];
       }
     }
-    res_sum<NT, 2, true>(w, a.slots, j++);
+    res_sum<NT, 2, true>(w, a.slots, j++, a.waits.polls, lost);
     PSB_RES_ROWS {
       const int t = k * NT + (int)threadIdx.x;
       if (t < rows) st_agent(a.xb[1] + r0 + t, gone);
@@ -1213,7 +1232,7 @@ __global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
         w[1] += (double)q[k] * (double)r[k];
       }
     }
-    res_sum<NT, 2, false>(w, a.slots, j++);
+    res_sum<NT, 2, false>(w, a.slots, j++, a.waits.polls, lost);
     if (threadIdx.x == 0) fin_apply<FIN_BI_X, 2>(&S, w, hist, nullptr);
     __syncthreads();
   }
@@ -1230,6 +1249,7 @@ __global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
     *a.st = S;
     a.ctl->sums = j;
   }
+  if (lost) give_up(a.waits);
 }
 #undef PSB_RES_ROWS
 #undef PSB_RES_VEC
@@ -1466,7 +1486,7 @@ static Mats<T> make_views(Solver& s) {
 // its own stores first) L = 100 took 16.4 ms.
 static bool folds(const Solver& s, int nb) { return s.fold && nb <= kFoldGrid; }
 static Fin fin_args(const Solver& s, int nb) {
-  return Fin{s.partials, folds(s, nb) ? s.fold : nullptr, s.hist};
+  return Fin{s.partials, folds(s, nb) ? s.fold : nullptr, s.hist, waits(kFoldPolls)};
 }
 // One-block finalisation after a fused kernel launched on nb blocks.
 template <int OP, int NP>
@@ -1652,13 +1672,14 @@ static int resident_setup(Solver& s, ResArgs<T>* a) {
   a->xb[0] = (T*)s.rx[0];
   a->xb[1] = (T*)s.rx[1];
   a->hist = s.hist;
+  a->waits = waits(kResPolls);
   return PSB_HIP_SUCCESS;
 }
 
 static int read_state(Solver& s) {
   PSB_HIP_CHECK(hipMemcpyAsync(s.hst, s.st, sizeof(KState), hipMemcpyDeviceToHost, s.stream));
   PSB_HIP_CHECK(hipStreamSynchronize(s.stream));
-  return PSB_HIP_SUCCESS;
+  return check_waits("krylov");
 }
 
 // Pipelined poll.  After queueing a batch of iterations the host queues a

@@ -1,5 +1,5 @@
 """Kernels whose workgroups wait for one another's values: when a wait is given
-up (forced by a bound of one poll) the kernel ends, the next call that brings a
+up (forced from the host: no polls at all) the kernel ends, the next call that brings a
 result to the host fails instead of handing out NaN, and with the usual bound
 the same objects work again."""
 import numpy as np
@@ -13,10 +13,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture
-def one_poll(gpu):
-    """Call it to bound every wait by one poll until the test ends; call it with 0
-    for the usual bounds."""
-    yield lambda polls=1: N.fn("psb_hip_set_wait_polls")(polls)
+def no_polls(gpu):
+    """Call it to have every wait given up until the test ends; call it with 0 for
+    the usual bounds."""
+    yield lambda polls=-1: N.fn("psb_hip_set_wait_polls")(polls)
     N.fn("psb_hip_set_wait_polls")(0)
 
 
@@ -26,7 +26,7 @@ def _fails(f):
     assert e.value.info == N.RUNTIME and "wait" in str(e.value)
 
 
-def test_triangular_solve(gpu, orc, one_poll):
+def test_triangular_solve(gpu, orc, no_polls):
     """A chain of 6,000 rows: eleven of its twelve tiles wait for the one before."""
     print("[gpu] case waits triangular solve", flush=True)
     n = 6000
@@ -45,9 +45,75 @@ def test_triangular_solve(gpu, orc, one_poll):
     for result in (y.get_vect, lambda: P.psb_genrm2(y), lambda: N.call("psb_hip_device_sync")):
         solve()
         assert np.array_equal(_bits(y.get_vect()), _bits(ref))
-        one_poll()
+        no_polls()
         solve()
-        one_poll(0)
+        no_polls(0)
         _fails(result)
         N.call("psb_hip_device_sync")      # said once
+    a.free()
+
+
+def _poisson(L, mold):
+    n = L ** 3
+    g = np.arange(n, dtype=np.int32).reshape(L, L, L)
+    ia, ja, val = [g.ravel()], [g.ravel()], [np.full(n, 6.0)]
+    for ax in range(3):
+        lo, hi = np.moveaxis(g, ax, 0)[:-1].ravel(), np.moveaxis(g, ax, 0)[1:].ravel()
+        ia += [lo, hi]
+        ja += [hi, lo]
+        val += [np.full(2 * lo.size, -1.0)]
+    return P.matrix_from_coo(n, n, np.concatenate(ia) + 1, np.concatenate(ja) + 1,
+                             np.concatenate(val), mold=mold)
+
+
+# iterations of one launch (HLG) and finalisations folded into launches per
+# step (CSR, and rows beyond what the chip holds)
+@pytest.mark.parametrize("fmt,L", [("HLG", 30), ("HLG", 64), ("CSRG", 64), ("HLG", 110)])
+@pytest.mark.parametrize("method", ["CG", "BICGSTAB"])
+def test_fused_solve(gpu, orc, no_polls, fmt, L, method):
+    print(f"[gpu] case waits fused {fmt} L={L} {method}", flush=True)
+    mold = P.psb_d_hip_hlg_sparse_mat(64) if fmt == "HLG" else P.psb_d_hip_csrg_sparse_mat()
+    a = _poisson(L, mold)
+    n = L ** 3
+    desc = P.psb_cdall(nl=n)
+    prec = P.psb_dprec_type("DIAG").build(a, desc)
+    b = P.vect_from(orc.uniform_pm1(2, n))
+    noalloc = n * 8 * 10 < 64 << 20
+
+    def solve(**kw):
+        x = P.psb_geall(desc)
+        it, err, _ = P.psb_krylov_fused(method, a, prec, b, x, 1e-8, desc, itmax=400, **kw)
+        assert err <= 1e-8
+        return it, x.get_vect()
+
+    it, x = solve()
+    no_polls()
+    _fails(solve)
+    if noalloc:
+        _fails(lambda: solve(noalloc=True))
+    no_polls(0)
+    again = [solve()] + ([solve(noalloc=True)] if noalloc else [])
+    assert all(i == it and np.array_equal(_bits(y), _bits(x)) for i, y in again)
+    a.free()
+
+
+@pytest.mark.parametrize("variant", ["restart", "reliable"])
+def test_mixed_solve(gpu, orc, no_polls, variant):
+    print(f"[gpu] case waits mixed {variant}", flush=True)
+    a = _poisson(40, P.psb_d_hip_hlg_sparse_mat(64))
+    n = 40 ** 3
+    desc = P.psb_cdall(nl=n)
+    prec = P.psb_dprec_type("DIAG").build(a, desc)
+    b = P.vect_from(orc.uniform_pm1(3, n))
+
+    def solve():
+        x = P.psb_geall(desc)
+        out = P.psb_krylov_mixed("CG", a, prec, b, x, 1e-10, desc, variant=variant)
+        return out, x.get_vect()
+
+    _, x = solve()
+    no_polls()
+    _fails(solve)
+    no_polls(0)
+    assert np.array_equal(_bits(solve()[1]), _bits(x))
     a.free()
