@@ -78,8 +78,9 @@ int psb_hip_device_sync(void);
    fused solvers, batch engine) give a wait up after a bounded number of polls,
    seconds in all.  The kernel then ends with NaN for what did not come, and the
    next call that brings a result to the host (a vector, buffer or scalar, a
-   solver's state, psb_hip_device_sync) returns PSB_HIP_RUNTIME.  This call sets
-   the polls of every later launch, for tests of that way out; 0 (default): each
+   solver's state, psb_hip_device_sync) returns PSB_HIP_RUNTIME; a batch engine's
+   step and poll do from then on.  This call sets the polls of every later launch
+   (a batch engine's from its first step on), for tests of that way out; 0 (default): each
    kernel's own bound; negative: every wait is given up at once.  Returns the
    previous value. */
 int psb_hip_set_wait_polls(int polls);

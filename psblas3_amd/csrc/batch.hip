@@ -93,7 +93,9 @@ constexpr int kSlotMask = kLastTile - 1;
 // their own tiles, so the other blocks always find a place: the chip holds at
 // least two of these blocks on each of its 256 CUs.
 constexpr int kFoldSlots = 256;
-// polls of a partial before the wait is given up (the sum is then NaN)
+// polls of a partial before the wait is given up (the sum is then NaN and the
+// engine has failed: a partial that comes late would be taken for the next
+// kernel's)
 constexpr int kFoldPolls = 1 << 22;
 
 struct BTables {
@@ -105,6 +107,7 @@ struct BTables {
   double* partials;                // two per tile; with fold kUnsetBits between uses
   int tcap;                        // tile table entries (>= kBGrid)
   int fold;                        // finalise in the tile kernels (no kb_fin launches)
+  Waits waits;
 };
 
 __device__ __forceinline__ bool b_iterating(const BState* s) {
@@ -385,10 +388,13 @@ __device__ __forceinline__ void fold_tiles(const BTables& tb) {
       U* p = reinterpret_cast<U*>(tb.partials) + 2 * (size_t)(rg.x + k);
       U ua, ub;
       int polls = 0;
+      bool all;
       do {
         ua = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         ub = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      } while ((ua == kUnsetBits || ub == kUnsetBits) && ++polls < kFoldPolls);
+        all = ua != kUnsetBits && ub != kUnsetBits;
+      } while (!all && ++polls < tb.waits.polls);
+      if (!all || tb.waits.polls == 0) give_up(tb.waits);
       st_unset(p);
       st_unset(p + 1);
       a += __builtin_bit_cast(double, ua);
@@ -820,6 +826,8 @@ struct Batch {
   BSys* sys = nullptr;
   BState* st = nullptr;
   double* partials = nullptr;
+  unsigned int* gave_up = nullptr;            // pinned and coherent: a wait ran out (Waits)
+  bool failed = false;                        // ... and was reported
   // host
   std::vector<BMat> mats;
   std::vector<BSlot> slots;
@@ -845,6 +853,7 @@ static BTables tables(const Batch& B) {
   t.partials = B.partials;
   t.tcap = B.tmax;
   t.fold = B.fold ? 1 : 0;
+  t.waits = Waits{waits(kFoldPolls).polls, B.gave_up};
   return t;
 }
 
@@ -971,6 +980,15 @@ static int upload(Batch& B) {
   return PSB_HIP_SUCCESS;
 }
 
+// PSB_HIP_RUNTIME once a wait of the engine's kernels was given up: its systems'
+// scalars and partials are not to be relied on from then on.
+static int check_engine(Batch& B, const char* who) {
+  if (__atomic_load_n(B.gave_up, __ATOMIC_RELAXED) != 0) B.failed = true;
+  if (!B.failed) return PSB_HIP_SUCCESS;
+  return set_error(PSB_HIP_RUNTIME, who,
+                   "a wait between workgroups ran out: free this engine and create another one");
+}
+
 static void destroy(Batch* B) {
   if (!B) return;
   if (B->stream) (void)hipStreamSynchronize(B->stream);
@@ -987,6 +1005,7 @@ static void destroy(Batch* B) {
       if (p) (void)hipHostFree(p);
     if (S.ev) (void)hipEventDestroy(S.ev);
   }
+  if (B->gave_up) (void)hipHostFree(B->gave_up);
   for (int k = 0; k < 2; k++) {
     if (B->ring[k]) (void)hipHostFree(B->ring[k]);
     if (B->ring_ev[k]) (void)hipEventDestroy(B->ring_ev[k]);
@@ -1050,6 +1069,9 @@ int psb_hip_batch_create(void** batch, int method, int max_systems, int64_t aren
     hm((void**)&S.states, sizeof(BState) * max_systems);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&S.ev, hipEventDisableTiming);
   }
+  if (e == hipSuccess)
+    e = hipHostMalloc((void**)&B->gave_up, sizeof(unsigned int), hipHostMallocCoherent);
+  if (e == hipSuccess) *B->gave_up = 0;
   for (int k = 0; k < 2; k++) {
     if (e == hipSuccess)
       e = hipHostMalloc((void**)&B->ring[k], sizeof(BState) * max_systems, hipHostMallocDefault);
@@ -1222,7 +1244,8 @@ int psb_hip_batch_can_admit(void* batch, int mat_id) {
 int psb_hip_batch_step(void* batch) {
   Batch* B = (Batch*)batch;
   if (!B) return PSB_HIP_INVALID;
-  int rc = upload(*B);
+  int rc = check_engine(*B, __func__);
+  if (!rc) rc = upload(*B);
   if (rc) return rc;
   if (B->use_graph) {
     if (!B->exec) {
@@ -1258,6 +1281,8 @@ int psb_hip_batch_poll(void* batch, int wait_last, int max_out, int* ids, int* i
   const long sidx = (wait_last || B->steps < 2) ? B->steps - 1 : B->steps - 2;
   const int k = (int)(sidx & 1);
   PSB_HIP_CHECK(hipEventSynchronize(B->ring_ev[k]));
+  const int rc = check_engine(*B, __func__);
+  if (rc) return rc;
   const BState* S = B->ring[k];
   for (int s = 0; s < B->nslots && *nout < max_out; s++) {
     BSlot& sl = B->slots[s];

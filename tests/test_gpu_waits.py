@@ -117,3 +117,34 @@ def test_mixed_solve(gpu, orc, no_polls, variant):
     no_polls(0)
     assert np.array_equal(_bits(solve()[1]), _bits(x))
     a.free()
+
+
+@pytest.mark.parametrize("method,refine", [("CG", "reliable"), ("BICGSTAB", "restart"),
+                                           ("BICGSTAB", "reliable")])
+@pytest.mark.parametrize("graph", [True, False])
+def test_batch_engine(gpu, orc, no_polls, method, refine, graph):
+    """An engine one of whose waits was given up stays failed; another one works."""
+    print(f"[gpu] case waits batch {method} {refine} graph={graph}", flush=True)
+    coo = orc.gen_aniso2d(70, 0.5)        # 5 tiles
+    a = P.matrix_from_coo(coo.nr, coo.nc, coo.ia, coo.ja, coo.val,
+                          mold=P.psb_d_hip_hlg_sparse_mat(64))
+    prec = P.psb_dprec_type("DIAG").build(a, P.psb_cdall(nl=coo.nr))
+    b = P.vect_from(orc.uniform_pm1(4, coo.nr))
+
+    def engine():
+        eng = P.psb_hip_batch(method, max_systems=4, arena_bytes=16 << 20, refine=refine,
+                              use_graph=graph)
+        return eng, eng.register(a, prec)
+
+    no_polls()
+    eng, mid = engine()
+    _fails(lambda: eng.solve([(mid, b, P.psb_d_hip_vect().all(coo.nr))], eps=1e-6, itmax=500))
+    no_polls(0)
+    _fails(eng.step)
+    _fails(eng.poll)
+    eng.free()
+    N.call("psb_hip_device_sync")          # the engine's failure is its own
+    eng, mid = engine()
+    res = eng.solve([(mid, b, P.psb_d_hip_vect().all(coo.nr))], eps=1e-6, itmax=500)
+    assert res[0]["status"] == 1
+    eng.free()
