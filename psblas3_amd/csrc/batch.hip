@@ -7,8 +7,9 @@
 // tiles; the tile table lists (slot, first row) system after system.  Every
 // streaming kernel walks the tile table grid-stride and skips the tiles of
 // systems that are not in the phase it serves; every reduction stores one
-// partial per tile, and the block of a system's last tile waits for the
-// others', adds them in tile order and updates the system's scalars.  A
+// partial per tile, and the highest block that has one of a system's tiles
+// waits for the others', adds them in tile order and updates the system's
+// scalars.  A
 // system's arithmetic therefore does not depend on which other systems share
 // the launch: its results are the same alone and in any mix.
 //
@@ -84,14 +85,23 @@ struct BSys {
   float *v, *f, *s, *t;         // BiCGSTAB only
 };
 
-// Bits of a tile entry's slot word: the slot, and whether the tile is its
-// system's last.
-constexpr int kLastTile = 1 << 30;
-constexpr int kSlotMask = kLastTile - 1;
-// Slots up to which the tile kernels finalise by themselves (BTables::fold).
-// The blocks that wait for partials are at most one per system, and only after
-// their own tiles, so the other blocks always find a place: the chip holds at
-// least two of these blocks on each of its 256 CUs.
+// Bits of a tile entry's slot word: the slot, and whether the tile's block
+// finalises the system (fin_tile).
+constexpr int kFinTile = 1 << 30;
+constexpr int kSlotMask = kFinTile - 1;
+// Which of a system's tiles first .. last that is: the one of its highest block
+// (tile t is block t % kBGrid's).  So a block waits, after its own tiles, only
+// for blocks of lower index, and the wait ends however few blocks the chip or
+// an XCD holds at once: an XCD starts its blocks in ascending order, so the
+// lowest block that has not ended either runs, and nothing it waits for has
+// yet to end, or has a place next.  (The kernels of all engines are on one
+// stream.)
+static int fin_tile(int first, int last) {
+  const int turn = last / kBGrid;
+  return first / kBGrid == turn ? last : turn * kBGrid - 1;
+}
+// Slots up to which the tile kernels finalise by themselves (BTables::fold): a
+// waiting block holds its place, and there is one for every system.
 constexpr int kFoldSlots = 256;
 // polls of a partial before the wait is given up (the sum is then NaN and the
 // engine has failed: a partial that comes late would be taken for the next
@@ -99,7 +109,7 @@ constexpr int kFoldSlots = 256;
 constexpr int kFoldPolls = 1 << 22;
 
 struct BTables {
-  const int2* __restrict__ tiles;  // (slot | kLastTile, first row)
+  const int2* __restrict__ tiles;  // (slot | kFinTile, first row)
   const int* ntiles;               // device scalar
   const int2* __restrict__ range;  // per slot: first tile, tile count
   const BSys* __restrict__ sys;
@@ -169,7 +179,7 @@ __device__ __forceinline__ T b_row(const BSys& sy, const T* a, int r, const T* _
 
 // The same for kernels whose body leaves the tile's two sums in a_ and b_:
 // they become the tile's partials, and after its tiles a block that had some
-// system's last one finalises it.
+// system's finalising one (fin_tile) finalises it.
 #define PSB_BATCH_SUMS(TB, OP, COND, ...)                                \
   {                                                                      \
     int last_ = 0;                                                       \
@@ -177,7 +187,7 @@ __device__ __forceinline__ T b_row(const BSys& sy, const T* a, int r, const T* _
       double a_ = 0.0, b_ = 0.0;                                         \
       __VA_ARGS__                                                        \
       tile_partials(a_, b_, TB, t_);                                     \
-      last_ |= tl_.x & kLastTile;                                        \
+      last_ |= tl_.x & kFinTile;                                        \
     })                                                                   \
     if ((TB).fold && last_) fold_tiles<OP>(TB);                          \
   }
@@ -366,12 +376,12 @@ __global__ __launch_bounds__(kBT) void kb_fin(BTables tb) {
   if (threadIdx.x == 0) fin_apply<OP>(st, a, b);
 }
 
-// The finalisation of the systems whose last tile is one of this block's: waits
+// The finalisation of the systems whose fin_tile is one of this block's: waits
 // for the partials of the system's other tiles (each is there once it holds
 // something else than kUnsetBits), sets them back (tiles of one system, and of
 // neighbouring ones, share lines: st_unset), adds them as kb_fin does.
 // The wait ends: every block stores its tiles' partials before it waits, and
-// the waiting ones leave room for the others (kFoldSlots).
+// waits for lower blocks only (fin_tile).
 template <int OP>
 __device__ __forceinline__ void fold_tiles(const BTables& tb) {
   typedef unsigned long long U;
@@ -379,7 +389,7 @@ __device__ __forceinline__ void fold_tiles(const BTables& tb) {
   const int nt = *tb.ntiles;
   for (int t = blockIdx.x; t < nt; t += gridDim.x) {
     const int2 tl = tb.tiles[t];
-    if (!(tl.x & kLastTile)) continue;
+    if (!(tl.x & kFinTile)) continue;
     BState* st = tb.st + (tl.x & kSlotMask);
     if (fin_transiting(OP) ? !b_transiting(st) : !b_iterating(st)) continue;
     const int2 rg = tb.range[tl.x & kSlotMask];
@@ -953,7 +963,8 @@ static int upload(Batch& B) {
       const int nk = sl.live ? (B.sys_h[k].n + kTileRows - 1) / kTileRows : 0;
       if (nt + nk > B.tmax) return set_error(PSB_HIP_RUNTIME, "batch", "tile table overflow");
       S.range[k] = make_int2(nt, nk);
-      for (int j = 0; j < nk; j++) S.tiles[nt + j] = make_int2(k | (j == nk - 1 ? kLastTile : 0), j * kTileRows);
+      for (int j = 0; j < nk; j++) S.tiles[nt + j] = make_int2(k, j * kTileRows);
+      if (nk > 0) S.tiles[fin_tile(nt, nt + nk - 1)].x |= kFinTile;
       nt += nk;
     }
     *S.ntiles = nt;

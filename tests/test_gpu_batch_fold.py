@@ -47,9 +47,10 @@ def test_slots_do_not_change_the_bits(gpu, orc, method, refine):
 
 
 def test_more_tiles_than_blocks(gpu, orc):
-    """2,100 tiles on 2,048 blocks: some blocks have two tiles, one of them their
-    system's last."""
-    print("[gpu] case batch fold 2100 tiles", flush=True)
+    """2,112 tiles on 2,048 blocks: some blocks have two tiles, and the last
+    system's are those of the highest blocks and the lowest, finalised by the
+    highest."""
+    print("[gpu] case batch fold 2112 tiles", flush=True)
     coo = orc.gen_aniso2d(600, 0.5)       # 352 tiles a system
     a = P.matrix_from_coo(coo.nr, coo.nc, coo.ia, coo.ja, coo.val,
                           mold=P.psb_d_hip_hlg_sparse_mat(64))
@@ -86,6 +87,33 @@ def test_partials_that_share_lines(gpu, orc, order):
         jobs = [(ids[k], P.vect_from(systems[k][2]), P.psb_d_hip_vect().all(len(systems[k][2])))
                 for k in order]
         res = eng.solve(jobs, eps=1e-6, itmax=400)
+        got = [(r["iterations"], r["status"], x.get_vect()) for r, (_, _, x) in zip(res, jobs)]
+        if ref is None:
+            ref = got
+        for (i0, s0, x0), (i1, s1, x1) in zip(ref, got):
+            assert i0 == i1 and s0 == s1 and np.array_equal(x0, x1)
+        eng.free()
+
+
+def test_systems_round_the_grid(gpu, orc):
+    """Systems of more tiles than the 2,048 blocks and systems that begin in the
+    highest blocks and end in the lowest, up to the third turn: finalised by the
+    same sums in tile order as with a launch of its own."""
+    print("[gpu] case batch fold systems round the grid", flush=True)
+    big, mid = orc.gen_aniso2d(1500, 0.5), orc.gen_aniso2d(600, 0.5)   # 2198 and 352 tiles
+    mats = []
+    for k, coo in enumerate((mid, big)):
+        a = P.matrix_from_coo(coo.nr, coo.nc, coo.ia, coo.ja, coo.val,
+                              mold=P.psb_d_hip_hlg_sparse_mat(64))
+        mats.append((a, P.psb_dprec_type("DIAG").build(a, P.psb_cdall(nl=coo.nr)),
+                     orc.uniform_pm1(8 + k, coo.nr)))
+    ref = None
+    for slots in (12, 257):
+        eng = P.psb_hip_batch("CG", max_systems=slots, arena_bytes=600 << 20)
+        ids = [eng.register(a, p) for a, p, _ in mats]
+        jobs = [(ids[k], P.vect_from(mats[k][2]), P.psb_d_hip_vect().all(len(mats[k][2])))
+                for k in (0, 0, 0, 0, 0, 0, 1, 0, 0, 0)]
+        res = eng.solve(jobs, eps=1e-2, itmax=60)
         got = [(r["iterations"], r["status"], x.get_vect()) for r, (_, _, x) in zip(res, jobs)]
         if ref is None:
             ref = got
