@@ -212,17 +212,17 @@ __device__ __forceinline__ T block_max(T v, T* lds) {
   return r;
 }
 
-// A result the host waits for: the kernel stores it in pinned coherent memory
-// and the host, which set the slot to this NaN pattern before the launch,
-// reads it as soon as it changes.  A computed NaN with these bits is stored as
-// the default NaN.
-constexpr unsigned long long kUnsetBits = 0x7ff8d1e5a2c4b693ull;
+// A result for the host, in pinned coherent memory: no copy back.
 __device__ __forceinline__ void st_host(double* p, double v) {
-  unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  if (u == kUnsetBits) u = 0x7ff8000000000000ull;
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), u, __ATOMIC_RELAXED,
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p),
+                     __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_SYSTEM);
 }
+
+// What a slot that blocks poll for a sum holds until the sum is there: a quiet
+// NaN with a payload of its own.  A computed NaN with these bits is stored as
+// the default NaN.
+constexpr unsigned long long kUnsetBits = 0x7ff8d1e5a2c4b693ull;
 
 // A slot that blocks poll, set back to "not there".  At agent scope as every
 // access of such a slot: a plain access leaves its 128-byte line in the XCD's

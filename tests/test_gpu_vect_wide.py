@@ -1,6 +1,7 @@
 """Vector operations by 16-byte loads at the sizes where they can go wrong:
 remainders of a vector and of a thread's share, one grid-stride turn more or
-less, more columns than one batch of results, infinities and NaN."""
+less, more columns than one batch of results, infinities and NaN; a reduction
+leaves the library stream idle."""
 import ctypes as C
 import math
 
@@ -71,3 +72,19 @@ def test_nonfinite_and_empty(gpu):
     res = (C.c_double * 1)(7.0)
     N.call("psb_hip_mv_dot", res, 0, xv.dev, ones.dev)
     assert res[0] == 0.0
+
+
+@pytest.mark.parametrize("n,cols", [(1, 1), (1001, 33), (4000003, 1)])
+def test_reductions_synchronise(gpu, orc, n, cols):
+    """A call that returns a host scalar synchronises the library stream
+    (include/psb_hip.h): nothing is left on it, for any of the reductions."""
+    print(f"[gpu] case reductions synchronise n={n} cols={cols}", flush=True)
+    hip = C.CDLL("libamdhip64.so")
+    stream = C.c_void_p(N.fn("psb_hip_get_stream")())
+    v = _vec(np.full((n, cols) if cols > 1 else n, 0.5))
+    P.psb_geaxpby(1.0, v, 0.0, v)
+    res = (C.c_double * cols)()
+    for name in ("psb_hip_mv_dot", "psb_hip_mv_nrm2", "psb_hip_mv_amax", "psb_hip_mv_asum"):
+        for _ in range(20):
+            N.call(name, res, n, v.dev, *([v.dev] if name == "psb_hip_mv_dot" else []))
+            assert hip.hipStreamQuery(stream) == 0, name
