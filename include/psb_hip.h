@@ -590,6 +590,13 @@ int psb_hip_krylov_fused_noalloc(int method, int fmt, void *dmat, void *diag, vo
                                  double eps, int itmax, int istop, int check_every, int *iter,
                                  double *err, double *hist);
 
+/* Fused solves of up to 1,048,576 rows run many iterations in one launch, whose
+   workgroups hold the whole chip.  Where they do not all come to run within a
+   millisecond (the chip is shared) the solve goes on with launches per step, as
+   do the solves of the next second.  For tests: launch > 0 has every solve
+   leave at that one of its launches, 0 (default) none; the call also forgets
+   that the chip was busy, and returns how many solves left since the last call. */
+int psb_hip_set_resident_leave(int launch);
 /* FP32-inner / FP64-outer iterative refinement on a double HLL matrix with a
    single copy (psb_hip_hll_make_single).  FP64: r = b - A x, x += d and the
    convergence norms; FP32: the matrix values, the inner Krylov vectors and

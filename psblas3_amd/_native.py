@@ -177,6 +177,7 @@ _SIGS = {
     "psb_hip_krylov_fused": (i32, [i32, i32, vp, vp, vp, vp, f64, i32, i32, i32, pi32, pf64, vp]),
     "psb_hip_krylov_fused_noalloc": (i32, [i32, i32, vp, vp, vp, vp, f64, i32, i32, i32, pi32, pf64,
                                            vp]),
+    "psb_hip_set_resident_leave": (i32, [i32]),
     "psb_hip_krylov_mixed": (i32, [i32, vp, vp, vp, vp, f64, i32, f64, i32, i32, i32, pi32,
                                    pi32, pf64]),
     "psb_hip_mm_read_coo": (i32, [C.c_char_p, i64, pi32, pi32, pi64, vp, vp, vp]),

@@ -32,6 +32,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <chrono>
 #include <vector>
 
 #include "psb_hip_internal.hpp"
@@ -720,10 +721,12 @@ __global__ __launch_bounds__(kBlock) void k_bi_x(int n, T* __restrict__ x, T* __
 //
 // Blocks wait for one another, so all of them have to be on the chip: the grid
 // is at most what it holds, and before anything is changed the blocks agree
-// that all have arrived (res_enter); where that takes over a tenth of a second
-// (another process has the chip) they agree to leave, and the solve goes on
-// with the launches per step.  After that no block waits for anything but
-// blocks that run.
+// that all have arrived (res_enter); where that takes over a millisecond
+// (another process or stream has the chip; the blocks of a free chip arrive in
+// tens of microseconds) they agree to leave, and the solve goes on with the
+// launches per step, as do the solves of the second after it (resident_busy), so
+// that a shared chip costs a millisecond a second.  After that no block waits
+// for anything but blocks that run.
 constexpr int kResGrid = 256;     // blocks: one per CU, and the sums' slots
 constexpr int kResSlots = 8;      // slots of a row in registers
 constexpr int kResIters = 48;     // iterations of a launch (its vectors are loaded and stored once)
@@ -731,6 +734,10 @@ constexpr int kResIters = 48;     // iterations of a launch (its vectors are loa
 // recurrence breaks down and the solve fails); a poll takes under a microsecond,
 // a real wait tens
 constexpr int kResPolls = 1 << 20;
+// ticks of the 100 MHz clock that a block waits for the others to arrive, and
+// nanoseconds for which a refusal is remembered
+constexpr long long kResPatience = 100000;
+constexpr int64_t kResBusy = 1000000000;
 
 struct ResCtl {
   unsigned int arrived;    // blocks of all launches so far
@@ -749,17 +756,20 @@ struct ResArgs {
   double* hist;
   int iters;
   unsigned int launch;     // 1, 2, ... of the solve
+  unsigned int leave;      // the launch that leaves whoever arrives (tests; 0: none)
   Waits waits;
 };
 
 // Whether all blocks of the launch run together (see above).  Every block
-// arrives in every launch, so the count tells.
-__device__ __forceinline__ bool res_enter(ResCtl* c, unsigned int launch, KState* st) {
+// arrives in every launch, so the count tells.  Once a launch has left, those
+// queued behind it leave too.
+__device__ __forceinline__ bool res_enter(ResCtl* c, unsigned int launch, unsigned int leave,
+                                          KState* st) {
   __shared__ int go;
   if (threadIdx.x == 0) {
     __hip_atomic_fetch_add(&c->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     go = 0;
-    if (!halted(st)) {
+    if (!halted(st) && !st->left) {
       const unsigned int yes = 2 * launch + 1, no = yes + 1;
       const long long t0 = wall_clock64();   // 100 MHz
       for (;;) {
@@ -769,9 +779,10 @@ __device__ __forceinline__ bool res_enter(ResCtl* c, unsigned int launch, KState
           go = d == yes;
           break;
         }
-        const bool all = __hip_atomic_load(&c->arrived, __ATOMIC_RELAXED,
+        const bool all = launch != leave &&
+                         __hip_atomic_load(&c->arrived, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT) == launch * gridDim.x;
-        if (all || wall_clock64() - t0 > 10000000)
+        if (all || launch == leave || wall_clock64() - t0 > kResPatience)
           __hip_atomic_compare_exchange_strong(&c->decision, &d, all ? yes : no, __ATOMIC_RELAXED,
                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
@@ -1044,7 +1055,7 @@ __global__ __launch_bounds__(NT) void k_res_cg(M m, ResArgs<T> a) {
   __shared__ T ps[NT * RPT];
   __shared__ KState S;
   bool lost = false;   // a wait was given up (res_sum, res_group)
-  if (!res_enter(a.ctl, a.launch, a.st)) return;
+  if (!res_enter(a.ctl, a.launch, a.leave, a.st)) return;
   const int n = m.nr, r0 = blockIdx.x * (NT * RPT);
   const int rows = min(NT * RPT, n - r0);
   unsigned int j = a.ctl->sums;
@@ -1135,7 +1146,7 @@ __global__ __launch_bounds__(NT) void k_res_bi(M m, ResArgs<T> a) {
   __shared__ T ps[NT * RPT];
   __shared__ KState S;
   bool lost = false;   // a wait was given up (res_sum, res_group)
-  if (!res_enter(a.ctl, a.launch, a.st)) return;
+  if (!res_enter(a.ctl, a.launch, a.leave, a.st)) return;
   const int n = m.nr, r0 = blockIdx.x * (NT * RPT);
   const int rows = min(NT * RPT, n - r0);
   unsigned int j = a.ctl->sums;
@@ -1398,14 +1409,29 @@ static int res_width(const Solver& s) {
   return s.fmt == FMT_HLL ? ((HllDev*)s.mat)->max_width : ((EllDev*)s.mat)->nzm;
 }
 
+// Whether a resident solve was refused the chip within the last second, and the
+// note of a refusal.
+static int64_t steady_ns() {
+  return std::chrono::duration_cast<std::chrono::nanoseconds>(
+             std::chrono::steady_clock::now().time_since_epoch())
+      .count();
+}
+static bool resident_busy() {
+  return steady_ns() < __atomic_load_n(&ctx().resident_not_before, __ATOMIC_RELAXED);
+}
+static void resident_refused() {
+  __atomic_store_n(&ctx().resident_not_before, steady_ns() + kResBusy, __ATOMIC_RELAXED);
+  __atomic_fetch_add(&ctx().resident_left, 1, __ATOMIC_RELAXED);
+}
+
 // Rows per thread of a resident solve of n rows in blocks of nt threads, 0
-// where the solve takes launches per step: CSR, more rows than threads hold
+// where the solve takes launches per step: a busy chip, CSR, more rows than threads hold
 // (four rows each for CG and two for BiCGSTAB), several rows a thread wider
 // than the registers hold or, four of FP64, not in 16-bit storage (ResRows),
 // fewer CUs than blocks, or buffers that the allocation-free entry point could
 // not hold (both entry points choose alike).
 static int resident_rows(const Solver& s, int itmax, int* nt) {
-  if (s.fmt == FMT_CSR || s.n <= 0) return 0;
+  if (s.fmt == FMT_CSR || s.n <= 0 || resident_busy()) return 0;
   if ((s.fmt == FMT_HLL ? ((HllDev*)s.mat)->max_col : ((EllDev*)s.mat)->max_col) > s.n) return 0;
   if (solve_bytes(s.method, s.n, s.etype, itmax) + align256(kFoldBytes) +
           resident_bytes(s.n, s.etype) > kScratchBytes)
@@ -1672,6 +1698,7 @@ static int resident_setup(Solver& s, ResArgs<T>* a) {
   a->xb[0] = (T*)s.rx[0];
   a->xb[1] = (T*)s.rx[1];
   a->hist = s.hist;
+  a->leave = (unsigned int)__atomic_load_n(&ctx().resident_leave, __ATOMIC_RELAXED);
   a->waits = waits(kResPolls);
   return PSB_HIP_SUCCESS;
 }
@@ -1799,6 +1826,7 @@ static int solve(Solver& s, const T* b, T* x, const T* d, double eps, int itmax,
     if ((rc = read_state(s))) return rc;
     if (s.hst->done) break;
     if (s.hst->left) {   // the chip was not free: go on from here with launches per step
+      resident_refused();
       rpt = 0;
       s.hst->left = 0;
       PSB_HIP_CHECK(hipMemcpyAsync(s.st, s.hst, sizeof(KState), hipMemcpyHostToDevice, s.stream));
@@ -2002,6 +2030,7 @@ static int mixed_reliable(HllDev* h, const double* b, double* x, const double* d
     }
     if ((rc = read_state(inner))) return rc;
     if (inner.hst->left) {   // the chip was not free: go on with launches per step
+      resident_refused();
       rpt = 0;
       inner.hst->left = 0;
       PSB_HIP_CHECK(hipMemcpyAsync(inner.st, inner.hst, sizeof(KState), hipMemcpyHostToDevice,
@@ -2176,6 +2205,13 @@ int psb_hip_krylov_fused_noalloc(int method, int fmt, void* dmat, void* diag, vo
     if ((rc = s.alloc((void**)&s.fold, kFoldBytes)) || (rc = clear_fold(s))) return rc;
   }
   return fused_run(__func__, s, diag, bv, xv, eps, itmax, istop, check_every, iter, err, hist);
+}
+
+int psb_hip_set_resident_leave(int launch) {
+  Context& c = ctx();
+  __atomic_store_n(&c.resident_leave, launch > 0 ? launch : 0, __ATOMIC_RELAXED);
+  __atomic_store_n(&c.resident_not_before, 0, __ATOMIC_RELAXED);
+  return __atomic_exchange_n(&c.resident_left, 0, __ATOMIC_RELAXED);
 }
 
 int psb_hip_krylov_mixed(int method, void* dmat, void* diag, void* bv, void* xv, double eps,

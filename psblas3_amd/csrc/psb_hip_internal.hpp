@@ -49,6 +49,11 @@ struct Context {
   char* scratch = nullptr;
   size_t scratch_bytes = 0;
   void* scratch_host = nullptr;         // pinned, kScratchHostBytes
+  // resident solves (krylov.hip; accessed atomically): until when the chip
+  // counts as busy after one did not come to run (steady clock, ns), the launch
+  // at which a test has them leave (0: none), and how many have left
+  int64_t resident_not_before = 0;
+  int resident_leave = 0, resident_left = 0;
   hipEvent_t scratch_ev[2] = {nullptr, nullptr};
 };
 // size of the device scratch array and of its pinned host companion
