@@ -62,9 +62,10 @@
 #include <string.h>
 
 #include <algorithm>
-#include <thread>
+#include <new>
 #include <vector>
 
+#include "host_parallel.hpp"
 #include "psb_hip_internal.hpp"
 
 namespace psbhip {
@@ -453,18 +454,6 @@ static void order_levels(int n, int nlev, const std::vector<int>& lev, std::vect
   for (int i = 0; i < n; i++) rows[fill[lev[i]]++] = i;
 }
 
-// f(thread, lo, hi) over [0, n) on host threads (one below min_n).
-template <typename F>
-static void host_parallel(int n, int min_n, F f) {
-  const int hw = (int)std::thread::hardware_concurrency();
-  const int nt = n < min_n ? 1 : std::max(1, std::min({hw, 8, n}));
-  std::vector<std::thread> th;
-  for (int k = 1; k < nt; k++)
-    th.emplace_back([=, &f] { f(k, (int)((int64_t)n * k / nt), (int)((int64_t)n * (k + 1) / nt)); });
-  f(0, 0, (int)((int64_t)n / nt));
-  for (auto& t : th) t.join();
-}
-constexpr int kHostThreads = 8;
 constexpr int kHostMin = 32768;   // rows from which the planning uses threads
 
 // The offsets of a regular grid in natural order: every entry of the triangle
@@ -892,6 +881,18 @@ static void enqueue_apply(IluDev* F, hipStream_t s) {
   enqueue_levels<double>(F->U, nullptr, false, F->xa, F->ya, s);
 }
 
+// The host planning f behind a C entry point, out of host memory as a return code.
+template <typename F>
+static int plan(F f) {
+  try {
+    return f();
+  } catch (const std::bad_alloc&) {
+    return set_error(PSB_HIP_OUTOFMEM, "trsv", "host memory");
+  } catch (const std::exception& e) {
+    return set_error(PSB_HIP_RUNTIME, "trsv", e.what());
+  }
+}
+
 template <typename V>
 static void free_tri(TriLevels<V>& T) {
   void* p[] = {T.perm, T.irp, T.ja, T.val, T.tiles, T.trow, T.tdv, T.tval, T.tdep, T.tstep,
@@ -1015,17 +1016,8 @@ static int build_sv(TriSolve<V>* S, int n, const int* irp, const int* ja, const 
   return PSB_HIP_SUCCESS;
 }
 
-// The CSR matrix's prepared solve for key (lower | unit << 1 | trans << 2),
-// built from the device copy of the matrix on first use and kept until the
-// matrix is rewritten, freed or asked for another triangle or op.
 template <typename V>
-static int csr_sv_get(CsrDev* m, int key, TriSolve<V>** out) {
-  TriSolve<V>* S = (TriSolve<V>*)m->sv;
-  if (S && S->key == key) {
-    *out = S;
-    return PSB_HIP_SUCCESS;
-  }
-  release_csr_sv(m);
+static int csr_sv_build(TriSolve<V>* S, const CsrDev* m, int key) {
   std::vector<int> irp(m->rows + 1), ja(m->nnz > 0 ? m->nnz : 1);
   std::vector<V> val(m->nnz > 0 ? m->nnz : 1);
   hipStream_t s = ctx().stream;
@@ -1038,9 +1030,23 @@ static int csr_sv_get(CsrDev* m, int key, TriSolve<V>** out) {
                                  hipMemcpyDeviceToHost, s));
   }
   PSB_HIP_CHECK(hipStreamSynchronize(s));
+  return build_sv<V>(S, m->rows, irp.data(), ja.data(), val.data(), (key & 1) != 0,
+                     (key & 2) != 0, (key & 4) != 0);
+}
+
+// The CSR matrix's prepared solve for key (lower | unit << 1 | trans << 2),
+// built from the device copy of the matrix on first use and kept until the
+// matrix is rewritten, freed or asked for another triangle or op.
+template <typename V>
+static int csr_sv_get(CsrDev* m, int key, TriSolve<V>** out) {
+  TriSolve<V>* S = (TriSolve<V>*)m->sv;
+  if (S && S->key == key) {
+    *out = S;
+    return PSB_HIP_SUCCESS;
+  }
+  release_csr_sv(m);
   S = new TriSolve<V>();
-  const int rc = build_sv<V>(S, m->rows, irp.data(), ja.data(), val.data(), (key & 1) != 0,
-                             (key & 2) != 0, (key & 4) != 0);
+  const int rc = plan([&] { return csr_sv_build(S, m, key); });
   if (rc) {
     destroy_sv(S);
     return rc;
@@ -1100,8 +1106,10 @@ int psb_hip_ilu_alloc(void** ilu, int n, const int* lirp, const int* lja, const 
   for (TriForm form : {TRI_AUTO, TRI_TILES, TRI_LEVELS}) {   // both factors in the same form
     free_tri(F->L);
     free_tri(F->U);
-    rc = upload_tri(F->L, n, true, lirp, lja, lval, (const double*)nullptr, form);
-    if (!rc) rc = upload_tri(F->U, n, false, uirp, uja, uval, (const double*)nullptr, form);
+    rc = plan([&] {
+      const int rl = upload_tri(F->L, n, true, lirp, lja, lval, (const double*)nullptr, form);
+      return rl ? rl : upload_tri(F->U, n, false, uirp, uja, uval, (const double*)nullptr, form);
+    });
     if (rc || (F->L.ntiles > 0) == (F->U.ntiles > 0)) break;
   }
   if (rc) {
