@@ -1671,8 +1671,9 @@ template <typename T, int OP>
 static int resident_batch(Solver& s, const Mats<T>& m, const ResArgs<T>& a, int nt, int rpt) {
   if (s.fmt == FMT_HLL && m.hll.hksz == 64)
     return resident_launch<T, OP>(s, as64(m.hll), a, nt, rpt);
-  if (s.fmt == FMT_HLL) return resident_launch<T, OP>(s, m.hll, a, nt, rpt);
-  return resident_launch<T, OP>(s, m.ell, a, nt, rpt);
+  if constexpr (OP != FIN_RU_X)   // mixed solves take HLL only
+    if (s.fmt == FMT_ELL) return resident_launch<T, OP>(s, m.ell, a, nt, rpt);
+  return resident_launch<T, OP>(s, m.hll, a, nt, rpt);
 }
 
 // The buffers of a resident solve; every entry starts unset.

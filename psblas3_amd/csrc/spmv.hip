@@ -1442,17 +1442,23 @@ static int hll_spmm_launch(const HllDev* m, const T* val, const T* x, int ldx, T
     return PSB_HIP_SUCCESS;
   }
   // narrow rows (stencils of up to 9 points): column by column.  Byte offsets
-  // into a column are 32-bit.  FP32 rows of scattered columns (no 16-bit
-  // offsets) keep the groups of 8 up to 16 columns: every gather is a line of
-  // its own there, and two columns of a slot share the index arithmetic (6
+  // into a column are 32-bit.  A matrix without 16-bit offsets has hacks whose
+  // rows' columns in one slot lie over 65,536 apart: every gather is a line of
+  // its own, neighbouring slots share none, and two columns of a slot share the
+  // index arithmetic.  There FP32 keeps the groups of 8 up to 16 columns (6
   // random columns a row, n = 1M, k = 4, 8 and 16: 218, 482 and 1015 us against
-  // 261, 537 and 1162; k = 24 2214 against 1809; FP64 k = 8 693 against 575).
+  // 261, 537 and 1162; k = 24 2214 against 1809), and FP64, whose pairs of rows
+  // take more registers in groups, does not (k = 2, 4, 8 and 16: 146, 308, 689
+  // and 1439 us in groups against 143, 290, 575 and 1226; n = 100,000, k = 2, 4
+  // and 8: 10.1, 18.2 and 33.8 against 9.7, 16.9 and 32.9; 3 columns a row,
+  // k = 2 and 4: 82.4 and 169 against 83.2 and 167).
   const bool scattered = !hll_use_idx16(m);
   if (m->max_width <= kSpmmWidth && ncols > 1 &&
       !(scattered && sizeof(T) == 4 && m->hksz % 2 == 0 && ncols <= 16) &&
       (uint64_t)m->max_col * sizeof(T) <= 0xffffffffull) {
-    if (sizeof(T) == 8 && m->hksz % 2 == 0)
-      return hll_spmm_cols<T, 2>(m, val, x, ldx, alpha, beta, y, ldy, ncols);
+    if constexpr (sizeof(T) == 8)
+      if (m->hksz % 2 == 0)
+        return hll_spmm_cols<T, 2>(m, val, x, ldx, alpha, beta, y, ldy, ncols);
     return hll_spmm_cols<T, 1>(m, val, x, ldx, alpha, beta, y, ldy, ncols);
   }
   hipStream_t s = ctx().stream;
