@@ -22,7 +22,7 @@
 // computed as the CPU updates them, by running subtraction
 // y(c) = ((x(c) - v1 y(i1)) - v2 y(i2)) ..., then the division.
 //
-// The triangle is cut into tiles of at most kTileRows rows and one workgroup
+// The triangle is cut into tiles of about kTileRows rows and one workgroup
 // solves a tile: its rows in steps (the levels inside the tile, 64 rows at a
 // time, one wavefront), with the entries, the right-hand side and the solution
 // staged in LDS, so a step costs LDS traffic and arithmetic only.  A row's
@@ -70,8 +70,9 @@
 
 namespace psbhip {
 
-// Limits of a tile: rows, stored entries, halo entries, LDS bytes (64 KB
-// lets two workgroups share a CU; an 8 x 8 x 8 tile takes about 31 KB).
+// Limits of a tile that is a run of rows: rows, stored entries, halo entries; and
+// of any tile (boxes have up to 576 rows): LDS bytes (64 KB lets two workgroups
+// share a CU; an 8 x 8 x 8 tile takes about 31 KB).
 constexpr int kTileRows = 512;
 constexpr int kTileEntries = 2048;
 constexpr int kTileHalo = 1024;
@@ -488,8 +489,8 @@ static int assign_tiles(int n, bool lower, const int* irp, const int* ja,
   int o[3] = {1, 0, 0};
   const int m = grid_offsets(n, lower, irp, ja, o);
   if (m > 0) {
-    // 8 x 8 x 8: a level of the box is at most 48 rows, one step; 24 x 24 in
-    // two dimensions takes the same number of rows
+    // 8 x 8 x 8 (512 rows): a level of the box is at most 48 rows, one step; in
+    // two dimensions 24 x 24 (576 rows), at most 24 a level
     const int nx = o[1], ny = m == 3 ? o[2] / nx : (n + nx - 1) / nx;
     const int bx = m == 3 ? 8 : 24, by = bx, bz = 8;
     const int tx = (nx + bx - 1) / bx, ty = (ny + by - 1) / by;
