@@ -637,8 +637,7 @@ int psb_hip_ilu_alloc(void **ilu, int n, const int *lirp, const int *lja, const 
 int psb_hip_ilu_free(void *ilu);
 int psb_hip_ilu_levels(void *ilu, int *lower_levels, int *upper_levels);
 /* tiles of each factor, each solved by one workgroup (0 when the solves launch
-   once per level: the variant is 1, the factors have few levels, or a row does
-   not fit a tile) */
+   once per level: the variant is 1 or the factors have few levels) */
 int psb_hip_ilu_segments(void *ilu, int *lower_segments, int *upper_segments);
 /* triangular-solve kernels for factors allocated afterwards: 0 (default) tiles
    of rows, one workgroup each, that wait for one another's entries; 1 one

@@ -40,7 +40,8 @@
 // Tiles follow the grid when the triangle's entries sit at the offsets of a
 // regular grid in natural order (1, p and q, p dividing q: 5- and 7-point
 // stencils and their ILU(0) factors), as boxes of 8 x 8 x 8 or 24 x 24 rows;
-// otherwise they are runs of consecutive rows.  The chain of dependencies
+// otherwise they are runs of consecutive rows, and a row of more than 1024
+// entries is a tile of its own (wide_row).  The chain of dependencies
 // then crosses tiles once in 8 (24) rows along each axis, and only a crossing
 // pays the way through memory between XCDs.
 //
@@ -50,13 +51,12 @@
 // 10 x 10 x 10 53 / 114 / 228 us, of 8 x 8 x 4 44 / 106 / 224 us); 5-point
 // 1000 x 1000 2562 -> 647 us; 27-point L = 40, runs of rows, 1373 -> 407 us.
 //
-// A triangle of at most kFewLevels levels, with a row of more than
-// kTileEntries / 2 entries, or with the launch-per-level variant set, is
-// solved in level order instead: renumbered
-// so that level l holds positions lev_ptr[l] .. lev_ptr[l+1]-1 (rows ascending
-// inside a level), x gathered into that order, one launch per level (one
-// thread per row), the solution scattered back; captured once into a graph
-// that works on internal buffers.
+// A triangle of at most kFewLevels levels, or with the launch-per-level variant
+// set, is solved in level order instead: renumbered so that level l holds
+// positions lev_ptr[l] .. lev_ptr[l+1]-1 (rows ascending inside a level), x
+// gathered into that order, one launch per level (one thread per row), the
+// solution scattered back; captured once into a graph that works on internal
+// buffers.
 #pragma clang fp contract(off)
 
 #include <string.h>
@@ -168,20 +168,24 @@ __global__ __launch_bounds__(kBlock) void k_perm_scatter(int n, const int* __res
     dst[perm[p]] = src[p];
 }
 
-// y[perm[p]] = alpha * src[p] + beta * y[perm[p]] with the special cases of
-// the library's axpby (alpha or beta 0 or 1), separately rounded; beta == 0
-// and alpha == -1 negate, as the CPU solve's scaling does
+// alpha * s + beta * *y with the special cases of the library's axpby (alpha or
+// beta 0 or 1; y not read for beta == 0), separately rounded; beta == 0 and
+// alpha == -1 negate, as the CPU solve's scaling does
+template <typename T>
+__device__ __forceinline__ T axpby_y(T alpha, T s, T beta, const T* y) {
+  if (alpha == T(0)) return (beta == T(0)) ? T(0) : (beta == T(1) ? *y : beta * *y);
+  if (beta == T(0)) return (alpha == T(1)) ? s : alpha * s;
+  return alpha * s + beta * *y;
+}
+
+// y[perm[p]] = alpha * src[p] + beta * y[perm[p]]
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_perm_scatter_axpby(int n, const int* __restrict__ perm,
                                                                const T* __restrict__ src,
                                                                T alpha, T beta, T* y) {
   for (int p = blockIdx.x * kBlock + threadIdx.x; p < n; p += gridDim.x * kBlock) {
     const int i = perm[p];
-    T r;
-    if (alpha == T(0)) r = (beta == T(0)) ? T(0) : (beta == T(1) ? y[i] : beta * y[i]);
-    else if (beta == T(0)) r = (alpha == T(1)) ? src[p] : alpha * src[p];
-    else r = alpha * src[p] + beta * y[i];
-    y[i] = r;
+    y[i] = axpby_y(alpha, src[p], beta, y + i);
   }
 }
 
@@ -259,6 +263,56 @@ struct TileStep {
 // (padding: value 0 times the zero slot, which leaves the sum's bits
 // unchanged; the sum starts at +0, so it is never -0 there, and the running
 // form subtracts +0); W == 0: the step's own width.  Rows sum in CSR order.
+// A row of more entries than a tile stages, a tile of its own (no steps; its halo
+// lists the row of every entry): the workgroup polls the entries in chunks and
+// leaves the products in LDS, one thread adds them in CSR order (product and sum
+// rounded separately, as everywhere).  Bound by that chain of adds.  One such row
+// used to send the whole triangle to a launch per level: FP64, a chain of 20,000
+// rows under one of 1500 entries 31.5 -> 5.2 ms, the 7-point lower triangle at
+// L = 40 under one of 3000 955 -> 124 us and under 64 of 5000 45.8 -> 0.6 ms, a full
+// triangle of 2496 rows 398 -> 12.9 ms.
+constexpr int kWideChunk = 1024;
+template <typename T, bool DIV, bool RUN>
+__device__ __forceinline__ void wide_row(const TriTile& t, const int* __restrict__ trow,
+                                         const T* __restrict__ tdv, const T* __restrict__ tval,
+                                         const int* __restrict__ thalo, T* sol, T* next,
+                                         const T* x, const T* __restrict__ scale, T alpha, T beta,
+                                         T* y, T* prod, const Waits& waits) {
+  const int i = trow[t.row0];
+  T xi = x[i];
+  if (scale) xi = xi * scale[i];
+  T acc = RUN ? xi : T(0);
+  for (int c = 0; c < t.nent; c += kWideChunk) {
+    const int m = t.nent - c < kWideChunk ? t.nent - c : kWideChunk;
+    for (int e = threadIdx.x; e < m; e += kTileThreads) {
+      const T* from = sol + thalo[t.halo0 + c + e];
+      const T v = ld_stream(tval + t.ent0 + c + e);
+      T s = ld_agent(from);
+      for (int polls = 1; is_unset(s); polls++) {
+        if (polls >= waits.polls) {
+          give_up(waits);
+          s = __builtin_bit_cast(T, MarkBits<T>::nan);
+          break;
+        }
+        __builtin_amdgcn_s_sleep(16);
+        s = ld_agent(from);
+      }
+      prod[e] = v * s;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int e = 0; e < m; e++) acc = RUN ? acc - prod[e] : acc + prod[e];
+    __syncthreads();
+  }
+  if (threadIdx.x != 0) return;
+  T r = RUN ? acc : xi - acc;
+  if (DIV) r = r / tdv[t.row0];
+  r = set_value(r);
+  next[i] = __builtin_bit_cast(T, MarkBits<T>::unset);
+  st_agent(sol + i, r);
+  y[i] = axpby_y(alpha, r, beta, y + i);
+}
+
 template <typename T, int W, bool DIV, bool RUN>
 __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
     size_t stride, int ntiles, const TriTile* __restrict__ tiles, const int* __restrict__ trow,
@@ -276,6 +330,11 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
   T* sol = sol2 + (epoch & 1 ? stride : 0);    // no line of one in the other: sol_stride
   T* next = sol2 + (epoch & 1 ? 0 : stride);
   T* ys = reinterpret_cast<T*>(lds);
+  if (t.nstep == 0) {
+    wide_row<T, DIV, RUN>(t, trow, tdv, tval, thalo, sol, next, x, scale, alpha, beta, y, ys,
+                          waits);
+    return;
+  }
   char* at = lds + lds16(sizeof(T) * (size_t)(t.nrow + t.nhalo + 1));
   T* ev = reinterpret_cast<T*>(at);
   at += lds16(sizeof(T) * (size_t)t.nent);
@@ -420,12 +479,7 @@ __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
   __syncthreads();
   for (int p = threadIdx.x; p < t.nrow; p += kTileThreads) {
     const int i = rows[p];
-    const T s = ys[p];
-    T r;
-    if (alpha == T(0)) r = (beta == T(0)) ? T(0) : (beta == T(1) ? y[i] : beta * y[i]);
-    else if (beta == T(0)) r = (alpha == T(1)) ? s : alpha * s;
-    else r = alpha * s + beta * y[i];
-    y[i] = r;
+    y[i] = axpby_y(alpha, ys[p], beta, y + i);
   }
 }
 
@@ -456,6 +510,9 @@ static void order_levels(int n, int nlev, const std::vector<int>& lev, std::vect
 }
 
 constexpr int kHostMin = 32768;   // rows from which the planning uses threads
+
+// A row that takes a tile of its own (wide_row).
+static bool is_wide(int len) { return len > kTileEntries / 2; }
 
 // The offsets of a regular grid in natural order: every entry of the triangle
 // sits 1, p or q rows before its row (in solve order), q a multiple of p.
@@ -509,9 +566,11 @@ static int assign_tiles(int n, bool lower, const int* irp, const int* ja,
     bool bad[kHostThreads] = {};
     host_parallel(n, kHostMin, [&](int th, int lo, int hi) {
       bool any = false;
-      for (int t = lo; t < hi; t++)
-        for (int e = irp[row(t)] - 1; e < irp[row(t) + 1] - 1; e++)
-          any = any || tile[dep(e)] > tile[t];
+      for (int t = lo; t < hi; t++) {
+        const int b = irp[row(t)] - 1, m = irp[row(t) + 1] - 1 - b;
+        any = any || is_wide(m);   // an entry stored over and over
+        for (int e = b; e < b + m; e++) any = any || tile[dep(e)] > tile[t];
+      }
       bad[th] = any;
     });
     if (!*std::max_element(bad, bad + kHostThreads))
@@ -519,8 +578,21 @@ static int assign_tiles(int n, bool lower, const int* irp, const int* ja,
   }
   std::vector<int> seen(n > 0 ? n : 1, -1);
   int nt = 0, rows = 0, ent = 0, halo = 0, t0 = 0;
+  bool wide = false;   // the tile holds a wide row: nothing joins it
   for (int t = 0; t < n; t++) {
     const int b = irp[row(t)] - 1, e = irp[row(t) + 1] - 1;
+    const bool w = is_wide(e - b);
+    if (rows > 0 && (wide || w)) {
+      nt++;
+      rows = ent = halo = 0;
+      t0 = t;
+    }
+    wide = w;
+    if (w) {
+      rows = 1;
+      tile[t] = nt;
+      continue;
+    }
     for (;;) {
       int fresh = 0;   // halo entries this row would add
       for (int k = b; k < e; k++) {
@@ -568,15 +640,15 @@ struct TilePack {
 constexpr unsigned kHaloHash = 4 * kTileHalo;   // a tile has at most kTileHalo halo entries
 
 // Cuts the triangle into tiles and uploads them (T.ntiles > 0 then); leaves
-// T.ntiles at 0 when a row does not fit a tile.
+// T.ntiles at 0 when a tile does not fit LDS.
 template <typename V>
 static int plan_tiles(TriLevels<V>& T, bool lower, const int* irp, const int* ja, const V* val,
                       const V* diag, const std::vector<int>& lev) {
   const int n = T.n;
   if (n == 0) return PSB_HIP_SUCCESS;
-  int wmax = 0;
-  for (int i = 0; i < n; i++) wmax = std::max(wmax, irp[i + 1] - irp[i]);
-  if (wmax > kTileEntries / 2) return PSB_HIP_SUCCESS;
+  int wmax = 0;   // of the rows that share tiles
+  for (int i = 0; i < n; i++)
+    if (!is_wide(irp[i + 1] - irp[i])) wmax = std::max(wmax, irp[i + 1] - irp[i]);
   auto row = [&](int t) { return lower ? t : n - 1 - t; };
   auto dep = [&](int e) { return lower ? ja[e] - 1 : n - ja[e]; };
   std::vector<int> tile;
@@ -635,6 +707,18 @@ static int plan_tiles(TriLevels<V>& T, bool lower, const int* irp, const int* ja
       D.ent0 = (int)P.val.size();
       D.step0 = (int)P.step.size();
       D.halo0 = (int)P.halo.size();
+      if (nrow == 1 && is_wide(len(order[ptr[k]]))) {   // wide_row
+        const int i = row(order[ptr[k]]), b = irp[i] - 1, m = len(order[ptr[k]]);
+        trow[D.row0] = i;
+        if (diag) tdv[D.row0] = diag[i];
+        P.val.insert(P.val.end(), val + b, val + b + m);
+        P.dep.resize(P.val.size(), 0);
+        for (int e = b; e < b + m; e++) P.halo.push_back(ja[e] - 1);
+        D.nent = D.nhalo = m;
+        D.nstep = 0;
+        P.lds = std::max(P.lds, sizeof(V) * kWideChunk);
+        continue;
+      }
       // the tile's rows by level; begin: where each level that occurs begins
       trs.assign(order.begin() + ptr[k], order.begin() + ptr[k + 1]);
       int l0 = lv(trs[0]), l1 = l0;
@@ -729,7 +813,7 @@ static int plan_tiles(TriLevels<V>& T, bool lower, const int* irp, const int* ja
   hipStream_t s = ctx().stream;
   PSB_HIP_CHECK(hipMalloc((void**)&T.tval, sizeof(V) * std::max<size_t>(ents, 1)));
   PSB_HIP_CHECK(hipMalloc((void**)&T.tdep, sizeof(uint16_t) * std::max<size_t>(ents, 1)));
-  PSB_HIP_CHECK(hipMalloc((void**)&T.tstep, sizeof(int2) * steps));
+  PSB_HIP_CHECK(hipMalloc((void**)&T.tstep, sizeof(int2) * std::max<size_t>(steps, 1)));
   PSB_HIP_CHECK(hipMalloc((void**)&T.thalo, sizeof(int) * std::max<size_t>(halos, 1)));
   size_t e0 = 0, s0 = 0, h0 = 0;
   for (const TilePack<V>& P : pack) {

@@ -244,13 +244,14 @@ def test_chip_taken_mid_solve(gpu, orc, leave, fmt, n, method, ptype, at):
 
 @pytest.mark.parametrize("at", [1, 2, 3])
 @pytest.mark.parametrize("variant", ["restart", "reliable"])
-@pytest.mark.parametrize("ptype", ["DIAG", "NONE"])
-def test_chip_taken_mixed(gpu, orc, leave, variant, ptype, at):
-    """Mixed precision: the inner solve's launch finds the chip taken; the solution
+@pytest.mark.parametrize("ptype,n", [("DIAG", 100001), ("NONE", 100001), ("DIAG", 400001),
+                                     ("DIAG", 900001)])
+def test_chip_taken_mixed(gpu, orc, leave, variant, ptype, n, at):
+    """Mixed precision, one, two and four rows a thread: the inner solve's launch finds
+    the chip taken; the solution
     and the number of inner iterations are those of the undisturbed solve to the
     roundings of the sums."""
-    print(f"[gpu] case resident leave mixed {variant} {ptype} at={at}", flush=True)
-    n = 100001
+    print(f"[gpu] case resident leave mixed {variant} {ptype} n={n} at={at}", flush=True)
     a = _chain(n, "CG", P.psb_d_hip_hlg_sparse_mat(64))
     desc = P.psb_cdall(nl=n)
     prec = P.psb_dprec_type(ptype).build(a, desc)
