@@ -1431,10 +1431,35 @@ static void resident_refused() {
   __atomic_fetch_add(&ctx().resident_left, 1, __ATOMIC_RELAXED);
 }
 
+// Slots of the widest row up to which a resident solve is the faster one.  Its
+// threads stream the slots past the eighth, each group of eight waiting for the
+// other blocks' entries, where the products of launches per step read them from
+// L2 with more wavefronts to hide it.  Launches per step / resident, an iteration
+// of CG (FP64, FP32), random columns (no 16-bit offsets) and columns within 300 of
+// the row:
+//  - up to 65,536 rows (blocks of 256 threads): 1000 rows random, 118 slots 1.11,
+//    0.79, 54 slots 1.39, 1.08; 8000 rows banded, 139 slots 1.25, 0.84; 24,000 rows
+//    random, 100 slots 1.27, 0.94, 109 slots 0.99, 0.93, 61 slots 1.41, 1.04; 32,000
+//    rows banded, 89 slots 1.17, 1.01, 101 slots 0.98, 0.98; 60,000 rows banded, 49
+//    slots 1.24, 1.13, 59 slots 1.11, 0.96, 71 slots 0.99, 0.92; random, 37 slots
+//    1.40, 0.98, 50 slots 1.20, 0.91.
+//  - up to 131,072 rows (at most 128 blocks of 1024, half the CUs): 100,000 rows
+//    banded, 47 slots 1.11, 1.23, 61 slots 0.96, 0.89; random, 22 slots 1.16, 1.12, 32
+//    slots 0.91, 0.97.
+//  - beyond: 140,000 rows banded, 50 slots 1.34, 1.10, 81 slots 1.20, 0.90; random, 53
+//    slots 1.10, 0.93, 86 slots 1.01, 0.84; 255,000 rows banded, 123 slots 0.84, 1.01.
+static int res_most_width(int n, bool single, bool scattered) {
+  if (n > 128 * 1024) return single ? (scattered ? 48 : 64) : (scattered ? 64 : 88);
+  if (n > 64 * 1024) return scattered ? 22 : 44;
+  const int cap = single ? 56 : (n <= 8192 ? 150 : 104);
+  const int slots = single && scattered ? 2200000 : 3200000;   // of the whole matrix
+  return cap < slots / n ? cap : slots / n;
+}
+
 // Rows per thread of a resident solve of n rows in blocks of nt threads, 0
 // where the solve takes launches per step: a busy chip, CSR, more rows than threads hold
-// (four rows each for CG and two for BiCGSTAB), several rows a thread wider
-// than the registers hold or, four of FP64, not in 16-bit storage (ResRows),
+// (four rows each for CG and two for BiCGSTAB), rows wider than pays
+// (res_most_width) or, several a thread, than the registers hold, or, four of FP64, not in 16-bit storage (ResRows),
 // fewer CUs than blocks, or buffers that the allocation-free entry point could
 // not hold (both entry points choose alike).
 static int resident_rows(const Solver& s, int itmax, int* nt) {
@@ -1450,11 +1475,10 @@ static int resident_rows(const Solver& s, int itmax, int* nt) {
   if (rpt > most || (s.n + *nt * rpt - 1) / (*nt * rpt) > ctx().num_cus) return 0;
   const HllDev* h = (const HllDev*)s.mat;
   const EllDev* e = (const EllDev*)s.mat;
-  const bool hll = s.fmt == FMT_HLL;
-  if (rpt > 1 && res_width(s) > kResSlots) return 0;
-  if (rpt == 4 && s.etype == PSB_HIP_TYPE_DOUBLE &&
-      !(hll ? hll_use_idx16(h) && h->hksz % 64 == 0 : ell_use_idx16(e)))
-    return 0;
+  const bool hll = s.fmt == FMT_HLL, single = s.etype != PSB_HIP_TYPE_DOUBLE;
+  const bool i16 = hll ? hll_use_idx16(h) : ell_use_idx16(e);
+  if (res_width(s) > (rpt > 1 ? kResSlots : res_most_width(s.n, single, !i16))) return 0;
+  if (rpt == 4 && !single && !(i16 && (!hll || h->hksz % 64 == 0))) return 0;
   return rpt;
 }
 

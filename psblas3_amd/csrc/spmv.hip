@@ -1429,6 +1429,31 @@ static int hll_spmm_cols(const HllDev* m, const T* val, const T* x, int ldx, T a
   return PSB_HIP_SUCCESS;
 }
 
+// Whether the product of narrow rows runs column by column (k_hll_spmm_cols) or in
+// groups of columns (k_hll_spmm_pair up to 16, k_hll_spmm beyond).  7-point
+// stencils, groups -> columns in us:
+//  - 2 columns: a row's slots are read once either way and the pairs' two rows a
+//    lane win while the launch counts: FP64 64^3 6.8 -> 8.0, 72^3 8.7 -> 10.0, from
+//    76^3 (439,000 rows) on columns, 12.3 -> 11.6, 160^3 79.7 -> 77.4; FP32 64^3 5.9 ->
+//    7.3, 200^3 108 -> 113.
+//  - 3 and 4 columns: FP64 64^3 (262,144 rows) 9.3 -> 10.2, 68^3 (314,432) 14.2 -> 12.9;
+//    FP32 3 columns 64^3 7.0 -> 7.8, 68^3 8.7 -> 8.0; FP32 4 columns never slower.
+//  - over 16 columns, FP64: its blocks of 512 rows walk the columns one after another,
+//    the groups' blocks of 256 rows take 32 at a time.  With fewer than half the CUs
+//    busy that tells: 32 columns 20^3 13.0 -> 19.7, 40^3 (125 blocks) 16.3 -> 21.5, 42^3
+//    (145) 23.9 -> 22.4, 64^3 64 -> 38.
+//  - over 20 columns, FP32, about two blocks a CU: 32 columns 45^3 (356 blocks) 15.9 ->
+//    14.7, 48^3 (432) 16.3 -> 18.6, 50^3 (489) 16.3 -> 19.2, 55^3 (650) 23.0 -> 20.6; 64
+//    columns 50^3 34.4 -> 32.7.
+static bool spmm_by_columns(int rows, int hksz, int ncols, bool single) {
+  if (hksz % 2 == 0 && ncols <= 4) {   // pairs need an even hack size
+    if (ncols == 2) return !single && rows > 420000;
+    if (ncols == 3 || !single) return rows > 300000;
+  }
+  if (!single) return ncols <= 16 || rows > 128 * 2 * kBlock;
+  return ncols <= 20 || ncols > 32 || rows <= 400 * kBlock || rows > 512 * kBlock;
+}
+
 template <typename T>
 static int hll_spmm_launch(const HllDev* m, const T* val, const T* x, int ldx, T alpha, T beta,
                            T* y, int ldy, int ncols) {
@@ -1441,8 +1466,8 @@ static int hll_spmm_launch(const HllDev* m, const T* val, const T* x, int ldx, T
     }
     return PSB_HIP_SUCCESS;
   }
-  // narrow rows (stencils of up to 9 points): column by column.  Byte offsets
-  // into a column are 32-bit.  A matrix without 16-bit offsets has hacks whose
+  // narrow rows (stencils of up to 9 points): column by column where that is
+  // faster (spmm_by_columns).  Byte offsets into a column are 32-bit.  A matrix without 16-bit offsets has hacks whose
   // rows' columns in one slot lie over 65,536 apart: every gather is a line of
   // its own, neighbouring slots share none, and two columns of a slot share the
   // index arithmetic.  There FP32 keeps the groups of 8 up to 16 columns (6
@@ -1454,6 +1479,7 @@ static int hll_spmm_launch(const HllDev* m, const T* val, const T* x, int ldx, T
   // k = 2 and 4: 82.4 and 169 against 83.2 and 167).
   const bool scattered = !hll_use_idx16(m);
   if (m->max_width <= kSpmmWidth && ncols > 1 &&
+      spmm_by_columns(m->rows, m->hksz, ncols, sizeof(T) == 4) &&
       !(scattered && sizeof(T) == 4 && m->hksz % 2 == 0 && ncols <= 16) &&
       (uint64_t)m->max_col * sizeof(T) <= 0xffffffffull) {
     if constexpr (sizeof(T) == 8)

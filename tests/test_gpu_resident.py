@@ -289,10 +289,13 @@ def test_taken_chip_is_remembered(gpu, orc, leave):
 @pytest.mark.parametrize("method,n,wide,resident", [
     ("CG", 1048576, 2, True), ("CG", 1048577, 2, False), ("BICGSTAB", 524288, 3, True),
     ("BICGSTAB", 524289, 2, False), ("CG", 300001, 3, True), ("CG", 300001, 6, False),
-    ("CG", 65537, 20, True)])
+    ("CG", 65537, 39, True), ("CG", 65537, 40, False), ("CG", 65536, 43, True),
+    ("CG", 65536, 44, False), ("CG", 8192, 145, True), ("CG", 8192, 146, False),
+    ("CG", 8193, 99, True), ("CG", 8193, 100, False), ("CG", 131073, 83, True),
+    ("CG", 131073, 84, False)])
 def test_which_solves_are_resident(gpu, orc, leave, method, n, wide, resident):
-    """More rows than the threads hold, or several a thread wider than eight slots,
-    take launches per step."""
+    """More rows than the threads hold, several a thread wider than eight slots, or
+    rows too wide to gain by it (5 + wide slots), take launches per step."""
     print(f"[gpu] case resident rule {method} n={n} wide={wide}", flush=True)
     a = _system(n, P.psb_d_hip_hlg_sparse_mat(64), method == "CG", wide)
     desc = P.psb_cdall(nl=n)

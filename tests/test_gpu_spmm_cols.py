@@ -50,3 +50,30 @@ def test_columns_bitexact(gpu, orc, kind, n, w, single, hk):
             P.psb_spmm(alpha, a, vm.mold().bld(X[:, c].copy()), beta, y1)
             assert np.array_equal(out[:, c], y1.get_vect()), (k, c)
     a.free()
+
+
+@pytest.mark.parametrize("n,k,single", [
+    (420000, 2, False), (420001, 2, False), (300000, 3, False), (300001, 4, False),
+    (300000, 3, True), (300001, 3, True), (420001, 2, True), (2000, 4, True),
+    (65536, 17, False), (65537, 17, False), (102400, 21, True), (102401, 21, True),
+    (131072, 32, True), (131073, 32, True), (131072, 33, True)])
+def test_either_side_of_the_lines(gpu, orc, n, k, single):
+    """Row and column counts on both sides of the lines between columns one by one
+    and in groups: first, last and a middle column equal the single-vector
+    product bit for bit."""
+    print(f"[gpu] case spmm lines n={n} k={k} single={single}", flush=True)
+    ia, ja, val = _matrix("band", n, 7, np.random.default_rng(3))
+    dt = np.float32 if single else np.float64
+    vm = P.psb_s_hip_vect() if single else P.psb_d_hip_vect()
+    a = P.matrix_from_coo(n, n, ia, ja, val,
+                          mold=(P.psb_s_hip_hlg_sparse_mat if single
+                                else P.psb_d_hip_hlg_sparse_mat)(64))
+    X = np.stack([orc.uniform_pm1(70 + c, n) for c in range(k)], axis=1).astype(dt)
+    yv = vm.mold().bld(np.zeros((n, k), dt))
+    P.psb_spmm(1.5, a, vm.mold().bld(X), 0.0, yv)
+    out = yv.get_vect()
+    for c in {0, k // 2, k - 1}:
+        y1 = vm.mold().bld(np.zeros(n, dt))
+        P.psb_spmm(1.5, a, vm.mold().bld(X[:, c].copy()), 0.0, y1)
+        assert np.array_equal(out[:, c], y1.get_vect()), c
+    a.free()
