@@ -1457,11 +1457,12 @@ static int res_most_width(int n, bool single, bool scattered) {
 }
 
 // Rows per thread of a resident solve of n rows in blocks of nt threads, 0
-// where the solve takes launches per step: a busy chip, CSR, more rows than threads hold
-// (four rows each for CG and two for BiCGSTAB), rows wider than pays
-// (res_most_width) or, several a thread, than the registers hold, or, four of FP64, not in 16-bit storage (ResRows),
-// fewer CUs than blocks, or buffers that the allocation-free entry point could
-// not hold (both entry points choose alike).
+// where the solve takes launches per step: a busy chip, CSR, more rows than
+// threads hold (four rows each for CG and two for BiCGSTAB), rows wider than
+// pays (res_most_width) or, several a thread, than the registers hold, or, four
+// of FP64, not in 16-bit storage (ResRows), fewer CUs than blocks, or buffers
+// that the allocation-free entry point could not hold (both entry points choose
+// alike).
 static int resident_rows(const Solver& s, int itmax, int* nt) {
   if (s.fmt == FMT_CSR || s.n <= 0 || resident_busy()) return 0;
   if ((s.fmt == FMT_HLL ? ((HllDev*)s.mat)->max_col : ((EllDev*)s.mat)->max_col) > s.n) return 0;

@@ -1467,10 +1467,11 @@ static int hll_spmm_launch(const HllDev* m, const T* val, const T* x, int ldx, T
     return PSB_HIP_SUCCESS;
   }
   // narrow rows (stencils of up to 9 points): column by column where that is
-  // faster (spmm_by_columns).  Byte offsets into a column are 32-bit.  A matrix without 16-bit offsets has hacks whose
-  // rows' columns in one slot lie over 65,536 apart: every gather is a line of
-  // its own, neighbouring slots share none, and two columns of a slot share the
-  // index arithmetic.  There FP32 keeps the groups of 8 up to 16 columns (6
+  // faster (spmm_by_columns).  Byte offsets into a column are 32-bit.  A matrix
+  // without 16-bit offsets has hacks whose rows' columns in one slot lie over
+  // 65,536 apart: every gather is a line of its own, neighbouring slots share
+  // none, and two columns of a slot share the index arithmetic.  There FP32
+  // keeps the groups of 8 up to 16 columns (6
   // random columns a row, n = 1M, k = 4, 8 and 16: 218, 482 and 1015 us against
   // 261, 537 and 1162; k = 24 2214 against 1809), and FP64, whose pairs of rows
   // take more registers in groups, does not (k = 2, 4, 8 and 16: 146, 308, 689

@@ -253,16 +253,6 @@ struct TileStep {
   int row;
 };
 
-// One tile per workgroup.  Bound by the chain of dependencies: a step (the
-// LDS reads of W solution entries, W multiply-adds and, when DIV, a division)
-// is 0.26 us with the division (a chain of 20,000 rows 5.1 ms), a crossing
-// into the next tile one store and one load through memory between XCDs,
-// 1-2 us; the bytes (40 a row) would take 2 us at L = 64, not 91.  Polling by
-// every lane from the start instead of by the first ones until an entry
-// comes: 97 and 254 us at L = 64 and 110.  W > 0: every row has W entries
-// (padding: value 0 times the zero slot, which leaves the sum's bits
-// unchanged; the sum starts at +0, so it is never -0 there, and the running
-// form subtracts +0); W == 0: the step's own width.  Rows sum in CSR order.
 // A row of more entries than a tile stages, a tile of its own (no steps; its halo
 // lists the row of every entry): the workgroup polls the entries in chunks and
 // leaves the products in LDS, one thread adds them in CSR order (product and sum
@@ -313,6 +303,16 @@ __device__ __forceinline__ void wide_row(const TriTile& t, const int* __restrict
   y[i] = axpby_y(alpha, r, beta, y + i);
 }
 
+// One tile per workgroup.  Bound by the chain of dependencies: a step (the
+// LDS reads of W solution entries, W multiply-adds and, when DIV, a division)
+// is 0.26 us with the division (a chain of 20,000 rows 5.1 ms), a crossing
+// into the next tile one store and one load through memory between XCDs,
+// 1-2 us; the bytes (40 a row) would take 2 us at L = 64, not 91.  Polling by
+// every lane from the start instead of by the first ones until an entry
+// comes: 97 and 254 us at L = 64 and 110.  W > 0: every row has W entries
+// (padding: value 0 times the zero slot, which leaves the sum's bits
+// unchanged; the sum starts at +0, so it is never -0 there, and the running
+// form subtracts +0); W == 0: the step's own width.  Rows sum in CSR order.
 template <typename T, int W, bool DIV, bool RUN>
 __global__ __launch_bounds__(kTileThreads) void k_trsv_tiles(
     size_t stride, int ntiles, const TriTile* __restrict__ tiles, const int* __restrict__ trow,
